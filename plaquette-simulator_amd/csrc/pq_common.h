@@ -68,7 +68,8 @@ PQ_HD void add_mod4(uint64_t &a0, uint64_t &a1, uint64_t b0, uint64_t b1) {
 //  0-7) and kLayerStart if the batch opens a new layer (all ops of one layer
 //  act on pairwise distinct qubits); on the first op of a run -- a layer,
 //  or the part of a layer inside one staging chunk -- also the run length
-//  (bits 8-19);
+//  (bits 8-19); on the first op of a layer, or of its part in one staging
+//  chunk, the number of ops in that part (bits 20-30);
 //  PQ_OP_NOISE alone: qa, na;  M: qa, slot = record id, t0 = coin
 //  threshold, (na, nb) = coin stream (low, high 32 bits), pad = kMeasSuperseded
 //  when a later M of the same measurement segment writes the same record.
@@ -81,6 +82,8 @@ constexpr uint32_t kLayerStart = 0x80000000u;
 constexpr uint32_t kBatchLenMask = 0xFFu;
 constexpr uint32_t kRunShift = 8;
 constexpr uint32_t kRunMask = 0xFFFu;
+constexpr uint32_t kLayerLenShift = 20;
+constexpr uint32_t kLayerLenMask = 0x7FFu;
 // An M whose record a later M of its segment overwrites: the measurement still
 // runs (it may leave the scratch row), but its record write is skipped, so the
 // last write in program order is the one that stays even when both run at

@@ -98,7 +98,14 @@ struct ProgramArgs {
   // 1: the program has row-tiled gate segments; above 512 qubits it runs in
   // the 768-thread build (program_max_threads)
   uint32_t wide;
+  // Shared-X/Z run (launch_shared): kSharedKnown when the host knows X/Z to be
+  // the |0...0> tableau, kSharedVerify when each word group checks it first.
+  // done[w] (kSharedVerify): whether group w ran there; k_program passes over
+  // those groups.
+  uint32_t shared;
+  uint32_t *done;
 };
+constexpr uint32_t kSharedKnown = 1, kSharedVerify = 2;
 // One state of a mixed batch: its program arguments, run parameters and
 // noise descriptors (planes are generated by the batch prologue).
 struct BatchCircuit {
@@ -136,6 +143,16 @@ hipError_t prepare_kernels(uint32_t n);
 // kernels at run time, so a captured graph can be replayed with new values.
 hipError_t launch_program(hipStream_t s, const ProgramArgs &a, uint32_t threads,
                           uint32_t blocks, const void *params);
+// Shared-X/Z form of a persistent run (pq_shared.hip): programs without
+// flagged H/S/CX/CZ on the |0...0> tableau, one workgroup per word group.
+constexpr uint32_t kSharedThreads = 768;
+constexpr uint32_t kSharedMaxQubits = 2048;
+constexpr uint64_t kSharedLdsBytes = 158 * 1024;
+bool shared_fits(uint32_t n);
+size_t shared_lds_bytes(uint32_t n);
+// Raises the kernels' dynamic-LDS limit for n qubits (not in a capture).
+hipError_t prepare_shared(uint32_t n);
+hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params);
 // Zeroes n 32-bit device words (a kernel: graph-capturable).
 hipError_t launch_zero_u32(hipStream_t s, unsigned int *p, uint32_t n);
 // Whether `slices` workgroups per word group for `nwords` groups of n qubits

@@ -1696,8 +1696,10 @@ __global__ __launch_bounds__(MAXT) void k_program_t(pq::ProgramArgs a,
       program_word<NREG>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm, &ss);
     }
   } else {
-    for (uint64_t wi = blockIdx.x; wi < a.nwords; wi += gridDim.x)
+    for (uint64_t wi = blockIdx.x; wi < a.nwords; wi += gridDim.x) {
+      if (a.done && a.done[a.word0 + wi]) continue;  // k_program_shared ran it
       program_word<NREG>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm);
+    }
   }
   if (census) {
     __syncthreads();

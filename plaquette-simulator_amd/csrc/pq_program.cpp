@@ -78,7 +78,8 @@ int validate_ops(uint64_t n, const pq_op *ops, uint64_t nops) { return validate(
 // every staging-chunk start and where the op code changes (a layer's ops are
 // sorted by code), and ends before the next one; its length goes into bits
 // 8-19 of its first instruction's pad.  Every run then has one op code, so
-// the row-tiled kernel dispatches on it once per wave share.
+// the row-tiled kernel dispatches on it once per wave share.  The same for
+// layer parts (a layer, or its part in one chunk) in bits 20-30.
 static void mark_runs(pq_program_s *p, const DSegment &sg) {
   const uint32_t end = (uint32_t)p->instrs.size();
   uint32_t start = sg.begin;
@@ -91,6 +92,12 @@ static void mark_runs(pq_program_s *p, const DSegment &sg) {
       start = k;
     }
   }
+  start = sg.begin;
+  for (uint32_t k = sg.begin + 1; k <= end; ++k)
+    if (k == end || (p->instrs[k].pad & kLayerStart) || (k - sg.begin) % kProgramStage == 0) {
+      p->instrs[start].pad |= (k - start) << kLayerLenShift;
+      start = k;
+    }
 }
 
 // Row tiling of a gate segment.  Gates act on each tableau row on its own,
@@ -312,6 +319,11 @@ static std::vector<std::vector<uint32_t>> window_schedule(const std::vector<DIns
 int compile_program(pq_program_s *p) {
   const pq_op *ops = p->ops.data();
   const uint64_t nops = p->ops.size();
+  p->uniform = true;
+  for (uint64_t i = 0; i < nops; ++i)
+    if (ops[i].code == PQ_OP_H_FLAG || ops[i].code == PQ_OP_S_FLAG ||
+        ops[i].code == PQ_OP_CX_FLAG || ops[i].code == PQ_OP_CZ_FLAG)
+      p->uniform = false;
   uint32_t nnoise = 0, nmeas = 0;
   uint64_t i = 0;
   while (i < nops) {
@@ -427,7 +439,8 @@ pq_program_s::~pq_program_s() {
   for (hipEvent_t e : ev) (void)hipEventDestroy(e);
   if (done_ev) (void)hipEventDestroy(done_ev);
   for (void *q : {(void *)d_census, (void *)d_segs, (void *)d_segq, (void *)d_instrs,
-                  (void *)d_noise, (void *)d_planes, (void *)d_side, (void *)d_sync})
+                  (void *)d_noise, (void *)d_planes, (void *)d_side, (void *)d_sync,
+                  (void *)d_done})
     dev_free(q, alloc_stream);
 }
 
@@ -472,6 +485,7 @@ static int create_program(pq_state s, const pq_op *ops, uint64_t nops, hipStream
   p->threads = program_max_threads((uint32_t)s->n, p->tiled);
   p->blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(s->W, 1u << 20));
   if (!as) HIPCHK(prepare_kernels((uint32_t)s->n));
+  if (p->uniform && shared_fits((uint32_t)s->n)) HIPCHK(prepare_shared((uint32_t)s->n));
   *out = p.release();
   return PQ_OK;
 }
@@ -676,12 +690,27 @@ static int choose_slices(pq_state s, pq_program p, const ProgramArgs &a, bool al
   return PQ_OK;
 }
 
+// Whether a persistent run may take the shared-X/Z kernel when X/Z are the
+// |0...0> tableau: no flagged H/S/CX/CZ, at least as many ops as qubits (it
+// writes the whole tableau, where a shorter program touches a few columns),
+// no census (which counts the per-shot kernel's work) and no launch shape or
+// slice count asked for.
+static bool shared_allowed(const pq_state_s *s, const pq_program_s *p) {
+  return p->uniform && shared_fits((uint32_t)s->n) && p->instrs.size() >= s->n &&
+         !p->census_on && !p->slices_set && p->threads >= 256;
+}
+
+// shared: 0 the per-shot kernel, kSharedKnown the shared-X/Z kernel,
+// kSharedVerify the shared-X/Z kernel and behind it the per-shot one for the
+// word groups whose X/Z were not the |0...0> tableau.
 static int enqueue_persistent(pq_state s, pq_program p, bool timed, bool allow_slices,
-                              bool fresh = false) {
+                              bool fresh = false, uint32_t shared = 0) {
   ProgramArgs a = program_args(s, p, kProgramLdsBytes);
   a.fresh = fresh ? 1u : 0u;
+  a.shared = shared;
+  a.done = shared == kSharedVerify ? p->d_done : nullptr;
   uint32_t S = 1;
-  int rc = choose_slices(s, p, a, allow_slices, &S);
+  int rc = choose_slices(s, p, a, allow_slices && !shared, &S);
   if (rc) return rc;
   p->slices_used = S;
   if (S > 1) {
@@ -706,7 +735,9 @@ static int enqueue_persistent(pq_state s, pq_program p, bool timed, bool allow_s
     }
     HIPCHK(hipEventRecord(p->ev[p->ev_used], s->stream));
   }
-  HIPCHK(launch_program(s->stream, a, p->threads, p->blocks, s->params_dev));
+  if (shared) HIPCHK(launch_shared(s->stream, a, s->params_dev));
+  if (shared != kSharedKnown)
+    HIPCHK(launch_program(s->stream, a, p->threads, p->blocks, s->params_dev));
   if (timed) {
     HIPCHK(hipEventRecord(p->ev[p->ev_used + 1], s->stream));
     p->ev_used += 2;
@@ -759,10 +790,24 @@ static int program_run(pq_state s, pq_program p, int form) {
   if (form == PQ_RUN_FRAME && s->n > measure_max_qubits())
     return pq_set_error(PQ_ERR_UNSUPPORTED, "frame form supports at most 4095 qubits");
   if (form == PQ_RUN_FRAME) return run_frame(s, p);
+  // X/Z are the |0...0> tableau: the shared-X/Z kernel, which reads no X/Z
+  // (they may be pending) and writes them all.  The holder of a raw pointer
+  // may have changed them, so an exposed state's word groups are checked, and
+  // so are a captured run's at every replay.
+  uint32_t shared = 0;
+  if ((form == PQ_RUN_PERSISTENT && s->xz_identity) || form == PQ_RUN_GRAPH)
+    if (shared_allowed(s, p))
+      shared = form == PQ_RUN_GRAPH || s->exposed ? kSharedVerify : kSharedKnown;
+  if (shared == kSharedVerify && !p->d_done)
+    HIPCHK(dev_alloc((void **)&p->d_done, s->W * sizeof(uint32_t), p->alloc_stream));
+  if (shared == kSharedKnown) {
+    s->xz_pending = false;
+    s->xz_plan.reset();
+  }
   // X/Z still the identity after a reset, and the program opens with a
   // row-tiled gate segment over every qubit: the persistent kernel writes
   // that segment's tiles itself, so the identity fill is not needed
-  const bool fresh = form == PQ_RUN_PERSISTENT && s->xz_pending && !s->xz_plan &&
+  const bool fresh = !shared && form == PQ_RUN_PERSISTENT && s->xz_pending && !s->xz_plan &&
                      !p->segs.empty() && p->segs[0].kind == 0 && p->segs[0].nq == s->n &&
                      program_tile_rows(program_args(s, p, kProgramLdsBytes).lds_words,
                                        (uint32_t)s->n) > 0;
@@ -778,7 +823,7 @@ static int program_run(pq_state s, pq_program p, int form) {
                            s->noise_seq));
   s->meas_seq += p->nmeas;
   s->noise_seq += p->nnoise;
-  if (form == PQ_RUN_PERSISTENT) return enqueue_persistent(s, p, p->timing_on, true, fresh);
+  if (form == PQ_RUN_PERSISTENT) return enqueue_persistent(s, p, p->timing_on, true, fresh, shared);
   if (form != PQ_RUN_GRAPH) return pq_set_error(PQ_ERR_ARG, "unknown run form");
   if (p->gexec && (p->graph_state != s || p->graph_arena_gen != s->arena_gen)) {
     (void)hipGraphExecDestroy(p->gexec);
@@ -788,7 +833,7 @@ static int program_run(pq_state s, pq_program p, int form) {
   }
   if (!p->gexec) {
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-    rc = enqueue_persistent(s, p, false, false);
+    rc = enqueue_persistent(s, p, false, false, false, shared);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(s->stream, &g);
     if (rc) {
@@ -809,6 +854,8 @@ extern "C" int pq_program_set_slices(pq_program p, uint32_t slices) {
   if (!p) return pq_set_error(PQ_ERR_ARG, "null program");
   if (slices > 1024) return pq_set_error(PQ_ERR_ARG, "slices must be at most 1024");
   p->slices_req = slices;
+  p->slices_set = true;
+  p->drop_graph();
   return PQ_OK;
 }
 

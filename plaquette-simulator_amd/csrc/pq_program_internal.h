@@ -29,6 +29,7 @@ struct pq_program_s {
   std::vector<pq::NoiseDesc> noise;
   std::vector<uint32_t> segq;  // qubit lists of row-tiled gate segments
   bool tiled = false;          // some gate segment runs row-tiled
+  bool uniform = false;        // no flagged H/S/CX/CZ: X/Z change in every shot alike
   pq::DSegment *d_segs = nullptr;
   uint32_t *d_segq = nullptr;
   pq::DInstr *d_instrs = nullptr;
@@ -60,6 +61,8 @@ struct pq_program_s {
   // the state size and the device), last used, and the slices' barrier
   // counters ([W] words) and give-up flag (one word after them)
   uint32_t slices_req = 0, slices_used = 1;
+  bool slices_set = false;     // pq_program_set_slices was called: per-shot kernel
+  uint32_t *d_done = nullptr;  // shared-X/Z runs that verify: groups that ran, [W]
   uint32_t slice_wait = 0;  // polls before a barrier gives up (0: default)
   unsigned int *d_sync = nullptr;
   uint64_t sync_words = 0;

@@ -1,0 +1,168 @@
+"""Programs run on the packed tableau that all shots share.
+
+A program without flagged H/S/CX/CZ on the |0...0> tableau runs in the
+shared-X/Z kernel; a program whose slice count was set keeps the per-shot
+kernel.  Both must leave the oracle's words and records.  Sizes: one and two
+qubits, the edges of a 64-row word, the last size whose packed columns fit the
+LDS and the first that keeps them in the tableau, and the largest size taken
+with the first refused."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ps():
+    import plaquette_simulator as ps
+    import plaquette_simulator_bindings as b
+    if b.device_count() < 1:
+        pytest.skip("no GPU")
+    return ps
+
+
+def say(msg):
+    sys.stderr.write(msg + "\n")
+    sys.stderr.flush()
+
+
+def mixed_ops(n, nops, seed, meas, two=True):
+    """Every op the shared form takes: gates, Paulis, noise, flags from records
+    and random flags on Paulis, measurements into new and existing records."""
+    from plaquette_simulator import workloads as W
+    rng = np.random.default_rng(seed)
+    b = W.OpList()
+    for _ in range(nops):
+        q = int(rng.integers(0, n))
+        t = (q + 1 + int(rng.integers(0, max(1, n - 1)))) % n
+        u = rng.random()
+        if u < meas:
+            again = b.nrec > 3 and rng.random() < 0.2
+            b.measure(q, 0.5, int(rng.integers(0, b.nrec)) if again else None)
+        elif u < meas + 0.1:
+            b.noise(q, 0.05, 0.03, 0.04)
+        elif u < meas + 0.15 and b.nrec:
+            b.flagged(int(rng.choice([W.OP_X_FLAG, W.OP_Y_FLAG, W.OP_Z_FLAG])), q,
+                      int(rng.integers(0, b.nrec)))
+        elif u < meas + 0.2:
+            b.with_prob(int(rng.choice([W.OP_X, W.OP_Y, W.OP_Z])), q, 0.3)
+        else:
+            codes = [W.OP_H, W.OP_S, W.OP_X, W.OP_Y, W.OP_Z]
+            if n > 1:
+                codes += [W.OP_CX, W.OP_CX, W.OP_CZ]
+            code = int(rng.choice(codes))
+            b.gate(code, q, t if code in (W.OP_CX, W.OP_CZ) else 0)
+    return b.array()
+
+
+def check(st, orc):
+    st.sync_records()
+    x, z, r = st.device_to_host_numpy()
+    assert np.array_equal(x, orc.x), "x differs"
+    assert np.array_equal(z, orc.z), "z differs"
+    assert np.array_equal(r, orc.r), "r differs"
+    assert st.num_records == len(orc.records)
+    for i, (res, det) in enumerate(orc.records):
+        gres, gdet = st.get_record(i)
+        assert np.array_equal(gres, res), f"record {i} results differ"
+        assert np.array_equal(gdet, det), f"record {i} determined differ"
+
+
+@pytest.mark.parametrize("n,B,nops,meas", [
+    (1, 130, 60, 0.2), (2, 64, 80, 0.2), (3, 1, 80, 0.3),
+    (63, 65, 900, 0.1), (64, 65, 900, 0.1), (65, 65, 900, 0.1),
+    (128, 64, 1500, 0.05), (129, 70, 1500, 0.05),
+    (471, 3, 1600, 0.05), (472, 3, 1600, 0.05), (513, 3, 1600, 0.04),
+    (700, 3, 1500, 0.03), (2048, 1, 2400, 0.01), (2049, 1, 2400, 0.01),
+])
+def test_shared_equals_oracle(ps, n, B, nops, meas):
+    ops = mixed_ops(n, nops, 10 * n + B, meas)
+    say(f"[case] n={n} B={B} ops={len(ops)}")
+    orc = O.OracleState(n, B, 17)
+    orc.run_program(ops.astype(np.int32))
+    st = ps.CliffordState(n, B, 17, True)
+    ps.Program(st, ops).run(st, "persistent")
+    check(st, orc)
+
+
+@pytest.mark.parametrize("n,B", [(65, 200), (500, 70)])
+def test_per_shot_kernel_is_still_reached(ps, n, B):
+    # the same program in both kernels, and each again from the state it left
+    ops = mixed_ops(n, 3 * n, 5, 0.05)
+    a, b = (ps.CliffordState(n, B, 3, True) for _ in range(2))
+    pa, pb = ps.Program(a, ops), ps.Program(b, ops)
+    pb.set_slices(1)
+    for i in range(2):
+        say(f"[case] n={n} B={B} run {i}")
+        pa.run(a, "persistent")
+        pb.run(b, "persistent")
+        assert a.compare(b) == (0, 0)
+
+
+def test_graph_replays_from_any_state(ps):
+    n, B = 40, 150
+    ops = mixed_ops(n, 500, 8, 0.1)
+    st, ref = (ps.CliffordState(n, B, 9, True) for _ in range(2))
+    prog, pref = ps.Program(st, ops), ps.Program(ref, ops)
+    pref.set_slices(1)
+    for i, reset in enumerate([False, False, True, False, True]):
+        say(f"[case] graph replay {i} reset={reset}")
+        if reset:
+            st.reset_clifford_state()
+            ref.reset_clifford_state()
+        prog.run(st, "graph")
+        pref.run(ref, "persistent")
+        assert st.compare(ref) == (0, 0)
+
+
+_RAW_POINTER = """
+import sys
+import torch  # first: its HIP runtime must be the one the process loads
+assert torch.cuda.is_available()
+sys.path[:0] = sys.argv[1:]
+import plaquette_simulator as ps
+from test_gpu_shared import mixed_ops
+n, B = 70, 200
+ops = mixed_ops(n, 600, 4, 0.1)
+for where in ("none", "first", "last"):
+    got = []
+    for per_shot in (False, True):
+        st = ps.CliffordState(n, B, 21, True)
+        planes = torch.from_dlpack(st.planes_dlpack()).view(torch.int64)
+        st.reset_clifford_state()
+        st.synchronize()
+        if where == "first":    # H on qubit 0 of the first 64 shots
+            planes[0, [0, n]] = planes[0, [n, 0]]
+        elif where == "last":   # z of the last row, in two shots
+            planes[-1, 2 * n - 1, 2 * n - 1] = 5
+        torch.cuda.synchronize()
+        prog = ps.Program(st, ops)
+        if per_shot:
+            prog.set_slices(1)
+        prog.run(st, "persistent")
+        st.synchronize()
+        got.append((st, planes))
+    assert got[0][0].compare(got[1][0]) == (0, 0), where
+    del got, planes, st
+print("raw pointer ok")
+"""
+
+
+def test_words_changed_through_the_raw_pointer(ps):
+    """The holder of the planes may change words between the reset and the run:
+    those word groups run per shot, the others packed.  (In a child process
+    that imports torch before the engine: each carries its own HIP runtime.)"""
+    pytest.importorskip("torch")
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    say("[case] words changed through the raw pointer (child process)")
+    r = subprocess.run([sys.executable, "-c", _RAW_POINTER,
+                        os.path.join(root, "plaquette-simulator_amd"),
+                        os.path.join(root, "tests"), os.path.join(root, "oracle")],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "raw pointer ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
