@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <chrono>
 #include <cstdio>
@@ -68,6 +69,8 @@ struct pq_batch_s {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   std::vector<uint64_t> graph_gens;  // arena generations at capture
+  // LDS of the k_batch_shared launches (columns in LDS, in the tableau; 0: none)
+  std::array<size_t, 2> shared_lds{};
   ~pq_batch_s();
   void drop_graph() {
     if (gexec) (void)hipGraphExecDestroy(gexec);
@@ -114,7 +117,7 @@ extern "C" int pq_batch_create(pq_batch *out) {
     return pq_set_error(PQ_ERR_NODEV, "no HIP device available");
   auto b = std::make_unique<pq_batch_s>();
   HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
-  HIPCHK(hipMalloc(&b->d_counter, sizeof(unsigned long long)));
+  HIPCHK(hipMalloc(&b->d_counter, 4 * sizeof(unsigned long long)));
   HIPCHK(hipEventCreate(&b->ev_upload));
   HIPCHK(hipEventCreate(&b->ev_a));
   HIPCHK(hipEventCreate(&b->ev_b));
@@ -266,8 +269,9 @@ static int enqueue(pq_batch b) {
   const bool tiled = b->wtile > 1;
   return launch_batch(b->stream, b->d_circ, nc, tiled ? b->d_titems : b->d_items,
                       tiled ? b->ntitems : b->nitems, b->d_counter, b->threads,
-                      launch_blocks(b), launch_lds(b), b->noise_tasks, chain_n,
-                      b->wtile) == hipSuccess
+                      launch_blocks(b), launch_lds(b), b->noise_tasks, chain_n, b->wtile,
+                      b->nitems, (uint32_t)cu_count(), b->shared_lds[0],
+                      b->shared_lds[1]) == hipSuccess
              ? PQ_OK
              : pq_set_error(PQ_ERR_HIP, "batch launch failed");
 }
@@ -419,17 +423,34 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
   HIPCHK(hipEventSynchronize(b->ev_upload));
   const uint32_t nc = (uint32_t)b->members.size();
   std::vector<uint64_t> gens(nc);
+  std::array<size_t, 2> shared_lds{};
   for (uint32_t c = 0; c < nc; ++c) {
     pq_state s = b->members[c].first;
     pq_program p = b->members[c].second;
     int rc = prepare_records(s, p);
     if (rc) return rc;
+    // from |0...0> the shared-X/Z kernel, as in a standalone run; a captured
+    // launch holds both kernels, and the members' arguments say which
+    // one runs each
+    uint32_t shared = 0;
+    if (s->tab && shared_allowed(s, p)) {
+      size_t &lds = shared_lds[shared_wide((uint32_t)s->n) ? 1 : 0];
+      lds = std::max(lds, shared_lds_bytes((uint32_t)s->n));
+      if (s->xz_identity) shared = s->exposed ? kSharedVerify : kSharedKnown;
+    }
+    if (shared == kSharedVerify && (rc = ensure_done(s, p))) return rc;
+    if (shared == kSharedKnown) {
+      s->xz_pending = false;
+      s->xz_plan.reset();
+    }
     if ((rc = materialize_tableau(s))) return rc;
     HIPCHK(hipStreamSynchronize(s->stream));  // the member's own queued work first
     if (p->done_ev) HIPCHK(hipEventSynchronize(p->done_ev));  // the program's last run
     BatchCircuit &bc = b->h_circ[c];
     bc.a = program_args(s, p, b->lds_budget);
     bc.a.census = nullptr;
+    bc.a.shared = shared;
+    bc.a.done = shared == kSharedVerify ? p->d_done : nullptr;
     bc.seed = (uint64_t)s->seed;
     bc.mseq0 = s->meas_seq;
     bc.nseq0 = s->noise_seq;
@@ -441,6 +462,8 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     s->noise_seq += p->nnoise;
     gens[c] = s->arena_gen;
   }
+  if (shared_lds != b->shared_lds) b->drop_graph();
+  b->shared_lds = shared_lds;
   if (form != PQ_RUN_FRAME) {
     int rc = tiled_items(b);  // allocates: before any capture
     if (rc) return rc;

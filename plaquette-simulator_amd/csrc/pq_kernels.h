@@ -122,11 +122,15 @@ struct BatchCircuit {
 // chain_qubits: the largest member of 193..512 qubits (0: none); such members
 // keep their determined chains in registers when the block has at most 512
 // threads (the large build), in LDS otherwise.
+// counter: four words, zeroed here: items taken by k_batch_t and by the two
+// k_batch_shared kernels (1, 3), and the word groups (of `groups`) that ran
+// there (2).  lds_packed, lds_wide: as in launch_batch_shared.
 hipError_t launch_batch(hipStream_t s, const BatchCircuit *circ, uint32_t ncirc,
                         const uint64_t *items, uint64_t nitems,
                         unsigned long long *counter, uint32_t threads,
                         uint32_t blocks, size_t lds_bytes, uint64_t noise_tasks,
-                        uint32_t chain_qubits, uint32_t wtile = 1);
+                        uint32_t chain_qubits, uint32_t wtile, uint64_t groups,
+                        uint32_t cus, size_t lds_packed, size_t lds_wide);
 hipError_t prepare_batch_kernel();
 // Dynamic LDS bytes k_program needs for n qubits and det_waves slabs.
 size_t program_lds_bytes(uint32_t n, uint32_t det_waves);
@@ -153,6 +157,16 @@ size_t shared_lds_bytes(uint32_t n);
 // Raises the kernels' dynamic-LDS limit for n qubits (not in a capture).
 hipError_t prepare_shared(uint32_t n);
 hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params);
+// Whether n qubits' packed columns sit in the tableau, not in the LDS.
+bool shared_wide(uint32_t n);
+// The batch members whose a.shared is set, before launch_batch (whose
+// work items, word tile and counters it shares).  lds_packed / lds_wide: most
+// LDS bytes of a member with its packed columns in LDS / in the tableau (0: no
+// such member).
+hipError_t prepare_batch_shared();
+hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const uint64_t *items,
+                               uint64_t nitems, unsigned long long *counter, uint32_t cus,
+                               size_t lds_packed, size_t lds_wide, uint32_t wtile);
 // Zeroes n 32-bit device words (a kernel: graph-capturable).
 hipError_t launch_zero_u32(hipStream_t s, unsigned int *p, uint32_t n);
 // Whether `slices` workgroups per word group for `nwords` groups of n qubits

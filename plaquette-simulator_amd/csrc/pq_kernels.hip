@@ -1720,10 +1720,11 @@ __global__ __launch_bounds__(MAXT) void k_program_t(pq::ProgramArgs a,
 template <int NREG, int MAXT>
 __global__ __launch_bounds__(MAXT) void k_batch_t(
     const pq::BatchCircuit *__restrict__ circ, const uint64_t *__restrict__ items,
-    uint64_t nitems, unsigned long long *counter, uint32_t wtile) {
+    uint64_t nitems, unsigned long long *counter, uint32_t wtile, uint64_t groups) {
   extern __shared__ uint64_t dyn[];
   __shared__ MeasShared sh;
   __shared__ uint64_t s_item;
+  if (counter[2] == groups) return;  // k_batch_shared ran every word group
   for (;;) {
     if (threadIdx.x == 0) s_item = atomicAdd(counter, 1ull);
     __syncthreads();
@@ -1737,8 +1738,11 @@ __global__ __launch_bounds__(MAXT) void k_batch_t(
     // an item is `wtile` consecutive word groups of one circuit (fewer at
     // the circuit's end)
     const uint64_t wend = min(w + wtile, bc.a.nwords);
-    for (uint64_t wi = w; wi < wend; ++wi)
+    if (bc.a.shared == kSharedKnown) continue;  // k_batch_shared ran them
+    for (uint64_t wi = w; wi < wend; ++wi) {
+      if (bc.a.done && bc.a.done[wi]) continue;
       program_word<NREG>(bc.a, bc.seed, bc.mseq0, wi, dyn, sh, nullptr);
+    }
   }
 }
 
@@ -1840,8 +1844,8 @@ __global__ __launch_bounds__(256) void k_batch_frame_noise(const pq::BatchCircui
   }
 }
 
-__global__ void k_zero_counter(unsigned long long *counter) {
-  if (threadIdx.x == 0) *counter = 0;
+__global__ void k_zero_counter(unsigned long long *counter, uint32_t n) {
+  if (threadIdx.x < n) counter[threadIdx.x] = 0;
 }
 
 
@@ -2211,7 +2215,7 @@ hipError_t launch_zero_u32(hipStream_t s, unsigned int *p, uint32_t n) {
 }
 
 hipError_t launch_zero_word(hipStream_t s, unsigned long long *p) {
-  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, p);
+  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, p, 1u);
   return hipGetLastError();
 }
 
@@ -2412,24 +2416,29 @@ hipError_t launch_batch(hipStream_t s, const BatchCircuit *circ, uint32_t ncirc,
                         const uint64_t *items, uint64_t nitems,
                         unsigned long long *counter, uint32_t threads,
                         uint32_t blocks, size_t lds_bytes, uint64_t noise_tasks,
-                        uint32_t chain_qubits, uint32_t wtile) {
+                        uint32_t chain_qubits, uint32_t wtile, uint64_t groups,
+                        uint32_t cus, size_t lds_packed, size_t lds_wide) {
   if (!nitems) return hipSuccess;
-  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, counter);
+  hipLaunchKernelGGL(k_zero_counter, dim3(1), dim3(64), 0, s, counter, 4u);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (noise_tasks) {
     e = launch_batch_frame_noise(s, circ, ncirc, noise_tasks);
     if (e != hipSuccess) return e;
   }
+  if (lds_packed || lds_wide) {
+    e = launch_batch_shared(s, circ, items, nitems, counter, cus, lds_packed, lds_wide, wtile);
+    if (e != hipSuccess) return e;
+  }
   // the large build only where a member's chains use it and the block fits it
   if (!large_build(chain_qubits, false) || threads > kLargeThreads)
     hipLaunchKernelGGL((k_batch_t<kSmallRegs, kSmallThreads>), dim3(blocks),
                        dim3(std::min<uint32_t>(threads, kSmallThreads)), lds_bytes, s, circ,
-                       items, nitems, counter, std::max<uint32_t>(wtile, 1));
+                       items, nitems, counter, std::max<uint32_t>(wtile, 1), groups);
   else
     hipLaunchKernelGGL((k_batch_t<kLargeRegs, kLargeThreads>), dim3(blocks),
                        dim3(std::min<uint32_t>(threads, kLargeThreads)), lds_bytes, s, circ,
-                       items, nitems, counter, std::max<uint32_t>(wtile, 1));
+                       items, nitems, counter, std::max<uint32_t>(wtile, 1), groups);
   return hipGetLastError();
 }
 
@@ -2438,6 +2447,7 @@ hipError_t prepare_batch_kernel() {
       ensure_lds_attr((const void *)k_batch_t<kSmallRegs, kSmallThreads>, kProgramLdsBudget);
   if (e == hipSuccess)
     e = ensure_lds_attr((const void *)k_batch_t<kLargeRegs, kLargeThreads>, kProgramLdsBudget);
+  if (e == hipSuccess) e = prepare_batch_shared();
   return e;
 }
 

@@ -695,9 +695,15 @@ static int choose_slices(pq_state s, pq_program p, const ProgramArgs &a, bool al
 // writes the whole tableau, where a shorter program touches a few columns),
 // no census (which counts the per-shot kernel's work) and no launch shape or
 // slice count asked for.
-static bool shared_allowed(const pq_state_s *s, const pq_program_s *p) {
+bool shared_allowed(const pq_state_s *s, const pq_program_s *p) {
   return p->uniform && shared_fits((uint32_t)s->n) && p->instrs.size() >= s->n &&
          !p->census_on && !p->slices_set && p->threads >= 256;
+}
+
+int ensure_done(pq_state s, pq_program p) {
+  if (!p->d_done)
+    HIPCHK(dev_alloc((void **)&p->d_done, s->W * sizeof(uint32_t), p->alloc_stream));
+  return PQ_OK;
 }
 
 // shared: 0 the per-shot kernel, kSharedKnown the shared-X/Z kernel,
@@ -798,8 +804,7 @@ static int program_run(pq_state s, pq_program p, int form) {
   if ((form == PQ_RUN_PERSISTENT && s->xz_identity) || form == PQ_RUN_GRAPH)
     if (shared_allowed(s, p))
       shared = form == PQ_RUN_GRAPH || s->exposed ? kSharedVerify : kSharedKnown;
-  if (shared == kSharedVerify && !p->d_done)
-    HIPCHK(dev_alloc((void **)&p->d_done, s->W * sizeof(uint32_t), p->alloc_stream));
+  if (shared == kSharedVerify && (rc = ensure_done(s, p))) return rc;
   if (shared == kSharedKnown) {
     s->xz_pending = false;
     s->xz_plan.reset();

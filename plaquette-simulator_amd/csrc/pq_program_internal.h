@@ -85,6 +85,10 @@ constexpr uint64_t kProgramLdsBytes = 158 * 1024;  // dynamic-LDS cap (kProgramL
 int check_records(pq_state s, pq_program p);
 int prepare_records(pq_state s, pq_program p);
 pq::ProgramArgs program_args(pq_state s, pq_program p, uint64_t lds_budget);
+// Whether a persistent run of p on s from |0...0> may take the shared-X/Z
+// kernel, and the flags a run that verifies the tableau needs.
+bool shared_allowed(const pq_state_s *s, const pq_program_s *p);
+int ensure_done(pq_state s, pq_program p);
 // pq_program_create for a server-owned state: stream-ordered allocation and
 // copies on the state's stream.
 int create_program_on(pq_state s, const pq_op *ops, uint64_t nops, pq_program *out);

@@ -93,6 +93,10 @@ __host__ __device__ inline uint64_t shared_packed_words(uint32_t n) {
   return 2ull * n * (2ull * ((n + 63) / 64) + 1);
 }
 
+__host__ __device__ inline bool packed_in_lds(uint32_t n) {
+  return (shared_base_words(n) + shared_packed_words(n)) * 8 <= kSharedLdsBytes;
+}
+
 // One staged gate-segment op: `cw` = code (bits 0-7), has noise or a flag
 // (bit 8), ops of the layer part it opens inside the chunk (bits 10-20);
 // `qq` = qa | qb << 16.
@@ -685,13 +689,42 @@ __global__ __launch_bounds__(kSharedThreads) void k_program_shared(
   }
 }
 
+// The members of a mixed batch that may run packed: work items (circuit << 40 |
+// word group), taken from counter[1] (columns in LDS) or counter[3] (in the
+// tableau); counter[2] counts the word groups that ran.  k_batch_t runs what is
+// left.
+template <bool kLds>
+__global__ __launch_bounds__(kSharedThreads) void k_batch_shared(
+    const BatchCircuit *__restrict__ circ, const uint64_t *__restrict__ items, uint64_t nitems,
+    unsigned long long *counter, uint32_t wtile) {
+  extern __shared__ uint64_t dyn[];
+  __shared__ SharedLds sh;
+  for (;;) {
+    if (threadIdx.x == 0) sh.item = atomicAdd(counter + (kLds ? 1 : 3), 1ull);
+    __syncthreads();
+    const uint64_t it = rfl64(sh.item);
+    __syncthreads();
+    if (it >= nitems) break;
+    const uint64_t code = rfl64(items[it]);
+    const BatchCircuit &bc = circ[(uint32_t)(code >> 40)];
+    if (!bc.a.shared || packed_in_lds(bc.a.n) != kLds) continue;
+    const uint64_t w = code & ((1ull << 40) - 1);
+    const uint64_t wend = min(w + wtile, bc.a.nwords);
+    for (uint64_t wi = w; wi < wend; ++wi) {
+      const bool ran = shared_word<kLds>(bc.a, bc.seed, bc.mseq0, wi, dyn, sh);
+      if (threadIdx.x == 0) {
+        if (bc.a.done) bc.a.done[wi] = ran ? 1u : 0u;
+        if (ran) atomicAdd(counter + 2, 1ull);
+      }
+    }
+  }
+}
+
 }  // namespace
 
-bool shared_fits(uint32_t n) { return n >= 1 && n <= kSharedMaxQubits; }
+bool shared_wide(uint32_t n) { return !packed_in_lds(n); }
 
-static bool packed_in_lds(uint32_t n) {
-  return (shared_base_words(n) + shared_packed_words(n)) * 8 <= kSharedLdsBytes;
-}
+bool shared_fits(uint32_t n) { return n >= 1 && n <= kSharedMaxQubits; }
 
 size_t shared_lds_bytes(uint32_t n) {
   return 8 * (shared_base_words(n) + (packed_in_lds(n) ? shared_packed_words(n) : 0));
@@ -704,6 +737,33 @@ hipError_t prepare_shared(uint32_t n) {
                                     : (const void *)k_program_shared<false>;
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)kSharedLdsBytes);
+}
+
+hipError_t prepare_batch_shared() {
+  hipError_t e = hipSuccess;
+  for (const void *fn : {(const void *)k_batch_shared<true>, (const void *)k_batch_shared<false>})
+    if (e == hipSuccess)
+      e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)kSharedLdsBytes);
+  return e;
+}
+
+hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const uint64_t *items,
+                               uint64_t nitems, unsigned long long *counter, uint32_t cus,
+                               size_t lds_packed, size_t lds_wide, uint32_t wtile) {
+  wtile = std::max<uint32_t>(wtile, 1);
+  // as many workgroups per CU as the largest member's LDS allows
+  auto blocks = [&](size_t lds) {
+    return dim3((uint32_t)std::min<uint64_t>(
+        nitems, cus * std::min<uint64_t>(4, std::max<uint64_t>(1, 160 * 1024 / (lds + 1024)))));
+  };
+  if (nitems && lds_packed)
+    hipLaunchKernelGGL(k_batch_shared<true>, blocks(lds_packed), dim3(kSharedThreads), lds_packed,
+                       s, circ, items, nitems, counter, wtile);
+  if (nitems && lds_wide)
+    hipLaunchKernelGGL(k_batch_shared<false>, blocks(lds_wide), dim3(kSharedThreads), lds_wide, s,
+                       circ, items, nitems, counter, wtile);
+  return hipGetLastError();
 }
 
 hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params) {

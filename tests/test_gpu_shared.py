@@ -166,3 +166,40 @@ def test_words_changed_through_the_raw_pointer(ps):
                         os.path.join(root, "tests"), os.path.join(root, "oracle")],
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "raw pointer ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("form", ["persistent", "graph"])
+def test_batch_members_in_both_kernels(ps, form):
+    """A batch of members with packed columns in LDS and in the tableau, one with
+    a flagged H (per shot), run from |0...0>, then from the states that left, then
+    with one member reset: every member equals its standalone per-shot run."""
+    from plaquette_simulator import workloads as W
+    specs = [(40, 200, mixed_ops(40, 300, 1, 0.1)), (500, 130, mixed_ops(500, 700, 2, 0.03)),
+             (9, 65, mixed_ops(9, 200, 3, 0.2))]
+    b = W.OpList()
+    for q in range(12):
+        b.h(q)
+        b.with_prob(W.OP_H, q, 0.4)
+        b.cx(q, (q + 1) % 12)
+    for q in range(12):
+        b.measure(q)
+    specs.append((12, 100, b.array()))
+    batch, got, ref = ps.Batch(), [], []
+    for i, (n, B, ops) in enumerate(specs):
+        st, rs = (ps.CliffordState(n, B, 50 + i, True) for _ in range(2))
+        prog, rp = ps.Program(st, ops), ps.Program(rs, ops)
+        rp.set_slices(1)
+        batch.add(st, prog)
+        got.append((st, prog))
+        ref.append((rs, rp))
+    batch.set_word_tile(2)
+    for step in range(3):
+        say(f"[case] batch {form} step {step}")
+        if step == 2:
+            got[0][0].reset_clifford_state()
+            ref[0][0].reset_clifford_state()
+        batch.run(form)
+        batch.wait()
+        for (st, _), (rs, rp) in zip(got, ref):
+            rp.run(rs, "persistent")
+            assert st.compare(rs) == (0, 0)
