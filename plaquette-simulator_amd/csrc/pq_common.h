@@ -72,7 +72,8 @@ PQ_HD void add_mod4(uint64_t &a0, uint64_t &a1, uint64_t b0, uint64_t b1) {
 //  chunk, the number of ops in that part (bits 20-30);
 //  PQ_OP_NOISE alone: qa, na;  M: qa, slot = record id, t0 = coin
 //  threshold, (na, nb) = coin stream (low, high 32 bits), pad = kMeasSuperseded
-//  when a later M of the same measurement segment writes the same record.
+//  when a later M of the same measurement segment writes the same record, and
+//  from bit 8 the Ms left in the segment, this one included.
 struct DInstr {
   uint32_t code, qa, qb, slot, na, nb, t0, pad;
 };
@@ -89,6 +90,7 @@ constexpr uint32_t kLayerLenMask = 0x7FFu;
 // last write in program order is the one that stays even when both run at
 // once in a batch of fully determined measurements.
 constexpr uint32_t kMeasSuperseded = 1u;
+constexpr uint32_t kMeasLeftShift = 8;
 
 // Segment of a compiled program: a run of gate batches or a run of
 // measurements.  Gate segments hold `count` instructions in batches.  A gate

@@ -70,6 +70,7 @@ struct ProgramArgs {
   const DInstr *instrs;
   const uint64_t *coin_planes;  // optional replay planes [m][W] or nullptr
   uint32_t nseg;
+  uint32_t ninstr;
   uint32_t n, R, C;
   uint64_t W;
   uint64_t word0;  // first word group handled by this launch
@@ -151,7 +152,6 @@ hipError_t launch_program(hipStream_t s, const ProgramArgs &a, uint32_t threads,
 // flagged H/S/CX/CZ on the |0...0> tableau, one workgroup per word group.
 constexpr uint32_t kSharedThreads = 768;
 constexpr uint32_t kSharedMaxQubits = 2048;
-constexpr uint64_t kSharedLdsBytes = 158 * 1024;
 bool shared_fits(uint32_t n);
 size_t shared_lds_bytes(uint32_t n);
 // Raises the kernels' dynamic-LDS limit for n qubits (not in a capture).

@@ -343,6 +343,7 @@ int compile_program(pq_program_s *p) {
             pad = kMeasSuperseded;
             break;
           }
+        pad |= (uint32_t)std::min<uint64_t>(j - k, 0xFFFFFFu) << kMeasLeftShift;
         DInstr I{PQ_OP_M, ops[k].q0, 0, ops[k].slot, nmeas, 0, ops[k].t0, pad};
         ++nmeas;
         p->instrs.push_back(I);
@@ -619,6 +620,7 @@ ProgramArgs program_args(pq_state s, pq_program p, uint64_t lds_budget) {
   a.instrs = p->d_instrs;
   a.coin_planes = nullptr;
   a.nseg = (uint32_t)p->segs.size();
+  a.ninstr = (uint32_t)p->instrs.size();
   a.n = (uint32_t)s->n;
   a.R = (uint32_t)s->R;
   a.C = (uint32_t)s->C;

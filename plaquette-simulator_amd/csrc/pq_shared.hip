@@ -21,8 +21,8 @@
 // What this saves: the per-shot kernel (k_program_t) moves and computes
 // R = 2n+1 words of 64 shots per column and gate; here a column is 2 n/64 words
 // of rows.  n <= about 460: the packed columns (2n (2 n/64 + 1) words) sit in
-// LDS; up to 2048 qubits they sit at the start of their own column of the
-// group's tableau block, which the run overwrites anyway (L2-resident).
+// LDS; up to 2048 qubits they sit at the start of the group's tableau block,
+// which the run overwrites anyway.
 #include "pq_kernels.h"
 
 #include <algorithm>
@@ -36,7 +36,7 @@ namespace {
 #define PQ_CONST __attribute__((address_space(4)))
 
 constexpr uint32_t kChunk = 448;       // staged ops; must equal kStage in pq_kernels.hip
-constexpr uint32_t kChunkWords = kChunk * 5;
+constexpr uint32_t kWideCols = 6;      // columns a lane has in flight (wide states)
 constexpr uint32_t kWindow = 64;       // measurements whose pivots are checked at once
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
@@ -75,34 +75,50 @@ __device__ __forceinline__ uint32_t wave_sum_bit1(uint32_t v) {
   return ((b0 >> 1) ^ b1) & 1u;
 }
 
-struct SharedLds {
-  uint32_t bad;     // a word of the state is not the |0...0> tableau's
-  uint32_t tot;     // determined measurement (wide states): phase count
-  uint64_t piv;     // pivot check: measurements of the window with a pivot
-  uint64_t rx;      // determined measurement (wide states): XOR of Rv rows
-  uint64_t item;
-};
-
-// LDS words besides the packed columns: Rv, E, four KW-word row masks, the
-// staged ops.
-__host__ __device__ inline uint64_t shared_base_words(uint32_t n) {
-  const uint64_t KW = 2ull * ((n + 63) / 64) + 1;
-  return (2ull * n + 1) + 2ull * n + 4 * KW + kChunkWords;
-}
-__host__ __device__ inline uint64_t shared_packed_words(uint32_t n) {
-  return 2ull * n * (2ull * ((n + 63) / 64) + 1);
-}
-
-__host__ __device__ inline bool packed_in_lds(uint32_t n) {
-  return (shared_base_words(n) + shared_packed_words(n)) * 8 <= kSharedLdsBytes;
-}
-
-// One staged gate-segment op: `cw` = code (bits 0-7), has noise or a flag
-// (bit 8), ops of the layer part it opens inside the chunk (bits 10-20);
-// `qq` = qa | qb << 16.
+// One staged op: `cw` = the flags below, and from bit 12 the ops of the layer
+// part it opens, or the measurements left in its run; `qq` = qa | qb << 16 (qb
+// = qa for one-qubit ops).  Its four masks are what the op and the noise after
+// it XOR into the frame's x and z words of qa and of qb; an op flagged by a
+// record keeps the flag in the third and the record in the fourth.  A
+// measurement's first two hold record | coin threshold << 32 and the sequence
+// number.
 struct SharedOp {
   uint32_t cw, qq;
 };
+constexpr uint32_t kOpH = 1, kOpS = 2, kOpCX = 4, kOpCZ = 8, kOpGate = 15;
+constexpr uint32_t kOpMeas = 1u << 4;
+constexpr uint32_t kOpMasks = 1u << 5;    // some mask word is not zero
+constexpr uint32_t kOpRecX = 1u << 6;     // a record's flag goes to x
+constexpr uint32_t kOpRecZ = 1u << 7;     // ... to z
+constexpr uint32_t kOpDropped = 1u << 8;  // a later measurement writes its record
+constexpr uint32_t kOpRandom = 1u << 9;   // a measurement found random (set when it runs)
+constexpr uint32_t kOpLenShift = 12, kOpLenMask = 0xFFFu;
+
+constexpr uint32_t kMaxRowWords = 2 * (kSharedMaxQubits / 64) + 2;
+struct SharedLds {
+  SharedOp ops[kChunk + 1];
+  uint64_t msk[4 * kChunk];
+  uint64_t rc[kMaxRowWords];  // sign bits, laid out like a column
+  uint64_t sm[kMaxRowWords];  // row mask of the current random measurement
+  uint64_t c0[kMaxRowWords];  // and the low bits of its rows' phase sums
+  uint32_t list[512];         // its pivot row's columns (packed columns in LDS)
+  uint32_t bad;               // a word of the state is not the |0...0> tableau's
+  // determined measurements of wide states, two in turn: phase count, XOR of
+  // Rv rows
+  uint32_t tot[2];
+  uint64_t rx[2];
+  uint32_t nl;                // entries of list
+  uint64_t item;
+};
+constexpr uint64_t kSharedLdsBytes = 159 * 1024 - sizeof(SharedLds);  // dynamic LDS cap
+
+// Dynamic LDS words: Rv, the frame, and the packed columns if they fit.
+__host__ __device__ inline uint64_t packed_words(uint32_t n) {
+  return (2ull * n + 1) + 2ull * n + 2ull * n * (2ull * ((n + 63) / 64) + 1);
+}
+__host__ __device__ inline bool packed_in_lds(uint32_t n) {
+  return packed_words(n) * 8 <= kSharedLdsBytes;
+}
 
 // Runs the program on word group w.  Returns false, with the state untouched,
 // if a.shared asks to verify that the group's X/Z are the |0...0> tableau and
@@ -113,22 +129,19 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
   const uint32_t tid = threadIdx.x, NT = blockDim.x, lane = lane_id();
   const uint32_t wv = rfl(tid >> 6), nw = NT >> 6;
   const uint32_t n = a.n, R = a.R;
-  const uint32_t KH = (n + 63) / 64, KW = 2 * KH + 1;
+  const uint32_t KH = (n + 63) / 64, K2 = 2 * KH, KW = K2 + 1;
   const uint64_t W = a.W;
   uint64_t *T = a.tab + w * (uint64_t)a.C * R;
   uint64_t *Tr = T + 2ull * n * R;  // the R column
+  // packed column c (x_c, or z_{c-n}) starts at P + c * KW: one compact block,
+  // in LDS or at the start of the group's tableau block.  (At a stride of the
+  // tableau's own columns, 2n+1 words, neighbouring columns fall on one L2
+  // channel.)
   uint64_t *Rv = dyn;
-  uint64_t *E = Rv + R;             // E.x[0..n), E.z[n..2n)
-  uint64_t *rc = E + 2 * n;         // sign bits, laid out like a column
-  uint64_t *sm = rc + KW;           // row mask of the current measurement
-  uint64_t *s_c0 = sm + KW, *s_c1 = s_c0 + KW;
-  uint64_t *s_msk = s_c1 + KW;
-  SharedOp *s_ops = reinterpret_cast<SharedOp *>(s_msk + 4 * kChunk);
-  // packed column c (x_c, or z_{c-n}) starts at P + c * stride
-  uint64_t *P = kLds ? s_msk + kChunkWords : T;
-  const uint32_t stride = kLds ? KW : R;
+  uint64_t *E = Rv + R;  // E.x[0..n), E.z[n..2n)
+  uint64_t *P = kLds ? E + 2 * n : T;
+  uint64_t *const rc = sh.rc;
   const PQ_CONST DInstr *ins = (const PQ_CONST DInstr *)a.instrs;
-  const PQ_CONST DSegment *segs = (const PQ_CONST DSegment *)a.segs;
   const PQ_CONST uint64_t *gp = (const PQ_CONST uint64_t *)a.planes + 2ull * a.nk * w;
 
   if (a.shared == kSharedVerify) {
@@ -160,434 +173,332 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
     const uint32_t c = u / KW, k = u - c * KW;
     const uint32_t q = c < n ? c : c - n;
     const uint32_t kq = (c < n ? 0 : KH) + (q >> 6);
-    P[c * stride + k] = k == kq ? 1ull << (q & 63) : 0ull;
+    P[c * KW + k] = k == kq ? 1ull << (q & 63) : 0ull;
   }
   for (uint32_t i = tid; i < R; i += NT) Rv[i] = Tr[i];
   for (uint32_t i = tid; i < 2 * n; i += NT) E[i] = 0;
   if (tid < KW) rc[tid] = 0;
+  if (tid < 2) {
+    sh.tot[tid] = 0;
+    sh.rx[tid] = 0;
+  }
   __syncthreads();
 
   // this thread's share of a layer's column work: word my_k of every opp-th op
   const uint32_t opp = NT / KW;
   const uint32_t my_op = tid / KW, my_k = tid - my_op * KW;
   const bool on = my_op < opp;
+  // and of a random measurement's: word my_i of every rpp-th of its columns
+  const uint32_t rpp = NT / K2;
+  const uint32_t my_j = tid / K2, my_i = tid - my_j * K2;
 
-  for (uint32_t si = 0; si < a.nseg; ++si) {
-    const uint32_t kind = segs[si].kind, sbegin = segs[si].begin, scount = segs[si].count;
-    const uint32_t send = sbegin + scount;
-    if (kind == 0) {
-      uint64_t rp = 0;  // sign flips of row word my_k
-      for (uint32_t cb = sbegin; cb < send; cb += kChunk) {
-        const uint32_t cn = min(kChunk, send - cb);
-        for (uint32_t t = tid; t < cn; t += NT) {
-          const PQ_CONST DInstr *I = ins + cb + t;
-          const uint32_t code = I->code, na = I->na, nb = I->nb, slot = I->slot, pad = I->pad;
-          uint64_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
-          if (na != kNone) {
-            m0 = gp[2ull * na];
-            m1 = gp[2ull * na + 1];
-          }
-          if (nb != kNone) {
-            m2 = gp[2ull * nb];
-            m3 = gp[2ull * nb + 1];
-          } else if (code >= PQ_OP_H_FLAG && code != PQ_OP_NOISE) {
-            m2 = (slot & kSlotPlane) ? gp[2ull * (slot & ~kSlotPlane)]
-                                     : a.recs[(2ull * slot) * W + w];
-          }
-          SharedOp J;
-          J.cw = code | ((m0 | m1 | m2 | m3) ? 1u << 8 : 0u) |
-                 (((pad >> kLayerLenShift) & kLayerLenMask) << 10);
-          J.qq = I->qa | (I->qb << 16);
-          s_ops[t] = J;
-          s_msk[4 * t + 0] = m0;
-          s_msk[4 * t + 1] = m1;
-          s_msk[4 * t + 2] = m2;
-          s_msk[4 * t + 3] = m3;
+  uint64_t rp = 0;    // sign flips of row word my_k, not yet in rc
+  uint32_t slot2 = 0; // which of sh.tot / sh.rx is in use (wide states)
+  for (uint32_t base = 0; base < a.ninstr;) {
+    const uint32_t wn = min(kChunk, a.ninstr - base);
+    // instructions [base, base + wn) and their masks, whatever segments they
+    // belong to: two dependent loads per window, not per segment
+    bool flags = false;
+    for (uint32_t t = tid; t < wn; t += NT) {
+      const PQ_CONST DInstr *I = ins + base + t;
+      const uint32_t code = I->code, qa = I->qa, qb = I->qb, slot = I->slot, na = I->na,
+                     nb = I->nb, t0 = I->t0, pad = I->pad;
+      SharedOp J;
+      uint64_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
+      if (code == PQ_OP_M) {
+        J.cw = kOpMeas | (pad & kMeasSuperseded ? kOpDropped : 0u) |
+               (min(pad >> kMeasLeftShift, kChunk) << kOpLenShift);
+        J.qq = qa;
+        m0 = (uint64_t)slot | ((uint64_t)t0 << 32);
+        m1 = (uint64_t)na | ((uint64_t)nb << 32);
+      } else {
+        if (na != kNone) {
+          m0 = gp[2ull * na];
+          m1 = gp[2ull * na + 1];
         }
-        __syncthreads();
-        uint32_t b = 0;
-        while (b < cn) {
-          // a layer's ops act on distinct qubits: no barrier inside it
-          const uint32_t cnt = max(1u, (rfl(s_ops[b].cw) >> 10) & kLayerLenMask);
-          if (on) {
-            for (uint32_t o = my_op; o < cnt; o += opp) {
-              const SharedOp J = s_ops[b + o];
-              const uint32_t code = J.cw & 0xFFu, qa = J.qq & 0xFFFFu, qb = J.qq >> 16;
-              uint64_t *xa = P + (qa * stride + my_k), *za = xa + n * stride;
-              if (code == PQ_OP_CX) {
-                uint64_t *xb = P + (qb * stride + my_k), *zb = xb + n * stride;
-                const uint64_t x = *xa, z = *za, xt = *xb, zt = *zb;
-                rp ^= x & zt & ~(xt ^ z);
-                *xb = xt ^ x;
-                *za = z ^ zt;
-              } else if (code == PQ_OP_H) {
-                const uint64_t x = *xa, z = *za;
-                rp ^= x & z;
-                *xa = z;
-                *za = x;
-              } else if (code == PQ_OP_S) {
-                const uint64_t x = *xa, z = *za;
-                rp ^= x & z;
-                *za = z ^ x;
-              } else if (code == PQ_OP_CZ) {
-                uint64_t *xb = P + (qb * stride + my_k), *zb = xb + n * stride;
-                const uint64_t x = *xa, z = *za, xt = *xb, zt = *zb;
-                rp ^= x & xt & (zt ^ z);
-                *zb = zt ^ x;
-                *za = z ^ xt;
-              }
-            }
-          }
-          // the frame words, from the last threads down (the column work
-          // starts at thread 0)
-          for (uint32_t o = NT - 1 - tid; o < cnt; o += NT) {
-            const SharedOp J = s_ops[b + o];
-            const uint32_t code = J.cw & 0xFFu, qa = J.qq & 0xFFFFu, qb = J.qq >> 16;
-            const uint64_t *M = s_msk + 4 * (b + o);
-            uint64_t ex = E[qa], ez = E[n + qa];
-            const bool noisy = (J.cw >> 8) & 1u;
-            switch (code) {
-              case PQ_OP_H: {
-                const uint64_t t = ex;
-                ex = ez;
-                ez = t;
-                break;
-              }
-              case PQ_OP_S: ez ^= ex; break;
-              case PQ_OP_X: ex = ~ex; break;
-              case PQ_OP_Y: ex = ~ex; ez = ~ez; break;
-              case PQ_OP_Z: ez = ~ez; break;
-              case PQ_OP_CX:
-              case PQ_OP_CZ: {
-                uint64_t fx = E[qb], fz = E[n + qb];
-                if (code == PQ_OP_CX) {
-                  fx ^= ex;
-                  ez ^= fz;
-                } else {
-                  fz ^= ex;
-                  ez ^= fx;
-                }
-                if (noisy) {
-                  fx ^= M[2];
-                  fz ^= M[3];
-                }
-                E[qb] = fx;
-                E[n + qb] = fz;
-                break;
-              }
-              case PQ_OP_X_FLAG: ex ^= M[2]; break;
-              case PQ_OP_Y_FLAG: ex ^= M[2]; ez ^= M[2]; break;
-              case PQ_OP_Z_FLAG: ez ^= M[2]; break;
-              default: break;  // PQ_OP_NOISE: the masks below
-            }
-            if (noisy) {
-              ex ^= M[0];
-              ez ^= M[1];
-            }
-            E[qa] = ex;
-            E[n + qa] = ez;
-          }
-          b += cnt;
+        if (nb != kNone) {
+          m2 = gp[2ull * nb];
+          m3 = gp[2ull * nb + 1];
+        }
+        const bool two = code == PQ_OP_CX || code == PQ_OP_CZ;
+        const bool px = code == PQ_OP_X || code == PQ_OP_Y || code == PQ_OP_X_FLAG ||
+                        code == PQ_OP_Y_FLAG;
+        const bool pz = code == PQ_OP_Z || code == PQ_OP_Y || code == PQ_OP_Z_FLAG ||
+                        code == PQ_OP_Y_FLAG;
+        uint32_t rec = 0;
+        if (code >= PQ_OP_H_FLAG && code != PQ_OP_NOISE && !(slot & kSlotPlane)) {
+          rec = (px ? kOpRecX : 0u) | (pz ? kOpRecZ : 0u);
+          m2 = a.recs[(2ull * slot) * W + w];
+          m3 = slot;
+          flags = true;
+        } else if (px || pz) {
+          const uint64_t f =
+              code >= PQ_OP_H_FLAG ? gp[2ull * (slot & ~kSlotPlane)] : ~0ull;
+          if (px) m0 ^= f;
+          if (pz) m1 ^= f;
+        }
+        J.cw = (code == PQ_OP_H ? kOpH : code == PQ_OP_S ? kOpS : 0u) |
+               (code == PQ_OP_CX ? kOpCX : code == PQ_OP_CZ ? kOpCZ : 0u) |
+               ((m0 | m1 | m2 | m3) ? kOpMasks : 0u) | rec |
+               (((pad >> kLayerLenShift) & kLayerLenMask) << kOpLenShift);
+        J.qq = qa | ((two ? qb : qa) << 16);
+      }
+      sh.ops[t] = J;
+      sh.msk[4 * t + 0] = m0;
+      sh.msk[4 * t + 1] = m1;
+      sh.msk[4 * t + 2] = m2;
+      sh.msk[4 * t + 3] = m3;
+    }
+    // flags from records are read again where measurements of this window
+    // precede them
+    const bool reread = __syncthreads_or(flags);
+    bool measured = false;
+    uint32_t b = 0;
+    uint32_t cw = rfl(sh.ops[0].cw);  // of op b
+    while (b < wn) {
+      const uint32_t cnt = max(1u, (cw >> kOpLenShift) & kOpLenMask);
+      if (!(cw & kOpMeas)) {
+        if (b + cnt > wn) break;  // a layer part runs whole: it opens the next window
+        if (measured && reread) {
+          for (uint32_t t = b + tid; t < wn; t += NT)
+            if (sh.ops[t].cw & (kOpRecX | kOpRecZ))
+              sh.msk[4 * t + 2] = a.recs[2ull * sh.msk[4 * t + 3] * W + w];
           __syncthreads();
         }
+        measured = false;
+        // a layer's ops act on distinct qubits: no barrier inside it
+        if (on)
+          for (uint32_t o = my_op; o < cnt; o += opp) {
+            const SharedOp J = sh.ops[b + o];
+            uint64_t *xa = P + (__umul24(J.qq & 0xFFFFu, KW) + my_k), *za = xa + n * KW;
+            if (J.cw & kOpCX) {
+              uint64_t *xb = P + (__umul24(J.qq >> 16, KW) + my_k), *zb = xb + n * KW;
+              const uint64_t x = *xa, z = *za, xt = *xb, zt = *zb;
+              rp ^= x & zt & ~(xt ^ z);
+              *xb = xt ^ x;
+              *za = z ^ zt;
+            } else if (J.cw & kOpH) {
+              const uint64_t x = *xa, z = *za;
+              rp ^= x & z;
+              *xa = z;
+              *za = x;
+            } else if (J.cw & kOpS) {
+              const uint64_t x = *xa, z = *za;
+              rp ^= x & z;
+              *za = z ^ x;
+            } else if (J.cw & kOpCZ) {
+              uint64_t *xb = P + (__umul24(J.qq >> 16, KW) + my_k), *zb = xb + n * KW;
+              const uint64_t x = *xa, z = *za, xt = *xb, zt = *zb;
+              rp ^= x & xt & (zt ^ z);
+              *zb = zt ^ x;
+              *za = z ^ xt;
+            }
+          }
+        // The frame moves through a gate as a row does.  Its words are for the
+        // last threads: the column work starts at thread 0, and a wave's
+        // instruction stream is the bound here, not the SIMD.
+        for (uint32_t o = NT - 1 - tid; o < cnt; o += NT) {
+          const SharedOp J = sh.ops[b + o];
+          const uint32_t qa = J.qq & 0xFFFFu, qb = J.qq >> 16;
+          const uint64_t *M = sh.msk + 4 * (b + o);
+          uint64_t ex = E[qa], ez = E[n + qa];
+          if (J.cw & (kOpCX | kOpCZ)) {
+            uint64_t fx = E[qb], fz = E[n + qb];
+            if (J.cw & kOpCX) {
+              fx ^= ex;
+              ez ^= fz;
+            } else {
+              fz ^= ex;
+              ez ^= fx;
+            }
+            E[qb] = fx ^ M[2];
+            E[n + qb] = fz ^ M[3];
+          } else if (J.cw & kOpH) {
+            const uint64_t t = ex;
+            ex = ez;
+            ez = t;
+          } else if (J.cw & kOpS) {
+            ez ^= ex;
+          } else {
+            if (J.cw & kOpRecX) ex ^= M[2];
+            if (J.cw & kOpRecZ) ez ^= M[2];
+          }
+          if (J.cw & kOpMasks) {
+            ex ^= M[0];
+            ez ^= M[1];
+          }
+          E[qa] = ex;
+          E[n + qa] = ez;
+        }
+        b += cnt;
+        cw = rfl(sh.ops[b].cw);
+        __syncthreads();
+        continue;
       }
-      if (on && rp) lds_xor(rc + my_k, rp);
-      __syncthreads();
-      continue;
-    }
 
-    // ---- measurements ----
-    for (uint32_t mb = sbegin; mb < send; mb += kChunk) {
-      const uint32_t mn = min(kChunk, send - mb);
-      // staged: qubit | record << 32, coin threshold | pad << 32, sequence number
-      for (uint32_t t = tid; t < mn; t += NT) {
-        const PQ_CONST DInstr *I = ins + mb + t;
-        s_msk[4 * t + 0] = (uint64_t)I->qa | ((uint64_t)I->slot << 32);
-        s_msk[4 * t + 1] = (uint64_t)I->t0 | ((uint64_t)I->pad << 32);
-        s_msk[4 * t + 2] = (uint64_t)I->na | ((uint64_t)I->nb << 32);
+      // ---- measurements [b, b + mn) ----
+      if (!measured) {
+        if (on && rp) lds_xor(rc + my_k, rp);
+        rp = 0;
+        __syncthreads();
       }
-      if (!kLds && tid == 0) sh.piv = 0;
-      __syncthreads();
-      uint32_t k = 0;
-      while (k < mn) {
-        // which of the next measurements have a pivot (a stabilizer row
-        // with x_q set)?
-        uint32_t nm = min(mn - k, kWindow);
-        uint64_t piv;
+      measured = true;
+      const uint32_t mbeg = b, mend = min(wn, b + cnt);
+      while (b < mend) {
+        // Which of the next measurements have a pivot (a stabilizer row with
+        // x_q set)?  Every wave finds out by itself.  A determined one's
+        // outcome stays what it is while others are measured, so with the
+        // columns in LDS those wait for the end of the run, to share the
+        // waves.  Wide states: one measurement at a time, lane i keeping word i
+        // of x_q.
+        uint32_t nm, jr;
+        uint64_t xqv = 0;
         if (kLds) {
+          nm = min(mend - b, kWindow);
           uint64_t acc = 0;
           if (lane < nm) {
-            const uint64_t *xq = P + (uint32_t)s_msk[4 * (k + lane)] * stride + KH;
-            for (uint32_t i = 0; i < KH; ++i) acc |= xq[i];
+            const uint64_t *xq = P + __umul24(sh.ops[b + lane].qq, KW) + KH;
+            for (uint32_t i = 0; i < KH; i += 4)
+              acc |= xq[i] | xq[min(i + 1, KH - 1)] | xq[min(i + 2, KH - 1)] |
+                     xq[min(i + 3, KH - 1)];
           }
-          piv = __ballot(acc != 0);
+          const uint64_t piv = __ballot(acc != 0);
+          jr = piv ? (uint32_t)__ffsll((long long)piv) - 1 : nm;
         } else {
-          nm = min(nm, NT / KH);
-          const uint32_t i = tid / KH, kk = tid - i * KH;
-          if (i < nm && P[(uint32_t)s_msk[4 * (k + i)] * stride + KH + kk])
-            atomicOr(reinterpret_cast<unsigned long long *>(&sh.piv), 1ull << i);
-          __syncthreads();
-          piv = rfl64(sh.piv);
-          __syncthreads();
-          if (tid == 0) sh.piv = 0;
+          nm = 1;
+          xqv = lane < K2 ? P[sh.ops[b].qq * KW + lane] : 0ull;
+          jr = (__ballot(xqv != 0) >> KH) ? 0u : 1u;
         }
-        const uint32_t jr = piv ? (uint32_t)__ffsll((long long)piv) - 1 : nm;
 
-        // measurements [k, k + jr) are determined: the outcome is the sign of
-        // the product, in ascending order, of the stabilizers whose
-        // destabilizer has x_q set, which is Z_q up to that sign.  Writing a
-        // Pauli row as i^y X^x Z^z (y the number of Y's), the product's
-        // phase is i^(sum y) times -1 for every earlier z that meets a later x:
-        // per column, a prefix parity over the chain's rows.
-        if (kLds) {
-          for (uint32_t idx = wv; idx < jr; idx += nw) {
-            const uint64_t *M = s_msk + 4 * (k + idx);
-            const uint32_t q = rfl((uint32_t)M[0]), slot = rfl((uint32_t)(M[0] >> 32));
-            const uint64_t *cq = P + q * stride;
-            uint32_t len = 0, par = 0;
-            uint64_t rx = 0;
-            for (uint32_t kk = 0; kk < KH; ++kk) len += (uint32_t)__popcll(cq[kk]);
-            len = rfl(len);
-            for (uint32_t kk = 0; kk < KH; ++kk) {
-              uint64_t c = rfl64(cq[kk]);
-              par ^= (uint32_t)__popcll(c & rc[KH + kk]);
-              if (len <= 8) {
-                while (c) {
-                  const uint32_t i = (uint32_t)__ffsll((long long)c) - 1;
-                  c &= c - 1;
-                  rx ^= Rv[n + 64 * kk + i];
-                }
-              } else if ((c >> lane) & 1) {
-                rx ^= Rv[n + 64 * kk + lane];
-              }
-            }
-            if (len > 8) rx = wave_xor(rx);
-            uint32_t ph = 0;
-            if (len > 1) {
-              uint32_t tot = 0;
-              for (uint32_t j0 = 0; j0 < n; j0 += 64) {
-                const uint32_t j = min(j0 + lane, n - 1);
-                const uint64_t *xj = P + j * stride + KH, *zj = xj + n * stride;
-                uint64_t carry = 0;
-                uint32_t t = 0;
-                for (uint32_t kk = 0; kk < KH; ++kk) {
-                  const uint64_t c = rfl64(cq[kk]);
-                  if (!c) continue;
-                  const uint64_t xs = xj[kk] & c, zs = zj[kk] & c;
-                  if (__ballot((xs | zs) != 0) == 0) continue;
-                  const uint64_t inc = prefix_parity(zs);
-                  t += (uint32_t)__popcll(xs & zs) +
-                       2u * (uint32_t)__popcll(xs & ((inc << 1) ^ carry));
-                  carry ^= 0ull - (inc >> 63);
-                }
-                if (j0 + lane < n) tot += t;
-              }
-              ph = wave_sum_bit1(tot);
-            }
-            const uint32_t cst = (par ^ ph) & 1u;
-            if (lane == 0) {
-              if (!((M[1] >> 32) & kMeasSuperseded)) {
-                a.recs[(2ull * slot) * W + w] = rx ^ (0ull - (uint64_t)cst) ^ E[q];
-                a.recs[(2ull * slot + 1) * W + w] = ~0ull;
-              }
-            }
-            if (idx == jr - 1) {  // the scratch row keeps the last product
-              for (uint32_t j = lane; j < n; j += 64) {
-                P[j * stride + 2 * KH] = 0;
-                P[(n + j) * stride + 2 * KH] = j == q ? 1ull : 0ull;
-              }
-              if (lane == 0) {
-                rc[2 * KH] = cst;
-                Rv[2 * n] = rx;
-              }
-            }
-          }
-        } else {
-          // columns in global memory: the whole workgroup runs each, KH
+        if (!kLds && jr) {
+          // determined: as below, but the whole workgroup runs it, KH
           // lanes per column, so a column's words are one contiguous run
+          const uint32_t q = rfl(sh.ops[b].qq), slot = rfl((uint32_t)sh.msk[4 * b]);
           const uint32_t cpw = 64 / KH, sub = lane / KH, kk = lane - sub * KH;
           const uint64_t below = ((1ull << kk) - 1) << (sub * KH);
-          for (uint32_t idx = 0; idx < jr; ++idx) {
-            const uint64_t *M = s_msk + 4 * (k + idx);
-            const uint32_t q = rfl((uint32_t)M[0]), slot = rfl((uint32_t)(M[0] >> 32));
-            if (tid < KH) sm[tid] = P[q * stride + tid];
-            if (tid == 0) {
-              sh.tot = 0;
-              sh.rx = 0;
-            }
-            __syncthreads();
-            uint64_t rx = 0;
-            for (uint32_t i = tid; i < n; i += NT)
-              if ((sm[i >> 6] >> (i & 63)) & 1) rx ^= Rv[n + i];
-            if (__ballot(rx != 0)) {
-              rx = wave_xor(rx);
-              if (lane == 0) lds_xor(&sh.rx, rx);
-            }
-            uint32_t tot = 0;
-            const uint64_t c = sub < cpw ? sm[kk] : 0ull;
-            if (tid < KH) tot = 2u * (uint32_t)__popcll(c & rc[KH + kk]);
-            const uint32_t cstep = nw * cpw;
-            for (uint32_t j0 = wv * cpw; j0 < n; j0 += 4 * cstep) {
-              uint64_t xs[4], zs[4];
-#pragma unroll
-              for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t j = j0 + u * cstep + sub;
-                const bool use = c != 0 && j < n;
-                const uint64_t *xj = P + (use ? j * stride + KH + kk : 0u);
-                xs[u] = use ? xj[0] & c : 0ull;
-                zs[u] = use ? xj[n * stride] & c : 0ull;
-              }
-#pragma unroll
-              for (uint32_t u = 0; u < 4; ++u) {
-                const uint64_t inc = prefix_parity(zs[u]);
-                const uint64_t odd = __ballot(inc >> 63);
-                const uint64_t carry = 0ull - (uint64_t)(__popcll(odd & below) & 1);
-                tot += (uint32_t)__popcll(xs[u] & zs[u]) +
-                       2u * (uint32_t)__popcll(xs[u] & ((inc << 1) ^ carry));
-              }
-            }
-            // sum mod 4 over the wave: lanes' low bits and twos
-            {
-              const uint32_t s = (uint32_t)__popcll(__ballot(tot & 1u)) +
-                                 2u * (uint32_t)__popcll(__ballot((tot >> 1) & 1u));
-              if (lane == 0 && (s & 3u)) atomicAdd(&sh.tot, s & 3u);
-            }
-            __syncthreads();
-            const uint32_t cst = (sh.tot >> 1) & 1u;
-            if (idx == jr - 1) {
-              for (uint32_t j = tid; j < n; j += NT) {
-                P[j * stride + 2 * KH] = 0;
-                P[(n + j) * stride + 2 * KH] = j == q ? 1ull : 0ull;
-              }
-            }
-            if (tid == 0) {
-              const uint64_t rxa = sh.rx;
-              if (!((M[1] >> 32) & kMeasSuperseded)) {
-                a.recs[(2ull * slot) * W + w] = rxa ^ (0ull - (uint64_t)cst) ^ E[q];
-                a.recs[(2ull * slot + 1) * W + w] = ~0ull;
-              }
-              rc[2 * KH] = cst;
-              Rv[2 * n] = rxa;
-            }
-            __syncthreads();
+          uint64_t rx = 0;
+          for (uint32_t i = tid; i < n; i += NT)
+            if ((read_lane64(xqv, rfl(i >> 6)) >> lane) & 1) rx ^= Rv[n + i];
+          if (__ballot(rx != 0)) {
+            rx = wave_xor(rx);
+            if (lane == 0) lds_xor(&sh.rx[slot2], rx);
           }
+          const uint64_t cm = __shfl(xqv, kk, 64);
+          const uint64_t c = sub < cpw ? cm : 0ull;
+          uint32_t tot = tid < KH ? 2u * (uint32_t)__popcll(c & rc[KH + kk]) : 0u;
+          const uint32_t cstep = nw * cpw;
+          for (uint32_t j0 = wv * cpw; j0 < n; j0 += kWideCols * cstep) {
+            uint64_t xs[kWideCols], zs[kWideCols];
+#pragma unroll
+            for (uint32_t u = 0; u < kWideCols; ++u) {
+              const uint32_t j = j0 + u * cstep + sub;
+              const bool use = c != 0 && j < n;
+              const uint64_t *xj = P + (use ? j * KW + KH + kk : 0u);
+              xs[u] = use ? xj[0] & c : 0ull;
+              zs[u] = use ? xj[n * KW] & c : 0ull;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kWideCols; ++u) {
+              if (__ballot((xs[u] | zs[u]) != 0) == 0) continue;
+              const uint64_t inc = prefix_parity(zs[u]);
+              const uint64_t odd = __ballot(inc >> 63);
+              const uint64_t carry = 0ull - (uint64_t)(__popcll(odd & below) & 1);
+              tot += (uint32_t)__popcll(xs[u] & zs[u]) +
+                     2u * (uint32_t)__popcll(xs[u] & ((inc << 1) ^ carry));
+            }
+          }
+          // sum mod 4 over the wave: lanes' low bits and twos
+          const uint32_t s = ((uint32_t)__popcll(__ballot(tot & 1u)) +
+                              2u * (uint32_t)__popcll(__ballot((tot >> 1) & 1u))) & 3u;
+          if (lane == 0 && s) atomicAdd(&sh.tot[slot2], s);
+          // the other slot is free: it was read before this barrier
+          if (tid == 0) {
+            sh.tot[slot2 ^ 1] = 0;
+            sh.rx[slot2 ^ 1] = 0;
+          }
+          __syncthreads();
+          if (b + 1 == mend) {
+            for (uint32_t j = tid; j < n; j += NT) {
+              P[j * KW + K2] = 0;
+              P[(n + j) * KW + K2] = j == q ? 1ull : 0ull;
+            }
+          }
+          if (tid == 0) {
+            const uint32_t cst = (sh.tot[slot2] >> 1) & 1u;
+            const uint64_t rxa = sh.rx[slot2];
+            if (!(sh.ops[b].cw & kOpDropped)) {
+              a.recs[(2ull * slot) * W + w] = rxa ^ (0ull - (uint64_t)cst) ^ E[q];
+              a.recs[(2ull * slot + 1) * W + w] = ~0ull;
+            }
+            rc[K2] = cst;
+            Rv[2 * n] = rxa;
+          }
+          slot2 ^= 1;
         }
         if (jr == nm) {
-          k += nm;
-          __syncthreads();
+          b += nm;
+          // the scratch row's writes are in before the gates
+          if (!kLds && b == mend) __syncthreads();
           continue;
         }
 
-        // measurement k + jr is random in every shot, with one pivot p for
-        // all of them: rows with x_q set take the stabilizer row n+p, row p
+        // measurement b + jr is random in every shot, with one pivot p for all
+        // of them: rows with x_q set take the stabilizer row n+p, row p
         // becomes row n+p, and row n+p becomes Z_q with the coin as its sign
         {
-          const uint64_t *M = s_msk + 4 * (k + jr);
-          const uint32_t q = rfl((uint32_t)M[0]), slot = rfl((uint32_t)(M[0] >> 32));
-          const uint32_t coin_T = rfl((uint32_t)M[1]);
-          const uint64_t m = M[2];
-          const uint64_t *xq = P + q * stride;
-          const uint64_t sw = lane < KH ? xq[KH + lane] : 0ull;
-          const uint64_t hit = __ballot(sw != 0);
-          const uint32_t kp = (uint32_t)__ffsll((long long)hit) - 1;
-          const uint64_t pw = read_lane64(sw, kp);
-          const uint32_t bp = (uint32_t)__ffsll((long long)pw) - 1;
+          const uint32_t q = sh.ops[b + jr].qq;
+          const uint64_t M0 = sh.msk[4 * (b + jr)], m = sh.msk[4 * (b + jr) + 1];
+          if (kLds) xqv = lane < K2 ? P[__umul24(q, KW) + lane] : 0ull;
+          const uint64_t exq = E[q];
+          const uint32_t kp = (uint32_t)__ffsll((long long)(__ballot(xqv != 0) >> KH)) - 1;
+          const uint32_t bp = (uint32_t)__ffsll((long long)read_lane64(xqv, KH + kp)) - 1;
           const uint32_t p = 64 * kp + bp;
           const uint64_t bit = 1ull << bp;
-          const uint64_t Rs = Rv[n + p], exq = E[q];
-          const uint64_t rs = 0ull - ((rc[KH + kp] >> bp) & 1);  // row n+p's sign bit
-          if (tid < KW) {
-            uint64_t mk = tid < 2 * KH ? xq[tid] : 0ull;
-            if (tid == kp || tid == KH + kp) mk &= ~bit;
-            sm[tid] = mk;
-            s_c0[tid] = 0;
-            s_c1[tid] = 0;
+          const uint64_t Rs = Rv[n + p];
+          const uint64_t rck = rc[kp];
+          const uint64_t rs = 0ull - ((rc[KH + kp] >> bp) & 1);
+          if (lane == kp || lane == KH + kp) xqv &= ~bit;  // the rows to update
+          // the sign bits: rows to update take row n+p's (and their phase's), row
+          // p takes row n+p's, row n+p's is cleared
+          uint64_t dr = xqv & rs;
+          if (lane == kp) dr ^= (rs ^ rck) & bit;
+          if (lane == KH + kp) dr ^= rs & bit;
+          if (tid < K2) {
+            sh.sm[tid] = xqv;
+            sh.c0[tid] = 0;
+          }
+          if (tid == 0) {
+            sh.ops[b + jr].cw |= kOpRandom;
+            sh.nl = 0;
           }
           __syncthreads();
-          // phases: per row, the sum mod 4 over columns of the phase
-          // exponent of row * (row n+p), gathered with LDS atomics
-          // (the returned old value carries)
+          if (tid < K2 && dr) lds_xor(rc + tid, dr);
           if (kLds) {
-            for (uint32_t j = tid; j < n; j += NT) {
-              uint64_t *X = P + j * stride, *Z = X + n * stride;
-              const uint64_t wx = X[KH + kp], wz = Z[KH + kp];
-              const uint64_t xp = (wx >> bp) & 1, zp = (wz >> bp) & 1;
-              if (xp | zp) {
-                const uint64_t fx = 0ull - xp, fz = 0ull - zp;
-                for (uint32_t i = 0; i < 2 * KH; ++i) {
-                  const uint64_t mk = sm[i];
-                  if (!mk) continue;
-                  const uint64_t x = X[i], z = Z[i];
-                  uint64_t d0 = 0, d1 = 0;
-                  phase_acc(x, z, fx, fz, d0, d1);
-                  X[i] = x ^ (mk & fx);
-                  Z[i] = z ^ (mk & fz);
-                  d0 &= mk;
-                  if (d0) {
-                    d1 &= d0;
-                    d1 ^= d0 & atomicXor(reinterpret_cast<unsigned long long *>(s_c0 + i),
-                                         (unsigned long long)d0);
-                    if (d1) lds_xor(s_c1 + i, d1);
-                  }
-                }
+            // rows p and n+p, a lane per column; columns where row n+p is not
+            // the identity go on the list
+            for (uint32_t v = wv; v < KH; v += nw) {
+              const uint32_t j = 64 * v + lane;
+              uint32_t ent = 0;
+              if (j < n) {
+                uint64_t *X = P + __umul24(j, KW) + kp, *Z = X + n * KW;
+                const uint64_t wx = X[KH], wz = Z[KH], dx = X[0], dz = Z[0];
+                ent = (uint32_t)((wx >> bp) & 1) | ((uint32_t)((wz >> bp) & 1) << 1);
+                X[0] = (dx & ~bit) | (wx & bit);
+                Z[0] = (dz & ~bit) | (wz & bit);
+                X[KH] = wx & ~bit;
+                Z[KH] = (wz & ~bit) | (j == q ? bit : 0ull);
               }
-              X[kp] = (X[kp] & ~bit) | (xp << bp);
-              Z[kp] = (Z[kp] & ~bit) | (zp << bp);
-              X[KH + kp] &= ~bit;
-              Z[KH + kp] = (Z[KH + kp] & ~bit) | (j == q ? bit : 0ull);
-            }
-          } else {
-            // 2 KH lanes of one wave per column (a column's words are one
-            // run): its loads come before its stores in program order, so
-            // lanes read row n+p's bits before the lane that owns that word
-            // clears them
-            const uint32_t K2 = 2 * KH, cpw = 64 / K2, sub = lane / K2, i = lane - sub * K2;
-            const bool use = sub < cpw;
-            const uint64_t mk = use ? sm[i] : 0ull;
-            const uint32_t cstep = nw * cpw;
-            uint64_t c0 = 0, c1 = 0;
-            for (uint32_t j0 = wv * cpw + (use ? sub : 0u); j0 < n; j0 += 4 * cstep) {
-              uint64_t x[4], z[4], wx[4], wz[4];
-#pragma unroll
-              for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t j = min(j0 + u * cstep, n - 1);
-                const uint64_t *X = P + j * stride, *Z = X + n * stride;
-                x[u] = X[i];
-                z[u] = Z[i];
-                wx[u] = X[KH + kp];
-                wz[u] = Z[KH + kp];
-              }
-              __builtin_amdgcn_wave_barrier();
-#pragma unroll
-              for (uint32_t u = 0; u < 4; ++u) {
-                const uint32_t j = j0 + u * cstep;
-                if (use && j < n) {
-                  const uint64_t xp = (wx[u] >> bp) & 1, zp = (wz[u] >> bp) & 1;
-                  const uint64_t fx = mk & (0ull - xp), fz = mk & (0ull - zp);
-                  phase_acc(x[u], z[u], fx, fz, c0, c1);
-                  uint64_t nx = x[u] ^ fx, nz = z[u] ^ fz;
-                  if (i == kp) {
-                    nx = (nx & ~bit) | (xp << bp);
-                    nz = (nz & ~bit) | (zp << bp);
-                  } else if (i == KH + kp) {
-                    nx &= ~bit;
-                    nz = (nz & ~bit) | (j == q ? bit : 0ull);
-                  }
-                  uint64_t *X = P + j * stride + i;
-                  if (nx != x[u]) X[0] = nx;
-                  if (nz != z[u]) X[n * stride] = nz;
-                }
-              }
-            }
-            if (c0 | c1) {
-              c1 ^= c0 & atomicXor(reinterpret_cast<unsigned long long *>(s_c0 + i),
-                                   (unsigned long long)c0);
-              if (c1) lds_xor(s_c1 + i, c1);
+              const uint64_t bal = __ballot(ent != 0);
+              uint32_t at = 0;
+              if (lane == 0 && bal) at = atomicAdd(&sh.nl, (uint32_t)__popcll(bal));
+              at = rfl(at) + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
+              if (ent) sh.list[at] = j | (ent << 16);
             }
           }
-          for (uint32_t i = tid; i < 2 * n; i += NT) {
+          // (from the last threads down: the columns start at thread 0)
+          for (uint32_t i = NT - 1 - tid; i < 2 * n; i += NT) {
             const uint32_t ii = i < n ? i : i - n;
-            const uint64_t mk = sm[(i < n ? 0 : KH) + (ii >> 6)];
+            const uint64_t mk = sh.sm[(i < n ? 0 : KH) + (ii >> 6)];
             if ((mk >> (ii & 63)) & 1) Rv[i] ^= Rs;  // never rows p, n+p
           }
           if (wv == nw - 1) {
@@ -596,28 +507,190 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
               coin = a.coin_planes[m * W + w];
             } else {
               const uint64_t key = stream_key(seed, 2 * (mseq0 + m));
-              coin = __ballot((uint32_t)(draw_keyed(key, 64 * w + lane) >> 40) < coin_T);
+              coin = __ballot((uint32_t)(draw_keyed(key, 64 * w + lane) >> 40) < (uint32_t)(M0 >> 32));
             }
             if (lane == 0) {
               Rv[p] = Rs;
               Rv[n + p] = coin ^ exq;
-              a.recs[(2ull * slot) * W + w] = coin;
-              a.recs[(2ull * slot + 1) * W + w] = 0ull;
+              if (!(sh.ops[b + jr].cw & kOpDropped)) {
+                const uint32_t slot = (uint32_t)M0;
+                a.recs[(2ull * slot) * W + w] = coin;
+                a.recs[(2ull * slot + 1) * W + w] = 0ull;
+              }
             }
           }
-          __syncthreads();
-          if (tid < 2 * KH) {
-            uint64_t v = rc[tid] ^ (sm[tid] & (rs ^ s_c1[tid]));
-            if (tid == kp) v = (v & ~bit) | (rs & bit);
-            if (tid == KH + kp) v &= ~bit;
-            rc[tid] = v;
+          if (kLds) __syncthreads();
+          // phases: per row, the sum mod 4 over columns of the phase exponent
+          // of row * (row n+p): each thread's columns in registers, then
+          // LDS atomics; the low bits' old value gives the carry, and the high
+          // bits go into the signs
+          uint64_t c0 = 0, c1 = 0;
+          uint32_t ci = my_i;
+          if (kLds) {
+            const uint64_t mk = my_j < rpp ? sh.sm[my_i] : 0ull;
+            const uint32_t nl = sh.nl;
+            if (mk)
+              for (uint32_t e = my_j; e < nl; e += rpp) {
+                const uint32_t ent = sh.list[e];
+                uint64_t *X = P + (__umul24(ent & 0xFFFFu, KW) + my_i), *Z = X + n * KW;
+                const uint64_t x = *X, z = *Z;
+                const uint64_t fx = (ent >> 16) & 1 ? mk : 0ull, fz = ent >> 17 ? mk : 0ull;
+                phase_acc(x, z, fx, fz, c0, c1);
+                *X = x ^ fx;
+                *Z = z ^ fz;
+              }
+          } else {
+            // K2 lanes of one wave per column (a column's words are one run).
+            // Row n+p's bits come from the lane that holds its word, before
+            // any of the column's lanes stores.
+            const uint32_t cpw = 64 / K2, sub = lane / K2, i = lane - sub * K2;
+            const bool use = sub < cpw;
+            const uint64_t mi = __shfl(xqv, i, 64);
+            const uint64_t mk = use ? mi : 0ull;
+            const uint32_t src = min(sub, cpw - 1) * K2 + KH + kp;
+            const uint32_t cstep = nw * cpw;
+            for (uint32_t jw = wv * cpw; jw < n; jw += kWideCols * cstep) {
+              uint64_t x[kWideCols], z[kWideCols];
+#pragma unroll
+              for (uint32_t u = 0; u < kWideCols; ++u) {
+                const uint32_t j = min(jw + u * cstep + sub, n - 1);
+                const uint64_t *X = P + j * KW + i;
+                x[u] = X[0];
+                z[u] = X[n * KW];
+              }
+#pragma unroll
+              for (uint32_t u = 0; u < kWideCols; ++u) {
+                const uint32_t j = jw + u * cstep + sub;
+                const uint64_t xp = (__ballot((x[u] >> bp) & 1) >> src) & 1;
+                const uint64_t zp = (__ballot((z[u] >> bp) & 1) >> src) & 1;
+                if (use && j < n) {
+                  const uint64_t fx = mk & (0ull - xp), fz = mk & (0ull - zp);
+                  phase_acc(x[u], z[u], fx, fz, c0, c1);
+                  uint64_t nx = x[u] ^ fx, nzv = z[u] ^ fz;
+                  if (i == kp) {
+                    nx = (nx & ~bit) | (xp << bp);
+                    nzv = (nzv & ~bit) | (zp << bp);
+                  } else if (i == KH + kp) {
+                    nx &= ~bit;
+                    nzv = (nzv & ~bit) | (j == q ? bit : 0ull);
+                  }
+                  uint64_t *X = P + j * KW + i;
+                  if (nx != x[u]) X[0] = nx;
+                  if (nzv != z[u]) X[n * KW] = nzv;
+                }
+              }
+            }
+            ci = i;
+          }
+          if (c0 | c1) {
+            c1 ^= c0 & atomicXor(reinterpret_cast<unsigned long long *>(sh.c0 + ci),
+                                 (unsigned long long)c0);
+            if (c1) lds_xor(rc + ci, c1);
           }
           __syncthreads();
-          k += jr + 1;
+          b += jr + 1;
         }
       }
+      // the run's determined measurements: the outcome is the sign of
+      // the product, in ascending order, of the stabilizers whose
+      // destabilizer has x_q set, which is Z_q up to that sign.  Writing a
+      // Pauli row as i^y X^x Z^z (y the number of Y's), the product's
+      // phase is i^(sum y) times -1 for every earlier z that meets a later x:
+      // per column, a walk along the chain's rows, or where a word holds
+      // several of them a prefix parity.  Rows without x bits (the Z checks of
+      // a code) have no phase at all.
+      if (kLds) {
+        uint32_t last = mend;  // the last determined one
+        while (last > mbeg && (rfl(sh.ops[last - 1].cw) & kOpRandom)) --last;
+        --last;
+        for (uint32_t idx = mbeg + wv; idx < mend; idx += nw) {
+          const SharedOp J = sh.ops[idx];
+          if (rfl(J.cw) & kOpRandom) continue;
+          const uint32_t q = J.qq, slot = (uint32_t)sh.msk[4 * idx];
+          const uint64_t cv = lane < KH ? P[__umul24(q, KW) + lane] : 0ull;
+          const uint64_t rv = lane < KH ? rc[KH + lane] : 0ull;
+          const uint64_t exq = E[q];
+          const uint64_t nz = __ballot(cv != 0);
+          const bool chain = __ballot((cv & (cv - 1)) != 0) != 0 || (nz & (nz - 1)) != 0;
+          const uint32_t par = (uint32_t)__popcll(__ballot(__popcll(cv & rv) & 1));
+          uint64_t rx = 0, ry = 0;
+          uint32_t tot = 0, carry = 0;  // carry: bit u is column 64 u + lane's
+          bool wide = false;
+          uint64_t anyx = 0;
+          for (uint64_t left = nz; left; left &= left - 1) {
+            const uint32_t kk = (uint32_t)__ffsll((long long)left) - 1;
+            const uint64_t c = read_lane64(cv, kk);
+            const uint32_t cl = (uint32_t)__popcll(c);
+            if (cl <= 4) {
+              for (uint64_t r = c; r; r &= r - 1)
+                rx ^= Rv[n + 64 * kk + (uint32_t)__ffsll((long long)r) - 1];
+            } else {
+              wide = true;
+              if ((c >> lane) & 1) ry ^= Rv[n + 64 * kk + lane];
+            }
+            if (chain)
+              for (uint32_t j = lane; j < n; j += 64)
+                anyx |= P[__umul24(j, KW) + KH + kk] & c;
+          }
+          if (__ballot(anyx != 0)) {
+            for (uint64_t left = nz; left; left &= left - 1) {
+              const uint32_t kk = (uint32_t)__ffsll((long long)left) - 1;
+              const uint64_t c = read_lane64(cv, kk);
+              const bool one = (c & (c - 1)) == 0;
+              for (uint32_t u0 = 0; 64 * u0 < n; u0 += 3) {
+                uint64_t xs[3], zs[3];
+#pragma unroll
+                for (uint32_t u = 0; u < 3; ++u) {
+                  const uint32_t j = 64 * (u0 + u) + lane;
+                  const uint64_t *xj = P + min(j, n - 1) * KW + KH + kk;
+                  const uint64_t cm = j < n ? c : 0ull;
+                  xs[u] = xj[0] & cm;
+                  zs[u] = xj[n * KW] & cm;
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < 3; ++u) {
+                  const uint32_t cb = (carry >> (u0 + u)) & 1u;
+                  if (one) {
+                    const uint32_t xb = xs[u] != 0, zb = zs[u] != 0;
+                    tot += xb & zb;
+                    tot += 2u * (xb & cb);
+                    carry ^= zb << (u0 + u);
+                  } else if (__ballot((xs[u] | zs[u]) != 0)) {
+                    const uint64_t inc = prefix_parity(zs[u]);
+                    tot += (uint32_t)__popcll(xs[u] & zs[u]) +
+                           2u * (uint32_t)__popcll(xs[u] & ((inc << 1) ^ (0ull - (uint64_t)cb)));
+                    carry ^= (uint32_t)(inc >> 63) << (u0 + u);
+                  }
+                }
+              }
+            }
+          }
+          if (wide) rx ^= wave_xor(ry);
+          const uint32_t cst = (par ^ wave_sum_bit1(tot)) & 1u;
+          if (lane == 0 && !(J.cw & kOpDropped)) {
+            a.recs[(2ull * slot) * W + w] = rx ^ (0ull - (uint64_t)cst) ^ exq;
+            a.recs[(2ull * slot + 1) * W + w] = ~0ull;
+          }
+          if (idx == last) {  // the scratch row keeps the last product
+            for (uint32_t j = lane; j < n; j += 64) {
+              P[j * KW + K2] = 0;
+              P[(n + j) * KW + K2] = j == q ? 1ull : 0ull;
+            }
+            if (lane == 0) {
+              rc[K2] = cst;
+              Rv[2 * n] = rx;
+            }
+          }
+        }
+        __syncthreads();
+      }
+      b = mend;
+      if (b < wn) cw = rfl(sh.ops[b].cw);
     }
+    base += b;
   }
+  if (on && rp) lds_xor(rc + my_k, rp);
+  __syncthreads();
 
   // ---- the 64-shot words ----
   // <E, P_i> of 64 rows at a time: a column's word is the lane mask.  Row
@@ -631,12 +704,14 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
       uint64_t acc = 0;
       for (uint32_t j0 = ja; j0 < jb; j0 += 64) {
         const uint32_t jl = min(j0 + lane, n - 1);
-        const uint64_t xw = P[jl * stride + kk], zw = P[(n + jl) * stride + kk];
+        const uint64_t xw = P[jl * KW + kk], zw = P[(n + jl) * KW + kk];
+        const uint64_t xe = E[jl], ze = E[n + jl];
         const uint32_t cnt = min(64u, jb - j0);
         for (uint32_t t = 0; t < cnt; ++t) {
           const uint64_t sx = read_lane64(xw, t), sz = read_lane64(zw, t);
-          if (sx) acc ^= (0ull - ((sx >> lane) & 1)) & E[n + j0 + t];
-          if (sz) acc ^= (0ull - ((sz >> lane) & 1)) & E[j0 + t];
+          const uint64_t ex = read_lane64(xe, t), ez = read_lane64(ze, t);
+          acc ^= __builtin_amdgcn_inverse_ballot_w64(sx) ? ez : 0ull;
+          acc ^= __builtin_amdgcn_inverse_ballot_w64(sz) ? ex : 0ull;
         }
       }
       if (pt == 0) acc ^= 0ull - ((rc[kk] >> lane) & 1);
@@ -650,21 +725,32 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
   }
   __syncthreads();
   for (uint32_t i = tid; i < R; i += NT) Tr[i] = Rv[i];
-  // a wave per column: its packed words are read before the column is written
-  // over them
-  for (uint32_t c = wv; c < 2 * n; c += nw) {
-    const uint64_t *src = P + c * stride;
+  __syncthreads();
+  // Wide states: the packed block covers the first KW tableau columns; those
+  // are written last, from a copy.
+  const uint32_t c0 = kLds ? 0 : KW;
+  if (!kLds) {
+    for (uint32_t i = tid; i < c0 * KW; i += NT) dyn[i] = P[i];
+    __syncthreads();
+  }
+  // a wave per column
+  auto expand = [&](uint32_t c, const uint64_t *src) {
     const uint64_t v0 = lane < KW ? src[lane] : 0ull;
     const uint64_t v1 = lane + 64 < KW ? src[lane + 64] : 0ull;
-    __builtin_amdgcn_wave_barrier();
     uint64_t *dst = T + (uint64_t)c * R;
-    for (uint32_t kk = 0; kk < 2 * KH; ++kk) {
+    for (uint32_t kk = 0; kk < K2; ++kk) {
       const uint64_t s = kk < 64 ? read_lane64(v0, kk) : read_lane64(v1, kk - 64);
       const uint32_t ii = 64 * (kk < KH ? kk : kk - KH) + lane;
-      if (ii < n) dst[(kk < KH ? 0 : n) + ii] = 0ull - ((s >> lane) & 1);
+      if (ii < n)
+        dst[(kk < KH ? 0 : n) + ii] = __builtin_amdgcn_inverse_ballot_w64(s) ? ~0ull : 0ull;
     }
-    const uint64_t s = 2 * KH < 64 ? read_lane64(v0, 2 * KH) : read_lane64(v1, 2 * KH - 64);
+    const uint64_t s = K2 < 64 ? read_lane64(v0, K2) : read_lane64(v1, K2 - 64);
     if (lane == 0) dst[2 * n] = 0ull - (s & 1);
+  };
+  for (uint32_t c = c0 + wv; c < 2 * n; c += nw) expand(c, P + c * KW);
+  if (!kLds) {
+    __syncthreads();
+    for (uint32_t c = wv; c < c0; c += nw) expand(c, dyn + c * KW);
   }
   __syncthreads();
   return true;
@@ -727,12 +813,10 @@ bool shared_wide(uint32_t n) { return !packed_in_lds(n); }
 bool shared_fits(uint32_t n) { return n >= 1 && n <= kSharedMaxQubits; }
 
 size_t shared_lds_bytes(uint32_t n) {
-  return 8 * (shared_base_words(n) + (packed_in_lds(n) ? shared_packed_words(n) : 0));
+  return 8 * (packed_in_lds(n) ? packed_words(n) : 4ull * n + 1);
 }
 
 hipError_t prepare_shared(uint32_t n) {
-  const size_t lds = shared_lds_bytes(n);
-  if (lds <= 65536) return hipSuccess;
   const void *fn = packed_in_lds(n) ? (const void *)k_program_shared<true>
                                     : (const void *)k_program_shared<false>;
   return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -755,7 +839,7 @@ hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const ui
   // as many workgroups per CU as the largest member's LDS allows
   auto blocks = [&](size_t lds) {
     return dim3((uint32_t)std::min<uint64_t>(
-        nitems, cus * std::min<uint64_t>(4, std::max<uint64_t>(1, 160 * 1024 / (lds + 1024)))));
+        nitems, cus * std::min<uint64_t>(4, std::max<uint64_t>(1, 160 * 1024 / (lds + sizeof(SharedLds))))));
   };
   if (nitems && lds_packed)
     hipLaunchKernelGGL(k_batch_shared<true>, blocks(lds_packed), dim3(kSharedThreads), lds_packed,

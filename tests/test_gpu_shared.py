@@ -76,7 +76,7 @@ def check(st, orc):
     (1, 130, 60, 0.2), (2, 64, 80, 0.2), (3, 1, 80, 0.3),
     (63, 65, 900, 0.1), (64, 65, 900, 0.1), (65, 65, 900, 0.1),
     (128, 64, 1500, 0.05), (129, 70, 1500, 0.05),
-    (471, 3, 1600, 0.05), (472, 3, 1600, 0.05), (513, 3, 1600, 0.04),
+    (468, 3, 1600, 0.05), (469, 3, 1600, 0.05), (513, 3, 1600, 0.04),
     (700, 3, 1500, 0.03), (2048, 1, 2400, 0.01), (2049, 1, 2400, 0.01),
 ])
 def test_shared_equals_oracle(ps, n, B, nops, meas):
