@@ -434,11 +434,11 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     // one runs each
     uint32_t shared = 0;
     if (s->tab && shared_allowed(s, p)) {
-      size_t &lds = shared_lds[shared_wide((uint32_t)s->n) ? 1 : 0];
-      lds = std::max(lds, shared_lds_bytes((uint32_t)s->n));
+      size_t &lds = shared_lds[shared_wide((uint32_t)s->n, p->masked) ? 1 : 0];
+      lds = std::max(lds, shared_lds_bytes((uint32_t)s->n, p->masked));
       if (s->xz_identity) shared = s->exposed ? kSharedVerify : kSharedKnown;
     }
-    if (shared == kSharedVerify && (rc = ensure_done(s, p))) return rc;
+    if ((rc = ensure_shared(s, p, shared, false))) return rc;
     if (shared == kSharedKnown) {
       s->xz_pending = false;
       s->xz_plan.reset();

@@ -105,8 +105,12 @@ struct ProgramArgs {
   // those groups.
   uint32_t shared;
   uint32_t *done;
+  uint32_t masked;   // the program has noise or flagged ops
+  uint32_t gshift;   // log2 of the word groups per workgroup (launch_shared sets it)
+  uint64_t *packed;  // shared_packed_bytes(n), or null: the X/Z words are written in the kernel
 };
-constexpr uint32_t kSharedKnown = 1, kSharedVerify = 2;
+// (kSharedChecked: inside launch_shared, done[] already tells which groups run)
+constexpr uint32_t kSharedKnown = 1, kSharedVerify = 2, kSharedChecked = 3;
 // One state of a mixed batch: its program arguments, run parameters and
 // noise descriptors (planes are generated by the batch prologue).
 struct BatchCircuit {
@@ -149,21 +153,27 @@ hipError_t prepare_kernels(uint32_t n);
 hipError_t launch_program(hipStream_t s, const ProgramArgs &a, uint32_t threads,
                           uint32_t blocks, const void *params);
 // Shared-X/Z form of a persistent run (pq_shared.hip): programs without
-// flagged H/S/CX/CZ on the |0...0> tableau, one workgroup per word group.
+// flagged H/S/CX/CZ on the |0...0> tableau, one workgroup per 1, 2 or 4 word
+// groups.
 constexpr uint32_t kSharedThreads = 768;
 constexpr uint32_t kSharedMaxQubits = 2048;
+constexpr uint32_t kSharedMaxGroups = 4;
 bool shared_fits(uint32_t n);
-size_t shared_lds_bytes(uint32_t n);
-// Raises the kernels' dynamic-LDS limit for n qubits (not in a capture).
-hipError_t prepare_shared(uint32_t n);
+// Dynamic LDS of one word group per workgroup (as batches run).
+size_t shared_lds_bytes(uint32_t n, bool masked);
+// Whether the run checks the tableau and writes the X/Z words in launches of
+// their own; it then needs ProgramArgs::packed.
+bool shared_split(uint32_t n, uint64_t W, bool masked);
+uint64_t shared_packed_bytes(uint32_t n);
+// Raises the kernels' dynamic-LDS limit (not in a capture).
+hipError_t prepare_shared();
 hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params);
 // Whether n qubits' packed columns sit in the tableau, not in the LDS.
-bool shared_wide(uint32_t n);
+bool shared_wide(uint32_t n, bool masked);
 // The batch members whose a.shared is set, before launch_batch (whose
 // work items, word tile and counters it shares).  lds_packed / lds_wide: most
 // LDS bytes of a member with its packed columns in LDS / in the tableau (0: no
 // such member).
-hipError_t prepare_batch_shared();
 hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const uint64_t *items,
                                uint64_t nitems, unsigned long long *counter, uint32_t cus,
                                size_t lds_packed, size_t lds_wide, uint32_t wtile);

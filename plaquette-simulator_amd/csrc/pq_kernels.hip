@@ -2447,7 +2447,7 @@ hipError_t prepare_batch_kernel() {
       ensure_lds_attr((const void *)k_batch_t<kSmallRegs, kSmallThreads>, kProgramLdsBudget);
   if (e == hipSuccess)
     e = ensure_lds_attr((const void *)k_batch_t<kLargeRegs, kLargeThreads>, kProgramLdsBudget);
-  if (e == hipSuccess) e = prepare_batch_shared();
+  if (e == hipSuccess) e = prepare_shared();
   return e;
 }
 

@@ -321,6 +321,8 @@ int compile_program(pq_program_s *p) {
   const uint64_t nops = p->ops.size();
   p->uniform = true;
   for (uint64_t i = 0; i < nops; ++i)
+    if (ops[i].code == PQ_OP_NOISE || is_flag(ops[i].code)) p->masked = true;
+  for (uint64_t i = 0; i < nops; ++i)
     if (ops[i].code == PQ_OP_H_FLAG || ops[i].code == PQ_OP_S_FLAG ||
         ops[i].code == PQ_OP_CX_FLAG || ops[i].code == PQ_OP_CZ_FLAG)
       p->uniform = false;
@@ -441,7 +443,7 @@ pq_program_s::~pq_program_s() {
   if (done_ev) (void)hipEventDestroy(done_ev);
   for (void *q : {(void *)d_census, (void *)d_segs, (void *)d_segq, (void *)d_instrs,
                   (void *)d_noise, (void *)d_planes, (void *)d_side, (void *)d_sync,
-                  (void *)d_done})
+                  (void *)d_done, (void *)d_packed})
     dev_free(q, alloc_stream);
 }
 
@@ -486,7 +488,7 @@ static int create_program(pq_state s, const pq_op *ops, uint64_t nops, hipStream
   p->threads = program_max_threads((uint32_t)s->n, p->tiled);
   p->blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(s->W, 1u << 20));
   if (!as) HIPCHK(prepare_kernels((uint32_t)s->n));
-  if (p->uniform && shared_fits((uint32_t)s->n)) HIPCHK(prepare_shared((uint32_t)s->n));
+  if (p->uniform && shared_fits((uint32_t)s->n)) HIPCHK(prepare_shared());
   *out = p.release();
   return PQ_OK;
 }
@@ -616,6 +618,7 @@ ProgramArgs program_args(pq_state s, pq_program p, uint64_t lds_budget) {
   a.planes = p->d_planes;
   a.wide = p->tiled ? 1u : 0u;
   a.nk = (uint32_t)p->nnoise;
+  a.masked = p->masked ? 1u : 0u;
   a.segs = p->d_segs;
   a.instrs = p->d_instrs;
   a.coin_planes = nullptr;
@@ -702,9 +705,12 @@ bool shared_allowed(const pq_state_s *s, const pq_program_s *p) {
          !p->census_on && !p->slices_set && p->threads >= 256;
 }
 
-int ensure_done(pq_state s, pq_program p) {
-  if (!p->d_done)
+int ensure_shared(pq_state s, pq_program p, uint32_t shared, bool split) {
+  if (shared == kSharedVerify && !p->d_done)
     HIPCHK(dev_alloc((void **)&p->d_done, s->W * sizeof(uint32_t), p->alloc_stream));
+  if (shared && split && !p->d_packed)
+    HIPCHK(dev_alloc((void **)&p->d_packed, shared_packed_bytes((uint32_t)s->n),
+                     p->alloc_stream));
   return PQ_OK;
 }
 
@@ -717,6 +723,7 @@ static int enqueue_persistent(pq_state s, pq_program p, bool timed, bool allow_s
   a.fresh = fresh ? 1u : 0u;
   a.shared = shared;
   a.done = shared == kSharedVerify ? p->d_done : nullptr;
+  if (shared && shared_split(a.n, a.W, p->masked)) a.packed = p->d_packed;
   uint32_t S = 1;
   int rc = choose_slices(s, p, a, allow_slices && !shared, &S);
   if (rc) return rc;
@@ -806,7 +813,7 @@ static int program_run(pq_state s, pq_program p, int form) {
   if ((form == PQ_RUN_PERSISTENT && s->xz_identity) || form == PQ_RUN_GRAPH)
     if (shared_allowed(s, p))
       shared = form == PQ_RUN_GRAPH || s->exposed ? kSharedVerify : kSharedKnown;
-  if (shared == kSharedVerify && (rc = ensure_done(s, p))) return rc;
+  if ((rc = ensure_shared(s, p, shared, shared_split((uint32_t)s->n, s->W, p->masked)))) return rc;
   if (shared == kSharedKnown) {
     s->xz_pending = false;
     s->xz_plan.reset();

@@ -29,6 +29,7 @@ struct pq_program_s {
   std::vector<pq::NoiseDesc> noise;
   std::vector<uint32_t> segq;  // qubit lists of row-tiled gate segments
   bool tiled = false;          // some gate segment runs row-tiled
+  bool masked = false;         // noise or flagged ops
   bool uniform = false;        // no flagged H/S/CX/CZ: X/Z change in every shot alike
   pq::DSegment *d_segs = nullptr;
   uint32_t *d_segq = nullptr;
@@ -62,6 +63,7 @@ struct pq_program_s {
   // counters ([W] words) and give-up flag (one word after them)
   uint32_t slices_req = 0, slices_used = 1;
   bool slices_set = false;     // pq_program_set_slices was called: per-shot kernel
+  uint64_t *d_packed = nullptr;  // the shared X/Z columns, where a kernel of its own expands them
   uint32_t *d_done = nullptr;  // shared-X/Z runs that verify: groups that ran, [W]
   uint32_t slice_wait = 0;  // polls before a barrier gives up (0: default)
   unsigned int *d_sync = nullptr;
@@ -86,9 +88,9 @@ int check_records(pq_state s, pq_program p);
 int prepare_records(pq_state s, pq_program p);
 pq::ProgramArgs program_args(pq_state s, pq_program p, uint64_t lds_budget);
 // Whether a persistent run of p on s from |0...0> may take the shared-X/Z
-// kernel, and the flags a run that verifies the tableau needs.
+// kernel, and the buffers such a run needs (made once per program).
 bool shared_allowed(const pq_state_s *s, const pq_program_s *p);
-int ensure_done(pq_state s, pq_program p);
+int ensure_shared(pq_state s, pq_program p, uint32_t shared, bool split);
 // pq_program_create for a server-owned state: stream-ordered allocation and
 // copies on the state's stream.
 int create_program_on(pq_state s, const pq_op *ops, uint64_t nops, pq_program *out);

@@ -36,7 +36,7 @@ namespace {
 #define PQ_CONST __attribute__((address_space(4)))
 
 constexpr uint32_t kChunk = 448;       // staged ops; must equal kStage in pq_kernels.hip
-constexpr uint32_t kWideCols = 6;      // columns a lane has in flight (wide states)
+constexpr uint32_t kWideCols = 5;      // columns a lane has in flight (wide states)
 constexpr uint32_t kWindow = 64;       // measurements whose pivots are checked at once
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
@@ -77,19 +77,19 @@ __device__ __forceinline__ uint32_t wave_sum_bit1(uint32_t v) {
 
 // One staged op: `cw` = the flags below, and from bit 12 the ops of the layer
 // part it opens, or the measurements left in its run; `qq` = qa | qb << 16 (qb
-// = qa for one-qubit ops).  Its four masks are what the op and the noise after
-// it XOR into the frame's x and z words of qa and of qb; an op flagged by a
-// record keeps the flag in the third and the record in the fourth.  A
-// measurement's first two hold record | coin threshold << 32 and the sequence
-// number.
+// = qa for one-qubit ops).  Its four masks (per word group) are what the noise after it XORs into the
+// frame's x and z words of qa and of qb; a flagged op keeps its flag in the
+// third, and with a record as its flag the record in the fourth.  A
+// measurement has record | coin threshold << 32 and its sequence number there.
 struct SharedOp {
   uint32_t cw, qq;
 };
 constexpr uint32_t kOpH = 1, kOpS = 2, kOpCX = 4, kOpCZ = 8, kOpGate = 15;
 constexpr uint32_t kOpMeas = 1u << 4;
-constexpr uint32_t kOpMasks = 1u << 5;    // some mask word is not zero
-constexpr uint32_t kOpRecX = 1u << 6;     // a record's flag goes to x
-constexpr uint32_t kOpRecZ = 1u << 7;     // ... to z
+constexpr uint32_t kOpMasks = 1u << 5;    // some mask word may not be zero
+constexpr uint32_t kOpNotX = 1u << 6, kOpNotZ = 1u << 7;  // a Pauli on every shot: x, z flip
+constexpr uint32_t kOpFlagX = 1u << 10, kOpFlagZ = 1u << 11;  // flagged: the flag goes to x, z
+constexpr uint32_t kOpRecord = 1u << 24;  // the flag is a record
 constexpr uint32_t kOpDropped = 1u << 8;  // a later measurement writes its record
 constexpr uint32_t kOpRandom = 1u << 9;   // a measurement found random (set when it runs)
 constexpr uint32_t kOpLenShift = 12, kOpLenMask = 0xFFFu;
@@ -97,7 +97,6 @@ constexpr uint32_t kOpLenShift = 12, kOpLenMask = 0xFFFu;
 constexpr uint32_t kMaxRowWords = 2 * (kSharedMaxQubits / 64) + 2;
 struct SharedLds {
   SharedOp ops[kChunk + 1];
-  uint64_t msk[4 * kChunk];
   uint64_t rc[kMaxRowWords];  // sign bits, laid out like a column
   uint64_t sm[kMaxRowWords];  // row mask of the current random measurement
   uint64_t c0[kMaxRowWords];  // and the low bits of its rows' phase sums
@@ -106,67 +105,91 @@ struct SharedLds {
   // determined measurements of wide states, two in turn: phase count, XOR of
   // Rv rows
   uint32_t tot[2];
-  uint64_t rx[2];
+  uint64_t rx[2][kSharedMaxGroups];
   uint32_t nl;                // entries of list
   uint64_t item;
 };
 constexpr uint64_t kSharedLdsBytes = 159 * 1024 - sizeof(SharedLds);  // dynamic LDS cap
 
-// Dynamic LDS words: Rv, the frame, and the packed columns if they fit.
-__host__ __device__ inline uint64_t packed_words(uint32_t n) {
-  return (2ull * n + 1) + 2ull * n + 2ull * n * (2ull * ((n + 63) / 64) + 1);
+// Dynamic LDS words: Rv and the frame of each of the G word groups, their op
+// masks (programs with noise or flags), and the packed columns if they fit.
+// (Programs without masks keep only the measurements' two words there.)
+__host__ __device__ inline uint64_t groups_words(uint32_t n, bool masked, uint32_t gs) {
+  return ((4ull * n + 1) << gs) + (masked ? (4ull * kChunk) << gs : 2ull * kChunk);
 }
-__host__ __device__ inline bool packed_in_lds(uint32_t n) {
-  return packed_words(n) * 8 <= kSharedLdsBytes;
+__host__ __device__ inline uint64_t packed_words(uint32_t n) {
+  return 2ull * n * (2ull * ((n + 63) / 64) + 1);
+}
+__host__ __device__ inline bool packed_in_lds(uint32_t n, bool masked) {
+  return (groups_words(n, masked, 0) + packed_words(n)) * 8 <= kSharedLdsBytes;
 }
 
-// Runs the program on word group w.  Returns false, with the state untouched,
-// if a.shared asks to verify that the group's X/Z are the |0...0> tableau and
-// they are not.
+// Runs the program on word groups w0 .. w0 + G - 1 (those below a.W), which
+// share the packed X/Z, G = 1 << gs.  Groups whose X/Z are not the |0...0>
+// tableau (kSharedVerify: looked at here; kSharedChecked: told by a.done) are
+// left untouched.  Returns the groups that ran as a bit mask.  With a.packed
+// the 64-shot X/Z words are left to k_shared_expand, which reads the packed
+// columns there.
 template <bool kLds>
-__device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0, uint64_t w,
-                            uint64_t *dyn, SharedLds &sh) {
+__device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t mseq0, uint64_t w0,
+                                 uint32_t gs, uint64_t *dyn, SharedLds &sh) {
   const uint32_t tid = threadIdx.x, NT = blockDim.x, lane = lane_id();
   const uint32_t wv = rfl(tid >> 6), nw = NT >> 6;
   const uint32_t n = a.n, R = a.R;
   const uint32_t KH = (n + 63) / 64, K2 = 2 * KH, KW = K2 + 1;
   const uint64_t W = a.W;
-  uint64_t *T = a.tab + w * (uint64_t)a.C * R;
-  uint64_t *Tr = T + 2ull * n * R;  // the R column
-  // packed column c (x_c, or z_{c-n}) starts at P + c * KW: one compact block,
-  // in LDS or at the start of the group's tableau block.  (At a stride of the
-  // tableau's own columns, 2n+1 words, neighbouring columns fall on one L2
-  // channel.)
+  const uint32_t G = 1u << gs, g_mask = G - 1;
+  const uint64_t blk = (uint64_t)a.C * R;
+  uint64_t *const T0 = a.tab + w0 * blk;  // group g's block: T0 + g * blk
+  const bool masked = a.masked;
+  // per-group arrays: group g's Rv at g * R, its frame at g * 2n, its masks of
+  // op t at (t * G + g) * 4
   uint64_t *Rv = dyn;
-  uint64_t *E = Rv + R;  // E.x[0..n), E.z[n..2n)
-  uint64_t *P = kLds ? E + 2 * n : T;
+  uint64_t *E = Rv + R * G;
+  uint64_t *msk = E + 2 * n * G;
+  const uint32_t mstep = masked ? 4 * G : 2;  // op t's measurement words: msk + t * mstep
   uint64_t *const rc = sh.rc;
   const PQ_CONST DInstr *ins = (const PQ_CONST DInstr *)a.instrs;
-  const PQ_CONST uint64_t *gp = (const PQ_CONST uint64_t *)a.planes + 2ull * a.nk * w;
 
-  if (a.shared == kSharedVerify) {
+  uint32_t live = w0 + G <= W ? (1u << G) - 1 : (1u << (W - w0)) - 1;
+  if (a.shared == kSharedChecked) {
+    for (uint32_t g = 0; g < G; ++g)
+      if (((live >> g) & 1) && !rfl(a.done[w0 + g])) live &= ~(1u << g);
+  } else if (a.shared == kSharedVerify) {
     // word t of the X/Z block is all ones iff t is a multiple of R + 1
     if (tid == 0) sh.bad = 0;
     __syncthreads();
     const uint32_t total = 2 * n * R, M = R + 1, step = NT % M;
-    uint32_t rem = tid % M;
-    for (uint32_t base = tid; base < total; base += 8 * NT) {
-      uint64_t v[8];
+    for (uint32_t g = 0; g < G; ++g) {
+      if (!((live >> g) & 1)) continue;
+      const uint64_t *T = T0 + g * blk;
+      uint32_t rem = tid % M;
+      for (uint32_t base = tid; base < total; base += 8 * NT) {
+        uint64_t v[8];
 #pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) v[u] = T[min(base + u * NT, total - 1)];
-      bool bad = false;
+        for (uint32_t u = 0; u < 8; ++u) v[u] = T[min(base + u * NT, total - 1)];
+        bool bad = false;
 #pragma unroll
-      for (uint32_t u = 0; u < 8; ++u) {
-        bad |= base + u * NT < total && v[u] != (rem == 0 ? ~0ull : 0ull);
-        rem += step;
-        if (rem >= M) rem -= M;
+        for (uint32_t u = 0; u < 8; ++u) {
+          bad |= base + u * NT < total && v[u] != (rem == 0 ? ~0ull : 0ull);
+          rem += step;
+          if (rem >= M) rem -= M;
+        }
+        if (bad) atomicOr(&sh.bad, 1u << g);
+        if (__ballot(bad) || ((*(volatile uint32_t *)&sh.bad >> g) & 1)) break;
       }
-      if (bad) sh.bad = 1;
-      if (__ballot(bad) || *(volatile uint32_t *)&sh.bad) break;
     }
     __syncthreads();
-    if (sh.bad) return false;
+    live &= ~rfl(sh.bad);
+    if (tid < G && w0 + tid < W) a.done[w0 + tid] = (live >> tid) & 1;
   }
+  if (!live) return 0;
+
+  // packed column c (x_c, or z_{c-n}) starts at P + c * KW: one compact block,
+  // in LDS, or at the start of a group's tableau block, which the run
+  // overwrites anyway
+  uint64_t *P = kLds ? msk + (masked ? 4 * kChunk * G : 2 * kChunk)
+                     : T0 + ((uint32_t)__ffs((int)live) - 1) * blk;
 
   // ---- |0...0>: destabilizer i = X_i, stabilizer i = Z_i ----
   for (uint32_t u = tid; u < 2 * n * KW; u += NT) {
@@ -175,12 +198,14 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
     const uint32_t kq = (c < n ? 0 : KH) + (q >> 6);
     P[c * KW + k] = k == kq ? 1ull << (q & 63) : 0ull;
   }
-  for (uint32_t i = tid; i < R; i += NT) Rv[i] = Tr[i];
-  for (uint32_t i = tid; i < 2 * n; i += NT) E[i] = 0;
+  for (uint32_t g = 0; g < G; ++g)
+    for (uint32_t i = tid; i < R; i += NT)
+      Rv[g * R + i] = (live >> g) & 1 ? T0[g * blk + 2ull * n * R + i] : 0ull;
+  for (uint32_t i = tid; i < 2 * n * G; i += NT) E[i] = 0;
   if (tid < KW) rc[tid] = 0;
   if (tid < 2) {
     sh.tot[tid] = 0;
-    sh.rx[tid] = 0;
+    for (uint32_t g = 0; g < kSharedMaxGroups; ++g) sh.rx[tid][g] = 0;
   }
   __syncthreads();
 
@@ -199,55 +224,59 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
     // instructions [base, base + wn) and their masks, whatever segments they
     // belong to: two dependent loads per window, not per segment
     bool flags = false;
-    for (uint32_t t = tid; t < wn; t += NT) {
+    const uint32_t ss = masked ? gs : 0;  // one thread per op and group, or per op
+    for (uint32_t u = tid; u < wn << ss; u += NT) {
+      const uint32_t t = u >> ss, g = u & ((1u << ss) - 1);
       const PQ_CONST DInstr *I = ins + base + t;
       const uint32_t code = I->code, qa = I->qa, qb = I->qb, slot = I->slot, na = I->na,
                      nb = I->nb, t0 = I->t0, pad = I->pad;
       SharedOp J;
-      uint64_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
       if (code == PQ_OP_M) {
         J.cw = kOpMeas | (pad & kMeasSuperseded ? kOpDropped : 0u) |
                (min(pad >> kMeasLeftShift, kChunk) << kOpLenShift);
         J.qq = qa;
-        m0 = (uint64_t)slot | ((uint64_t)t0 << 32);
-        m1 = (uint64_t)na | ((uint64_t)nb << 32);
+        if (g == 0) {
+          msk[t * mstep] = (uint64_t)slot | ((uint64_t)t0 << 32);
+          msk[t * mstep + 1] = (uint64_t)na | ((uint64_t)nb << 32);
+        }
       } else {
-        if (na != kNone) {
-          m0 = gp[2ull * na];
-          m1 = gp[2ull * na + 1];
-        }
-        if (nb != kNone) {
-          m2 = gp[2ull * nb];
-          m3 = gp[2ull * nb + 1];
-        }
         const bool two = code == PQ_OP_CX || code == PQ_OP_CZ;
+        const bool flg = code >= PQ_OP_H_FLAG && code != PQ_OP_NOISE;
+        const bool rec = flg && !(slot & kSlotPlane);
         const bool px = code == PQ_OP_X || code == PQ_OP_Y || code == PQ_OP_X_FLAG ||
                         code == PQ_OP_Y_FLAG;
         const bool pz = code == PQ_OP_Z || code == PQ_OP_Y || code == PQ_OP_Z_FLAG ||
                         code == PQ_OP_Y_FLAG;
-        uint32_t rec = 0;
-        if (code >= PQ_OP_H_FLAG && code != PQ_OP_NOISE && !(slot & kSlotPlane)) {
-          rec = (px ? kOpRecX : 0u) | (pz ? kOpRecZ : 0u);
-          m2 = a.recs[(2ull * slot) * W + w];
-          m3 = slot;
-          flags = true;
-        } else if (px || pz) {
-          const uint64_t f =
-              code >= PQ_OP_H_FLAG ? gp[2ull * (slot & ~kSlotPlane)] : ~0ull;
-          if (px) m0 ^= f;
-          if (pz) m1 ^= f;
-        }
         J.cw = (code == PQ_OP_H ? kOpH : code == PQ_OP_S ? kOpS : 0u) |
                (code == PQ_OP_CX ? kOpCX : code == PQ_OP_CZ ? kOpCZ : 0u) |
-               ((m0 | m1 | m2 | m3) ? kOpMasks : 0u) | rec |
+               (px ? (flg ? kOpFlagX : kOpNotX) : 0u) | (pz ? (flg ? kOpFlagZ : kOpNotZ) : 0u) |
+               (rec ? kOpRecord : 0u) | (na != kNone || nb != kNone || flg ? kOpMasks : 0u) |
                (((pad >> kLayerLenShift) & kLayerLenMask) << kOpLenShift);
         J.qq = qa | ((two ? qb : qa) << 16);
+        if (J.cw & kOpMasks) {
+          const uint64_t w = min(w0 + g, W - 1);
+          const PQ_CONST uint64_t *gp = (const PQ_CONST uint64_t *)a.planes + 2ull * a.nk * w;
+          uint64_t m0 = 0, m1 = 0, m2 = 0, m3 = 0;
+          if (na != kNone) {
+            m0 = gp[2ull * na];
+            m1 = gp[2ull * na + 1];
+          }
+          if (nb != kNone) {
+            m2 = gp[2ull * nb];
+            m3 = gp[2ull * nb + 1];
+          } else if (flg) {
+            m2 = rec ? a.recs[(2ull * slot) * W + w] : gp[2ull * (slot & ~kSlotPlane)];
+            m3 = slot;
+          }
+          uint64_t *M = msk + 4 * u;
+          M[0] = m0;
+          M[1] = m1;
+          M[2] = m2;
+          M[3] = m3;
+          flags |= rec;
+        }
       }
-      sh.ops[t] = J;
-      sh.msk[4 * t + 0] = m0;
-      sh.msk[4 * t + 1] = m1;
-      sh.msk[4 * t + 2] = m2;
-      sh.msk[4 * t + 3] = m3;
+      if (g == 0) sh.ops[t] = J;
     }
     // flags from records are read again where measurements of this window
     // precede them
@@ -260,9 +289,9 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
       if (!(cw & kOpMeas)) {
         if (b + cnt > wn) break;  // a layer part runs whole: it opens the next window
         if (measured && reread) {
-          for (uint32_t t = b + tid; t < wn; t += NT)
-            if (sh.ops[t].cw & (kOpRecX | kOpRecZ))
-              sh.msk[4 * t + 2] = a.recs[2ull * sh.msk[4 * t + 3] * W + w];
+          for (uint32_t u = (b << gs) + tid; u < wn << gs; u += NT)
+            if (sh.ops[u >> gs].cw & kOpRecord)
+              msk[4 * u + 2] = a.recs[2ull * msk[4 * u + 3] * W + min(w0 + (u & g_mask), W - 1)];
           __syncthreads();
         }
         measured = false;
@@ -297,13 +326,14 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
         // The frame moves through a gate as a row does.  Its words are for the
         // last threads: the column work starts at thread 0, and a wave's
         // instruction stream is the bound here, not the SIMD.
-        for (uint32_t o = NT - 1 - tid; o < cnt; o += NT) {
-          const SharedOp J = sh.ops[b + o];
+        for (uint32_t u = NT - 1 - tid; u < cnt << gs; u += NT) {
+          const SharedOp J = sh.ops[b + (u >> gs)];
           const uint32_t qa = J.qq & 0xFFFFu, qb = J.qq >> 16;
-          const uint64_t *M = sh.msk + 4 * (b + o);
-          uint64_t ex = E[qa], ez = E[n + qa];
+          const uint64_t *M = msk + 4 * ((b << gs) + u);
+          uint64_t *Ex = E + (u & g_mask) * 2 * n, *Ez = Ex + n;
+          uint64_t ex = Ex[qa], ez = Ez[qa];
           if (J.cw & (kOpCX | kOpCZ)) {
-            uint64_t fx = E[qb], fz = E[n + qb];
+            uint64_t fx = Ex[qb], fz = Ez[qb];
             if (J.cw & kOpCX) {
               fx ^= ex;
               ez ^= fz;
@@ -311,8 +341,12 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
               fz ^= ex;
               ez ^= fx;
             }
-            E[qb] = fx ^ M[2];
-            E[n + qb] = fz ^ M[3];
+            if (J.cw & kOpMasks) {
+              fx ^= M[2];
+              fz ^= M[3];
+            }
+            Ex[qb] = fx;
+            Ez[qb] = fz;
           } else if (J.cw & kOpH) {
             const uint64_t t = ex;
             ex = ez;
@@ -320,15 +354,17 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
           } else if (J.cw & kOpS) {
             ez ^= ex;
           } else {
-            if (J.cw & kOpRecX) ex ^= M[2];
-            if (J.cw & kOpRecZ) ez ^= M[2];
+            if (J.cw & kOpNotX) ex = ~ex;
+            if (J.cw & kOpNotZ) ez = ~ez;
+            if (J.cw & kOpFlagX) ex ^= M[2];
+            if (J.cw & kOpFlagZ) ez ^= M[2];
           }
           if (J.cw & kOpMasks) {
             ex ^= M[0];
             ez ^= M[1];
           }
-          E[qa] = ex;
-          E[n + qa] = ez;
+          Ex[qa] = ex;
+          Ez[qa] = ez;
         }
         b += cnt;
         cw = rfl(sh.ops[b].cw);
@@ -343,6 +379,7 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
         __syncthreads();
       }
       measured = true;
+      uint32_t scratch_q = kNone;  // wide states: qubit of the last determined one
       const uint32_t mbeg = b, mend = min(wn, b + cnt);
       while (b < mend) {
         // Which of the next measurements have a pivot (a stabilizer row with
@@ -373,15 +410,17 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
         if (!kLds && jr) {
           // determined: as below, but the whole workgroup runs it, KH
           // lanes per column, so a column's words are one contiguous run
-          const uint32_t q = rfl(sh.ops[b].qq), slot = rfl((uint32_t)sh.msk[4 * b]);
+          const uint32_t q = rfl(sh.ops[b].qq), slot = rfl((uint32_t)msk[b * mstep]);
           const uint32_t cpw = 64 / KH, sub = lane / KH, kk = lane - sub * KH;
           const uint64_t below = ((1ull << kk) - 1) << (sub * KH);
-          uint64_t rx = 0;
-          for (uint32_t i = tid; i < n; i += NT)
-            if ((read_lane64(xqv, rfl(i >> 6)) >> lane) & 1) rx ^= Rv[n + i];
-          if (__ballot(rx != 0)) {
-            rx = wave_xor(rx);
-            if (lane == 0) lds_xor(&sh.rx[slot2], rx);
+          for (uint32_t g = 0; g < G; ++g) {
+            uint64_t rx = 0;
+            for (uint32_t i = tid; i < n; i += NT)
+              if ((read_lane64(xqv, rfl(i >> 6)) >> lane) & 1) rx ^= Rv[g * R + n + i];
+            if (__ballot(rx != 0)) {
+              rx = wave_xor(rx);
+              if (lane == 0) lds_xor(&sh.rx[slot2][g], rx);
+            }
           }
           const uint64_t cm = __shfl(xqv, kk, 64);
           const uint64_t c = sub < cpw ? cm : 0ull;
@@ -414,31 +453,25 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
           // the other slot is free: it was read before this barrier
           if (tid == 0) {
             sh.tot[slot2 ^ 1] = 0;
-            sh.rx[slot2 ^ 1] = 0;
+            for (uint32_t g = 0; g < G; ++g) sh.rx[slot2 ^ 1][g] = 0;
           }
           __syncthreads();
-          if (b + 1 == mend) {
-            for (uint32_t j = tid; j < n; j += NT) {
-              P[j * KW + K2] = 0;
-              P[(n + j) * KW + K2] = j == q ? 1ull : 0ull;
-            }
-          }
-          if (tid == 0) {
+          scratch_q = q;
+          if (tid < G) {
             const uint32_t cst = (sh.tot[slot2] >> 1) & 1u;
-            const uint64_t rxa = sh.rx[slot2];
-            if (!(sh.ops[b].cw & kOpDropped)) {
-              a.recs[(2ull * slot) * W + w] = rxa ^ (0ull - (uint64_t)cst) ^ E[q];
-              a.recs[(2ull * slot + 1) * W + w] = ~0ull;
+            const uint64_t rxa = sh.rx[slot2][tid];
+            if (!(sh.ops[b].cw & kOpDropped) && ((live >> tid) & 1)) {
+              uint64_t *rec = a.recs + (2ull * slot) * W + w0 + tid;
+              rec[0] = rxa ^ (0ull - (uint64_t)cst) ^ E[tid * 2 * n + q];
+              rec[W] = ~0ull;
             }
-            rc[K2] = cst;
-            Rv[2 * n] = rxa;
+            if (tid == 0) rc[K2] = cst;
+            Rv[tid * R + 2 * n] = rxa;
           }
           slot2 ^= 1;
         }
         if (jr == nm) {
           b += nm;
-          // the scratch row's writes are in before the gates
-          if (!kLds && b == mend) __syncthreads();
           continue;
         }
 
@@ -447,14 +480,16 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
         // becomes row n+p, and row n+p becomes Z_q with the coin as its sign
         {
           const uint32_t q = sh.ops[b + jr].qq;
-          const uint64_t M0 = sh.msk[4 * (b + jr)], m = sh.msk[4 * (b + jr) + 1];
+          const uint64_t M0 = msk[(b + jr) * mstep], m = msk[(b + jr) * mstep + 1];
           if (kLds) xqv = lane < K2 ? P[__umul24(q, KW) + lane] : 0ull;
-          const uint64_t exq = E[q];
           const uint32_t kp = (uint32_t)__ffsll((long long)(__ballot(xqv != 0) >> KH)) - 1;
           const uint32_t bp = (uint32_t)__ffsll((long long)read_lane64(xqv, KH + kp)) - 1;
           const uint32_t p = 64 * kp + bp;
           const uint64_t bit = 1ull << bp;
-          const uint64_t Rs = Rv[n + p];
+          // group of this thread's Rv rows, and of this wave's coin
+          const uint32_t rg = (NT - 1 - tid) & g_mask, cg = nw - 1 - wv;
+          const uint64_t Rs = Rv[rg * R + n + p];
+          const uint64_t Rc = cg < G ? Rv[cg * R + n + p] : 0ull;
           const uint64_t rck = rc[kp];
           const uint64_t rs = 0ull - ((rc[KH + kp] >> bp) & 1);
           if (lane == kp || lane == KH + kp) xqv &= ~bit;  // the rows to update
@@ -496,26 +531,28 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
             }
           }
           // (from the last threads down: the columns start at thread 0)
-          for (uint32_t i = NT - 1 - tid; i < 2 * n; i += NT) {
-            const uint32_t ii = i < n ? i : i - n;
+          for (uint32_t u = NT - 1 - tid; u < (2 * n) << gs; u += NT) {
+            const uint32_t i = u >> gs, ii = i < n ? i : i - n;
             const uint64_t mk = sh.sm[(i < n ? 0 : KH) + (ii >> 6)];
-            if ((mk >> (ii & 63)) & 1) Rv[i] ^= Rs;  // never rows p, n+p
+            if ((mk >> (ii & 63)) & 1) Rv[rg * R + i] ^= Rs;  // never rows p, n+p
           }
-          if (wv == nw - 1) {
+          if (cg < G) {
+            const uint64_t w = min(w0 + cg, W - 1);
             uint64_t coin;
             if (a.coin_planes) {
               coin = a.coin_planes[m * W + w];
             } else {
               const uint64_t key = stream_key(seed, 2 * (mseq0 + m));
-              coin = __ballot((uint32_t)(draw_keyed(key, 64 * w + lane) >> 40) < (uint32_t)(M0 >> 32));
+              coin = __ballot((uint32_t)(draw_keyed(key, 64 * w + lane) >> 40) <
+                              (uint32_t)(M0 >> 32));
             }
             if (lane == 0) {
-              Rv[p] = Rs;
-              Rv[n + p] = coin ^ exq;
-              if (!(sh.ops[b + jr].cw & kOpDropped)) {
-                const uint32_t slot = (uint32_t)M0;
-                a.recs[(2ull * slot) * W + w] = coin;
-                a.recs[(2ull * slot + 1) * W + w] = 0ull;
+              Rv[cg * R + p] = Rc;
+              Rv[cg * R + n + p] = coin ^ E[cg * 2 * n + q];
+              if (!(sh.ops[b + jr].cw & kOpDropped) && ((live >> cg) & 1)) {
+                uint64_t *rec = a.recs + (2ull * (uint32_t)M0) * W + w;
+                rec[0] = coin;
+                rec[W] = 0ull;
               }
             }
           }
@@ -606,10 +643,11 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
         for (uint32_t idx = mbeg + wv; idx < mend; idx += nw) {
           const SharedOp J = sh.ops[idx];
           if (rfl(J.cw) & kOpRandom) continue;
-          const uint32_t q = J.qq, slot = (uint32_t)sh.msk[4 * idx];
+          const uint32_t q = J.qq, slot = (uint32_t)msk[idx * mstep];
+          // lane: group lane % G, and the (lane / G)-th slice of long chains
+          const uint64_t *Rg = Rv + (lane & g_mask) * R + n;
           const uint64_t cv = lane < KH ? P[__umul24(q, KW) + lane] : 0ull;
           const uint64_t rv = lane < KH ? rc[KH + lane] : 0ull;
-          const uint64_t exq = E[q];
           const uint64_t nz = __ballot(cv != 0);
           const bool chain = __ballot((cv & (cv - 1)) != 0) != 0 || (nz & (nz - 1)) != 0;
           const uint32_t par = (uint32_t)__popcll(__ballot(__popcll(cv & rv) & 1));
@@ -623,10 +661,11 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
             const uint32_t cl = (uint32_t)__popcll(c);
             if (cl <= 4) {
               for (uint64_t r = c; r; r &= r - 1)
-                rx ^= Rv[n + 64 * kk + (uint32_t)__ffsll((long long)r) - 1];
+                rx ^= Rg[64 * kk + (uint32_t)__ffsll((long long)r) - 1];
             } else {
               wide = true;
-              if ((c >> lane) & 1) ry ^= Rv[n + 64 * kk + lane];
+              for (uint32_t i = lane >> gs; i < 64; i += 64 >> gs)
+                if ((c >> i) & 1) ry ^= Rg[64 * kk + i];
             }
             if (chain)
               for (uint32_t j = lane; j < n; j += 64)
@@ -665,22 +704,31 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
               }
             }
           }
-          if (wide) rx ^= wave_xor(ry);
+          if (wide) {
+            for (uint32_t off = 32; off >= G; off >>= 1) ry ^= __shfl_xor(ry, off, 64);
+            rx ^= ry;
+          }
           const uint32_t cst = (par ^ wave_sum_bit1(tot)) & 1u;
-          if (lane == 0 && !(J.cw & kOpDropped)) {
-            a.recs[(2ull * slot) * W + w] = rx ^ (0ull - (uint64_t)cst) ^ exq;
-            a.recs[(2ull * slot + 1) * W + w] = ~0ull;
+          if (lane < G && ((live >> lane) & 1) && !(J.cw & kOpDropped)) {
+            uint64_t *rec = a.recs + (2ull * slot) * W + w0 + lane;
+            rec[0] = rx ^ (0ull - (uint64_t)cst) ^ E[lane * 2 * n + q];
+            rec[W] = ~0ull;
           }
           if (idx == last) {  // the scratch row keeps the last product
             for (uint32_t j = lane; j < n; j += 64) {
               P[j * KW + K2] = 0;
               P[(n + j) * KW + K2] = j == q ? 1ull : 0ull;
             }
-            if (lane == 0) {
-              rc[K2] = cst;
-              Rv[2 * n] = rx;
-            }
+            if (lane == 0) rc[K2] = cst;
+            if (lane < G) Rv[lane * R + 2 * n] = rx;
           }
+        }
+        __syncthreads();
+      }
+      if (!kLds && scratch_q != kNone) {  // the scratch row keeps the last product
+        for (uint32_t j = tid; j < n; j += NT) {
+          P[j * KW + K2] = 0;
+          P[(n + j) * KW + K2] = j == scratch_q ? 1ull : 0ull;
         }
         __syncthreads();
       }
@@ -694,18 +742,20 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
 
   // ---- the 64-shot words ----
   // <E, P_i> of 64 rows at a time: a column's word is the lane mask.  Row
-  // words times column shares over the waves, gathered in Rv.
+  // words times column shares times groups over the waves, gathered in Rv.
   {
-    const uint32_t parts = max(1u, 2 * nw / KW);
+    const uint32_t parts = max(1u, 2 * nw / (KW << gs));
     const uint32_t per = (n + parts - 1) / parts;
-    for (uint32_t task = wv; task < KW * parts; task += nw) {
-      const uint32_t kk = task / parts, pt = task - kk * parts;
+    for (uint32_t task = wv; task < (KW * parts) << gs; task += nw) {
+      const uint32_t g = task & g_mask, tk = task >> gs;
+      const uint32_t kk = tk / parts, pt = tk - kk * parts;
       const uint32_t ja = pt * per, jb = min(n, ja + per);
+      const uint64_t *Eg = E + g * 2 * n;
       uint64_t acc = 0;
       for (uint32_t j0 = ja; j0 < jb; j0 += 64) {
         const uint32_t jl = min(j0 + lane, n - 1);
         const uint64_t xw = P[jl * KW + kk], zw = P[(n + jl) * KW + kk];
-        const uint64_t xe = E[jl], ze = E[n + jl];
+        const uint64_t xe = Eg[jl], ze = Eg[n + jl];
         const uint32_t cnt = min(64u, jb - j0);
         for (uint32_t t = 0; t < cnt; ++t) {
           const uint64_t sx = read_lane64(xw, t), sz = read_lane64(zw, t);
@@ -716,25 +766,39 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
       }
       if (pt == 0) acc ^= 0ull - ((rc[kk] >> lane) & 1);
       const uint32_t ii = 64 * (kk < KH ? kk : kk - KH) + lane;
-      if (kk == 2 * KH) {
-        if (lane == 0) lds_xor(Rv + 2 * n, acc);
+      if (kk == K2) {
+        if (lane == 0) lds_xor(Rv + g * R + 2 * n, acc);
       } else if (ii < n) {
-        lds_xor(Rv + (kk < KH ? 0 : n) + ii, acc);
+        lds_xor(Rv + g * R + (kk < KH ? 0 : n) + ii, acc);
       }
     }
   }
   __syncthreads();
-  for (uint32_t i = tid; i < R; i += NT) Tr[i] = Rv[i];
+  for (uint32_t g = 0; g < G; ++g)
+    if ((live >> g) & 1)
+      for (uint32_t i = tid; i < R; i += NT) T0[g * blk + 2ull * n * R + i] = Rv[g * R + i];
+  if (a.packed) {
+    // one workgroup leaves the columns for k_shared_expand: the first that
+    // holds a group that ran
+    bool later = false;
+    if (a.shared == kSharedChecked)
+      for (uint64_t i = tid; i < w0; i += NT) later |= a.done[i] != 0;
+    else
+      later = w0 != 0;
+    if (!__syncthreads_or(later))
+      for (uint32_t i = tid; i < 2 * n * KW; i += NT) a.packed[i] = P[i];
+    return live;
+  }
   __syncthreads();
-  // Wide states: the packed block covers the first KW tableau columns; those
-  // are written last, from a copy.
+  // Columns in the tableau: the packed block covers the first KW tableau
+  // columns of its group; those are written last, from a copy.
   const uint32_t c0 = kLds ? 0 : KW;
   if (!kLds) {
     for (uint32_t i = tid; i < c0 * KW; i += NT) dyn[i] = P[i];
     __syncthreads();
   }
   // a wave per column
-  auto expand = [&](uint32_t c, const uint64_t *src) {
+  auto expand = [&](uint64_t *T, uint32_t c, const uint64_t *src) {
     const uint64_t v0 = lane < KW ? src[lane] : 0ull;
     const uint64_t v1 = lane + 64 < KW ? src[lane + 64] : 0ull;
     uint64_t *dst = T + (uint64_t)c * R;
@@ -747,32 +811,87 @@ __device__ bool shared_word(const ProgramArgs &a, uint64_t seed, uint64_t mseq0,
     const uint64_t s = K2 < 64 ? read_lane64(v0, K2) : read_lane64(v1, K2 - 64);
     if (lane == 0) dst[2 * n] = 0ull - (s & 1);
   };
-  for (uint32_t c = c0 + wv; c < 2 * n; c += nw) expand(c, P + c * KW);
-  if (!kLds) {
-    __syncthreads();
-    for (uint32_t c = wv; c < c0; c += nw) expand(c, dyn + c * KW);
+  for (uint32_t g = 0; g < G; ++g) {
+    if (!((live >> g) & 1)) continue;
+    uint64_t *T = T0 + g * blk;
+    for (uint32_t c = c0 + wv; c < 2 * n; c += nw) expand(T, c, P + c * KW);
+    if (!kLds) {
+      __syncthreads();
+      for (uint32_t c = wv; c < c0; c += nw) expand(T, c, dyn + c * KW);
+    }
   }
   __syncthreads();
-  return true;
+  return live;
 }
 
 struct ProgParams {
   uint64_t seed, mseq0, nseq0;
 };
 
-// One workgroup per word group.  With a.done, groups that ran are marked
-// there and the per-shot kernel launched behind this one passes over them.
+// One workgroup per G = 1 << a.gshift word groups.  With a.done, groups that
+// ran are marked there and the per-shot kernel launched behind this one passes
+// over them.
 template <bool kLds>
 __global__ __launch_bounds__(kSharedThreads) void k_program_shared(
     ProgramArgs a, const ProgParams *__restrict__ pp) {
   extern __shared__ uint64_t dyn[];
   __shared__ SharedLds sh;
   const uint64_t seed = pp->seed, mseq0 = pp->mseq0;
-  for (uint64_t wi = blockIdx.x; wi < a.nwords; wi += gridDim.x) {
-    const bool ran = shared_word<kLds>(a, seed, mseq0, a.word0 + wi, dyn, sh);
-    if (a.done && threadIdx.x == 0) a.done[a.word0 + wi] = ran ? 1u : 0u;
+  for (uint64_t i = blockIdx.x; i << a.gshift < a.W; i += gridDim.x) {
+    shared_words<kLds>(a, seed, mseq0, i << a.gshift, a.gshift, dyn, sh);
     __syncthreads();
   }
+}
+
+// done[w] = whether group w's X/Z are the |0...0> tableau; done starts at 1.
+// One block per group and share of its words.
+__global__ __launch_bounds__(256) void k_shared_verify(const uint64_t *__restrict__ tab,
+                                                       uint32_t n, uint32_t R, uint64_t blk,
+                                                       uint64_t W, uint32_t *done) {
+  const uint32_t total = 2 * n * R, M = R + 1;
+  const uint32_t NT = 256 * gridDim.x, first = blockIdx.x * 256 + threadIdx.x, step = NT % M;
+  for (uint64_t w = blockIdx.y; w < W; w += gridDim.y) {
+    const uint64_t *T = tab + w * blk;
+    uint32_t rem = first % M;
+    bool bad = false;
+    for (uint32_t base = first; base < total && !bad; base += 8 * NT) {
+      uint64_t v[8];
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) v[u] = T[min(base + u * NT, total - 1)];
+#pragma unroll
+      for (uint32_t u = 0; u < 8; ++u) {
+        bad |= base + u * NT < total && v[u] != (rem == 0 ? ~0ull : 0ull);
+        rem += step;
+        if (rem >= M) rem -= M;
+      }
+    }
+    if (bad) done[w] = 0;
+  }
+}
+
+__global__ void k_fill_u32(uint32_t *p, uint64_t n, uint32_t v) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
+       i += (uint64_t)gridDim.x * blockDim.x)
+    p[i] = v;
+}
+
+// The packed columns as 64-shot words in every word group (done: those that
+// ran).  A block per 256 rows of a column and share of the groups: the word is
+// the same in every group, so it is made once.
+__global__ __launch_bounds__(256) void k_shared_expand(uint64_t *__restrict__ tab,
+                                                       const uint64_t *__restrict__ packed,
+                                                       uint32_t n, uint32_t R, uint64_t blk,
+                                                       uint64_t W,
+                                                       const uint32_t *__restrict__ done) {
+  const uint32_t row = blockIdx.x * 256 + threadIdx.x, c = blockIdx.y;
+  if (row >= R) return;
+  const uint32_t KH = (n + 63) / 64, KW = 2 * KH + 1;
+  const uint32_t i = row < n ? row : row - n;
+  const uint32_t k = row < n ? i >> 6 : row < 2 * n ? KH + (i >> 6) : 2 * KH;
+  const uint32_t bit = row < 2 * n ? i & 63 : 0;
+  const uint64_t v = 0ull - ((packed[c * KW + k] >> bit) & 1);
+  for (uint64_t w = blockIdx.z; w < W; w += gridDim.z)
+    if (!done || done[w]) tab[w * blk + (uint64_t)c * R + row] = v;
 }
 
 // The members of a mixed batch that may run packed: work items (circuit << 40 |
@@ -793,39 +912,54 @@ __global__ __launch_bounds__(kSharedThreads) void k_batch_shared(
     if (it >= nitems) break;
     const uint64_t code = rfl64(items[it]);
     const BatchCircuit &bc = circ[(uint32_t)(code >> 40)];
-    if (!bc.a.shared || packed_in_lds(bc.a.n) != kLds) continue;
+    if (!bc.a.shared || packed_in_lds(bc.a.n, bc.a.masked) != kLds) continue;
     const uint64_t w = code & ((1ull << 40) - 1);
     const uint64_t wend = min(w + wtile, bc.a.nwords);
     for (uint64_t wi = w; wi < wend; ++wi) {
-      const bool ran = shared_word<kLds>(bc.a, bc.seed, bc.mseq0, wi, dyn, sh);
-      if (threadIdx.x == 0) {
-        if (bc.a.done) bc.a.done[wi] = ran ? 1u : 0u;
-        if (ran) atomicAdd(counter + 2, 1ull);
-      }
+      const uint32_t ran = shared_words<kLds>(bc.a, bc.seed, bc.mseq0, wi, 0, dyn, sh);
+      if (threadIdx.x == 0 && ran) atomicAdd(counter + 2, 1ull);
+      __syncthreads();
     }
   }
 }
 
 }  // namespace
 
-bool shared_wide(uint32_t n) { return !packed_in_lds(n); }
-
 bool shared_fits(uint32_t n) { return n >= 1 && n <= kSharedMaxQubits; }
 
-size_t shared_lds_bytes(uint32_t n) {
-  return 8 * (packed_in_lds(n) ? packed_words(n) : 4ull * n + 1);
+bool shared_wide(uint32_t n, bool masked) { return !packed_in_lds(n, masked); }
+
+static size_t lds_bytes(uint32_t n, bool masked, uint32_t gshift) {
+  return 8 * (groups_words(n, masked, gshift) +
+              (packed_in_lds(n, masked) ? packed_words(n) : 0));
 }
 
-hipError_t prepare_shared(uint32_t n) {
-  const void *fn = packed_in_lds(n) ? (const void *)k_program_shared<true>
-                                    : (const void *)k_program_shared<false>;
-  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)kSharedLdsBytes);
+size_t shared_lds_bytes(uint32_t n, bool masked) { return lds_bytes(n, masked, 0); }
+
+// Word groups per workgroup.  Groups that share a workgroup share the packed
+// X/Z work; more workgroups finish sooner on an empty GPU.
+uint32_t shared_gshift(uint32_t n, uint64_t W, bool masked) {
+  uint32_t gs = 0;
+  const uint64_t least = packed_in_lds(n, masked) ? 64 : 1;
+  while ((2u << gs) <= kSharedMaxGroups && (W >> (gs + 1)) >= least &&
+         lds_bytes(n, masked, gs + 1) <= kSharedLdsBytes)
+    ++gs;
+  return gs;
 }
 
-hipError_t prepare_batch_shared() {
+// Whether the tableau check and the 64-shot words are launches of their own,
+// over the whole GPU: for a small state the two launches cost more than they
+// save.
+bool shared_split(uint32_t n, uint64_t W, bool masked) {
+  return !packed_in_lds(n, masked) || W * (2ull * n + 1) * (2ull * n + 1) * 8 >= (32ull << 20);
+}
+
+uint64_t shared_packed_bytes(uint32_t n) { return 8 * packed_words(n); }
+
+hipError_t prepare_shared() {
   hipError_t e = hipSuccess;
-  for (const void *fn : {(const void *)k_batch_shared<true>, (const void *)k_batch_shared<false>})
+  for (const void *fn : {(const void *)k_program_shared<true>, (const void *)k_program_shared<false>,
+                         (const void *)k_batch_shared<true>, (const void *)k_batch_shared<false>})
     if (e == hipSuccess)
       e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
                               (int)kSharedLdsBytes);
@@ -838,8 +972,8 @@ hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const ui
   wtile = std::max<uint32_t>(wtile, 1);
   // as many workgroups per CU as the largest member's LDS allows
   auto blocks = [&](size_t lds) {
-    return dim3((uint32_t)std::min<uint64_t>(
-        nitems, cus * std::min<uint64_t>(4, std::max<uint64_t>(1, 160 * 1024 / (lds + sizeof(SharedLds))))));
+    const uint64_t per_cu = std::max<uint64_t>(1, 160 * 1024 / (lds + sizeof(SharedLds)));
+    return dim3((uint32_t)std::min<uint64_t>(nitems, cus * std::min<uint64_t>(4, per_cu)));
   };
   if (nitems && lds_packed)
     hipLaunchKernelGGL(k_batch_shared<true>, blocks(lds_packed), dim3(kSharedThreads), lds_packed,
@@ -850,17 +984,40 @@ hipError_t launch_batch_shared(hipStream_t s, const BatchCircuit *circ, const ui
   return hipGetLastError();
 }
 
-hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params) {
-  if (!a.nwords) return hipSuccess;
-  const size_t lds = shared_lds_bytes(a.n);
+hipError_t launch_shared(hipStream_t s, const ProgramArgs &args, const void *params) {
+  ProgramArgs a = args;
+  if (!a.W) return hipSuccess;
+  const uint64_t blk = (uint64_t)a.C * a.R;
+  if (a.packed && a.shared == kSharedVerify) {
+    a.shared = kSharedChecked;
+    hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)std::min<uint64_t>((a.W + 255) / 256, 256)),
+                       dim3(256), 0, s, a.done, a.W, 1u);
+    const uint64_t parts = std::max<uint64_t>(1, std::min<uint64_t>(2048 / a.W + 1,
+                                                                    (2ull * a.n * a.R) >> 13));
+    hipLaunchKernelGGL(k_shared_verify,
+                       dim3((uint32_t)parts, (uint32_t)std::min<uint64_t>(a.W, 65535)), dim3(256),
+                       0, s, a.tab, a.n, a.R, blk, a.W, a.done);
+  }
+  a.gshift = shared_gshift(a.n, a.W, a.masked);
+  const size_t lds = lds_bytes(a.n, a.masked, a.gshift);
+  const uint64_t wgs = (a.W + (1u << a.gshift) - 1) >> a.gshift;
+  const dim3 grid((uint32_t)std::min<uint64_t>(wgs, 1u << 20));
   const uint32_t threads = kSharedThreads;
-  const dim3 grid((uint32_t)std::min<uint64_t>(a.nwords, 1u << 20));
-  if (packed_in_lds(a.n))
+  if (packed_in_lds(a.n, a.masked))
     hipLaunchKernelGGL(k_program_shared<true>, grid, dim3(threads), lds, s, a,
                        (const ProgParams *)params);
   else
     hipLaunchKernelGGL(k_program_shared<false>, grid, dim3(threads), lds, s, a,
                        (const ProgParams *)params);
+  if (a.packed) {
+    // about 65536 blocks, each writing its rows in several word groups
+    const uint64_t blocks = (uint64_t)((a.R + 255) / 256) * 2 * a.n;
+    const uint64_t z = std::max<uint64_t>(1, std::min<uint64_t>(a.W, (65536 + blocks - 1) / blocks));
+    hipLaunchKernelGGL(k_shared_expand,
+                       dim3((a.R + 255) / 256, 2 * a.n, (uint32_t)std::min<uint64_t>(z, 64)),
+                       dim3(256), 0, s, a.tab, a.packed, a.n, a.R, blk, a.W,
+                       a.shared == kSharedChecked ? a.done : nullptr);
+  }
   return hipGetLastError();
 }
 

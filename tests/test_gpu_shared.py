@@ -76,8 +76,10 @@ def check(st, orc):
     (1, 130, 60, 0.2), (2, 64, 80, 0.2), (3, 1, 80, 0.3),
     (63, 65, 900, 0.1), (64, 65, 900, 0.1), (65, 65, 900, 0.1),
     (128, 64, 1500, 0.05), (129, 70, 1500, 0.05),
-    (468, 3, 1600, 0.05), (469, 3, 1600, 0.05), (513, 3, 1600, 0.04),
+    (464, 3, 1600, 0.05), (465, 3, 1600, 0.05), (513, 3, 1600, 0.04),
     (700, 3, 1500, 0.03), (2048, 1, 2400, 0.01), (2049, 1, 2400, 0.01),
+    # two and four word groups per workgroup, the last one short
+    (20, 8193, 300, 0.1), (20, 16385, 300, 0.1), (500, 323, 900, 0.03),
 ])
 def test_shared_equals_oracle(ps, n, B, nops, meas):
     ops = mixed_ops(n, nops, 10 * n + B, meas)
@@ -85,6 +87,42 @@ def test_shared_equals_oracle(ps, n, B, nops, meas):
     orc = O.OracleState(n, B, 17)
     orc.run_program(ops.astype(np.int32))
     st = ps.CliffordState(n, B, 17, True)
+    ps.Program(st, ops).run(st, "persistent")
+    check(st, orc)
+
+
+@pytest.mark.parametrize("n", [30, 500])
+def test_scratch_row_of_mixed_runs(ps, n):
+    """The scratch row keeps the last determined measurement of a run, also where
+    random ones follow it."""
+    from plaquette_simulator import workloads as W
+    b = W.OpList()
+    for r in range(4):
+        for q in range(n):
+            b.cx(q, (q + 1 + r) % n)
+        b.h(5 + r)
+        b.cx(5 + r, 9 + r)
+        for q in (0, 1 + r, 9 + r, 3, 5 + r, 9 + r, 12 + r)[:4 + r]:
+            b.measure(q)
+    ops = b.array()
+    say(f"[case] n={n} determined before random")
+    for cut in (len(ops), len(ops) - 2):
+        orc = O.OracleState(n, 3, 5)
+        orc.run_program(ops[:cut].astype(np.int32))
+        st = ps.CliffordState(n, 3, 5, True)
+        ps.Program(st, ops[:cut]).run(st, "persistent")
+        check(st, orc)
+
+
+@pytest.mark.parametrize("n", [487, 488])
+def test_programs_without_masks(ps, n):
+    # no noise, no flags: no mask area in LDS, so the packed columns fit longer
+    from plaquette_simulator import workloads as W
+    ops = W.random_clifford(n, 1500, n, meas_prob=0.05)
+    say(f"[case] n={n} without masks")
+    orc = O.OracleState(n, 3, 5)
+    orc.run_program(ops.astype(np.int32))
+    st = ps.CliffordState(n, 3, 5, True)
     ps.Program(st, ops).run(st, "persistent")
     check(st, orc)
 
@@ -126,9 +164,12 @@ assert torch.cuda.is_available()
 sys.path[:0] = sys.argv[1:]
 import plaquette_simulator as ps
 from test_gpu_shared import mixed_ops
-n, B = 70, 200
-ops = mixed_ops(n, 600, 4, 0.1)
-for where in ("none", "first", "last"):
+# the check inside the kernel, and as a launch of its own (columns in LDS, in
+# the tableau)
+for n, B, where in ((70, 200, "none"), (70, 200, "first"), (70, 200, "last"),
+                    (70, 14000, "first"), (70, 14000, "last"),
+                    (500, 300, "none"), (500, 300, "first"), (500, 300, "last")):
+    ops = mixed_ops(n, 600, 4, 0.1)
     got = []
     for per_shot in (False, True):
         st = ps.CliffordState(n, B, 21, True)
@@ -146,7 +187,7 @@ for where in ("none", "first", "last"):
         prog.run(st, "persistent")
         st.synchronize()
         got.append((st, planes))
-    assert got[0][0].compare(got[1][0]) == (0, 0), where
+    assert got[0][0].compare(got[1][0]) == (0, 0), (n, B, where)
     del got, planes, st
 print("raw pointer ok")
 """
