@@ -601,6 +601,38 @@ int simulate(pq_program_s *p, FramePlan &F, std::vector<Step> &steps,
         break;
     }
   };
+  // Determined measurements (MeasureDetermined, :189-201) of a run of
+  // measurements wait for its end: what they find is not changed by the
+  // others (Z_q stays in the stabilizer group with its sign), and they then
+  // neither split the run's random measurements into single steps nor wait
+  // for them one by one.
+  std::vector<std::pair<uint32_t, Meas>> pend;  // qubit, measurement
+  auto place_determined = [&]() -> int {
+    for (auto &d : pend) {
+      const uint32_t q = d.first;
+      Meas &m = d.second;
+      t.row_zero(2 * n);
+      uint8_t c = 0;
+      for (uint32_t i = 0; i < n; ++i) {
+        if (!t.x(i, q)) continue;
+        c ^= (t.phase(2 * n, n + i) ? 1 : 0) ^ cst[n + i];
+        t.row_xor(2 * n, n + i);
+        m.rows.push_back(n + i);
+      }
+      // the product is Z_q, whose frame part is E.x[q]
+      for (uint32_t j = 0; j < t.nw; ++j) {
+        const uint64_t zq = (q / 64 == j) ? (1ull << (q % 64)) : 0ull;
+        if (t.X[(size_t)(2 * n) * t.nw + j] != 0 || t.Z[(size_t)(2 * n) * t.nw + j] != zq)
+          return pq_set_error(PQ_ERR_HIP, "frame form: determined product is not Z_q");
+      }
+      cst[2 * n] = c;
+      m.c = c;
+      const uint32_t words = 4 + (uint32_t)m.rows.size();
+      place_meas(std::move(m), false, sx[q], words);
+    }
+    pend.clear();
+    return PQ_OK;
+  };
   for (size_t oi = 0; oi < p->ops.size(); ++oi) {
     const pq_op &o = p->ops[oi];
     const uint32_t q = o.q0, q1 = o.q1;
@@ -724,6 +756,12 @@ int simulate(pq_program_s *p, FramePlan &F, std::vector<Step> &steps,
       case PQ_OP_M: {
         need_rows();
         fold_flip();
+        for (const auto &d : pend)
+          if (d.second.slot == o.slot) {  // the record's last writer stays the last
+            int rc = place_determined();
+            if (rc) return rc;
+            break;
+          }
         Meas m;
         m.exq = E0 + sx[q];
         m.slot = o.slot;
@@ -752,25 +790,12 @@ int simulate(pq_program_s *p, FramePlan &F, std::vector<Step> &steps,
           cst[n + piv] = 0;
           const uint32_t words = 8 + (uint32_t)m.rows.size();
           place_meas(std::move(m), true, sx[q], words);
-        } else {  // MeasureDetermined, :189-201
-          t.row_zero(2 * n);
-          uint8_t c = 0;
-          for (uint32_t i = 0; i < n; ++i) {
-            if (!t.x(i, q)) continue;
-            c ^= (t.phase(2 * n, n + i) ? 1 : 0) ^ cst[n + i];
-            t.row_xor(2 * n, n + i);
-            m.rows.push_back(n + i);
-          }
-          // the product is Z_q, whose frame part is E.x[q]
-          for (uint32_t j = 0; j < t.nw; ++j) {
-            const uint64_t zq = (q / 64 == j) ? (1ull << (q % 64)) : 0ull;
-            if (t.X[(size_t)(2 * n) * t.nw + j] != 0 || t.Z[(size_t)(2 * n) * t.nw + j] != zq)
-              return pq_set_error(PQ_ERR_HIP, "frame form: determined product is not Z_q");
-          }
-          cst[2 * n] = c;
-          m.c = c;
-          const uint32_t words = 4 + (uint32_t)m.rows.size();
-          place_meas(std::move(m), false, sx[q], words);
+        } else {
+          pend.emplace_back(q, std::move(m));
+        }
+        if (oi + 1 == nops || p->ops[oi + 1].code != PQ_OP_M) {
+          int rc = place_determined();
+          if (rc) return rc;
         }
         break;
       }

@@ -1895,6 +1895,12 @@ __device__ __forceinline__ uint32_t rfl(uint32_t v) { return __builtin_amdgcn_re
 // ops.
 constexpr uint32_t kFrameWaves = kFrameThreads / 64;
 
+__device__ __forceinline__ uint64_t read_lane64(uint64_t v, uint32_t l) {
+  const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)v, l);
+  const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(v >> 32), l);
+  return (uint64_t)lo | ((uint64_t)hi << 32);
+}
+
 __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w) {
   extern __shared__ uint64_t dyn[];
   const uint32_t tid = threadIdx.x, lane = lane_id();
@@ -1997,56 +2003,82 @@ __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w)
         __syncthreads();
       } else if (kind == kFrameRandom) {
         // MeasureRandom (MeasurementFunctors.hpp:225-265) with pivot p: the
-        // rowsum rows first (all threads read Rv[n+p] before it changes),
-        // then Rv[p], Rv[n+p] = coin ^ E.x[q] and the record
-        const uint32_t p = h1, slot = rfl(sbuf[pos + 2]), mi = rfl(sbuf[pos + 3]);
-        const uint32_t Tc = rfl(sbuf[pos + 4]), ridx = rfl(sbuf[pos + 5]);
-        const uint32_t ne = rfl(sbuf[pos + 6]), exq = rfl(sbuf[pos + 7]);
-        const uint64_t Rs = Rl[n + p];
-        const uint32_t *ents = sbuf + pos + 8;
-        for (uint32_t e = tid; e < ne; e += kFrameThreads) Rl[ents[e]] ^= Rs;
+        // rowsum rows, then Rv[p], Rv[n+p] = coin ^ E.x[q] and the record.
+        // A run of them (up to 64): the waves draw the coins in turn, then
+        // wave 0 takes the measurements one after the other.  They are short
+        // (about 4 rows each) and each reads what the one before wrote: within
+        // a wave LDS order is enough, so a run costs two barriers, and its
+        // chain neither waits for a draw nor for the next header (d=9, 16384
+        // shots, with the determined ones after their run: 80 + 20 steps for
+        // 80 + 82, k_frame 148 -> 108 us; d=17, 32768 shots: 678 -> 500 us).
+        uint32_t m = 0, at = pos;
+        for (;;) {
+          if ((m & (kFrameWaves - 1)) == wv) {
+            const uint64_t key = stream_key(seed, 2 * (mseq0 + rfl(sbuf[at + 3])));
+            const uint32_t u = (uint32_t)(draw_keyed(key, 64 * w + lane) >> 40);
+            const uint64_t coin = __ballot(u < rfl(sbuf[at + 4]));
+            if (lane == 0) part[m] = coin;
+          }
+          at += 8 + rfl(sbuf[at + 6]);
+          ++m;
+          if (m == 64 || at >= cw || rfl(sbuf[at]) != kFrameRandom) break;
+        }
         __syncthreads();
         if (wv == 0) {
-          const uint64_t key = stream_key(seed, 2 * (mseq0 + mi));
-          const uint32_t u = (uint32_t)(draw_keyed(key, 64 * w + lane) >> 40);
-          const uint64_t coin = __ballot(u < Tc);
-          if (lane == 0) {
-            Rl[p] = Rs;
-            Rl[n + p] = coin ^ dyn[exq];
-            a.recs[(2ull * slot) * a.W + w] = coin;
-            a.recs[(2ull * slot + 1) * a.W + w] = 0ull;
-            if (ridx != kNone) dyn[a.lds_rec + ridx] = coin;
+          const uint64_t coins = part[min(lane, m - 1)];
+          uint32_t hd = sbuf[pos + (lane & 7)], ent = sbuf[min(pos + 8 + lane, cw - 1)];
+          for (uint32_t i = 0;;) {
+            const uint32_t p = __builtin_amdgcn_readlane(hd, 1);
+            const uint32_t slot = __builtin_amdgcn_readlane(hd, 2);
+            const uint32_t ridx = __builtin_amdgcn_readlane(hd, 5);
+            const uint32_t ne = __builtin_amdgcn_readlane(hd, 6);
+            const uint32_t exq = __builtin_amdgcn_readlane(hd, 7);
+            const uint32_t row = ent, here = pos;
+            pos += 8 + ne;
+            ++i;
+            if (i < m) {
+              hd = sbuf[pos + (lane & 7)];
+              ent = sbuf[min(pos + 8 + lane, cw - 1)];
+            }
+            const uint64_t Rs = Rl[n + p], ex = dyn[exq];
+            if (lane < ne) Rl[row] ^= Rs;
+            for (uint32_t e = 64 + lane; e < ne; e += 64) Rl[sbuf[here + 8 + e]] ^= Rs;
+            const uint64_t coin = read_lane64(coins, i - 1);
+            if (lane == 0) {
+              Rl[p] = Rs;
+              Rl[n + p] = coin ^ ex;
+              a.recs[(2ull * slot) * a.W + w] = coin;
+              a.recs[(2ull * slot + 1) * a.W + w] = 0ull;
+              if (ridx != kNone) dyn[a.lds_rec + ridx] = coin;
+            }
+            if (i >= m) break;
           }
         }
-        pos += 8 + ne;
+        pos = at;
         __syncthreads();
       } else {
-        // G determined measurements (MeasureDetermined, :189-201): lane j of
-        // every wave XORs every kFrameWaves-th row of measurement j, wave 0
-        // combines and adds the constant and E.x[q]; their rows exclude the
-        // scratch row, which takes the Rv part of the one flagged last
+        // G determined measurements (MeasureDetermined, :189-201): four lanes
+        // each XOR the measurement's rows in turn, the first adds the constant
+        // and E.x[q]; the rows exclude the scratch row, which takes the Rv
+        // part of the one flagged last
         const uint32_t G = h1;
         const uint32_t *desc = sbuf + pos + 8;
         const uint32_t *rows = desc + 4 * G + 1;
-        if (lane < G) {
-          const uint32_t o1 = lane + 1 < G ? desc[4 * lane + 7] : desc[4 * G];
+        for (uint32_t j = tid >> 2; j < G; j += kFrameThreads / 4) {
+          const uint32_t *dj = desc + 4 * j;
+          const uint32_t slot = dj[0], ridx = dj[1], xq = dj[2];
+          const uint32_t o1 = j + 1 < G ? dj[7] : dj[4];
           uint64_t acc = 0;
-          for (uint32_t e = desc[4 * lane + 3] + wv; e < o1; e += kFrameWaves)
-            acc ^= Rl[rows[e]];
-          part[wv * 64 + lane] = acc;
-        }
-        __syncthreads();
-        if (wv == 0 && lane < G) {
-          uint64_t acc = 0;
-#pragma unroll
-          for (uint32_t v = 0; v < kFrameWaves; ++v) acc ^= part[v * 64 + lane];
-          const uint32_t slot = desc[4 * lane], ridx = desc[4 * lane + 1];
-          const uint32_t xq = desc[4 * lane + 2];
-          const uint64_t res = acc ^ ((xq >> 31) ? ~0ull : 0ull) ^ dyn[xq & 0xFFFFu];
-          a.recs[(2ull * slot) * a.W + w] = res;
-          a.recs[(2ull * slot + 1) * a.W + w] = ~0ull;
-          if (ridx != kNone) dyn[a.lds_rec + ridx] = res;
-          if ((xq >> 30) & 1) Rl[2 * n] = acc;
+          for (uint32_t e = dj[3] + (tid & 3); e < o1; e += 4) acc ^= Rl[rows[e]];
+          acc ^= __shfl_xor(acc, 1, 64);
+          acc ^= __shfl_xor(acc, 2, 64);
+          if ((tid & 3) == 0) {
+            const uint64_t res = acc ^ ((xq >> 31) ? ~0ull : 0ull) ^ dyn[xq & 0xFFFFu];
+            a.recs[(2ull * slot) * a.W + w] = res;
+            a.recs[(2ull * slot + 1) * a.W + w] = ~0ull;
+            if (ridx != kNone) dyn[a.lds_rec + ridx] = res;
+            if ((xq >> 30) & 1) Rl[2 * n] = acc;
+          }
         }
         pos += 8 + 4 * G + 1 + rfl(desc[4 * G]);
         __syncthreads();
