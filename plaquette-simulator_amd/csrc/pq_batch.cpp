@@ -63,7 +63,7 @@ struct pq_batch_s {
   uint32_t threads = kProgramThreadsMax;
   uint32_t blocks = 0;             // 0: CUs x blocks per CU
   uint64_t lds_budget = kProgramLdsBytes;
-  uint64_t noise_tasks = 0;  // the run's noise tasks (word group x 32 ops), all members
+  uint64_t noise_tasks = 0;  // the run's noise tasks (64 pairs of word group and op), all members
   hipEvent_t ev_upload = nullptr, ev_a = nullptr, ev_b = nullptr;
   bool timed = false;
   hipGraph_t graph = nullptr;
@@ -362,12 +362,12 @@ static int run_frame_batch(pq_batch b) {
   }
   HIPCHK(hipMemcpyAsync(b->d_fargs, b->h_fargs, nc * sizeof(FrameArgs), hipMemcpyHostToDevice,
                         b->stream));
-  // the noise tasks (word group x 32 ops) of all members in one numbering
+  // the noise tasks (64 pairs of word group and op) of all members in one numbering
   uint64_t tasks = 0;
   for (uint32_t c = 0; c < nc; ++c) {
     BatchCircuit &bc = b->h_circ[c];
     bc.task0 = tasks;
-    tasks += bc.a.W * ((bc.nnoise + 31) / 32);
+    tasks += (bc.a.W * bc.nnoise + 63) / 64;
   }
   HIPCHK(hipMemcpyAsync(b->d_circ, b->h_circ, nc * sizeof(BatchCircuit), hipMemcpyHostToDevice,
                         b->stream));
@@ -469,13 +469,13 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     if (rc) return rc;
   }
   const uint64_t lds_words = launch_lds(b) / 8;
-  // the noise tasks (word group x 32 ops) of all members in one numbering
+  // the noise tasks (64 pairs of word group and op) of all members in one numbering
   b->noise_tasks = 0;
   for (uint32_t c = 0; c < nc; ++c) {
     BatchCircuit &bc = b->h_circ[c];
     bc.a.lds_words = lds_words;
     bc.task0 = b->noise_tasks;
-    b->noise_tasks += bc.a.W * ((bc.nnoise + 31) / 32);
+    b->noise_tasks += (bc.a.W * bc.nnoise + 63) / 64;
   }
   HIPCHK(hipMemcpyAsync(b->d_circ, b->h_circ, nc * sizeof(BatchCircuit),
                         hipMemcpyHostToDevice, b->stream));

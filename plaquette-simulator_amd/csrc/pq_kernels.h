@@ -118,7 +118,7 @@ struct BatchCircuit {
   uint64_t seed, mseq0, nseq0;
   const NoiseDesc *noise;
   uint32_t nnoise, pad;
-  uint64_t task0;  // first noise task (word group x 32 ops) of this circuit in the batch
+  uint64_t task0;  // first noise task (64 pairs of word group and op) of this circuit in the batch
 };
 // Work items are (circuit << 40 | word group), in execution order; with
 // wtile > 1 an item stands for wtile consecutive word groups of its circuit
@@ -244,7 +244,7 @@ hipError_t launch_frame_noise(hipStream_t s, uint64_t *planes, const NoiseDesc *
                               uint32_t nk, uint64_t w0, uint64_t wn, const void *params,
                               uint32_t ka = 0, uint32_t kb = ~0u);
 // The group-major noise planes of every circuit of a frame batch: `tasks`
-// (word group x 32 ops) over all circuits, circuit c's from circ[c].task0 on,
+// (64 pairs of word group and op) over all circuits, circuit c's from circ[c].task0 on,
 // split evenly over the waves.
 hipError_t launch_batch_frame_noise(hipStream_t s, const BatchCircuit *circ, uint32_t ncirc,
                                     uint64_t tasks);

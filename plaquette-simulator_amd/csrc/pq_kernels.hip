@@ -1746,74 +1746,129 @@ __global__ __launch_bounds__(MAXT) void k_batch_t(
   }
 }
 
-// Noise planes of every circuit of a batch (blockIdx.y = circuit).  The
-// block row's waves are laid out as (noise-op lane) x (word-group lane): one
-// stream key per op and wave, one draw per lane per (op, word group).
-// Lane `lane` of v takes the wave-uniform value val (v_writelane_b32; the
-// lane select goes through M0, so the instruction reads one SGPR).
-// The kernels that call it keep nothing in M0 (no LDS DMA), so the clobber
-// only documents the write.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ uint32_t write_lane(uint32_t v, uint32_t val, uint32_t lane) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tv_writelane_b32 %0, %1, m0"
-               : "+v"(v)
-               : "s"(val), "s"(lane)
-               : "m0");
-  return v;
+// Group-major noise planes [W][nk][2] (the persistent and frame forms).  A lane
+// draws for one noise op and 64, 32 or 16 consecutive shots of a word group
+// and keeps their mask bits in registers, so the lanes' words are one
+// contiguous run: no ballot, lane write or scalar key per draw.  What a draw
+// costs is the mix function (two 64-bit products, of which the second's upper
+// half suffices: 14 vector instructions) and one compare for two draws; only
+// where some lane's draw fires are the bits looked at.  VALU-bound, the SIMDs
+// full, at 40 ns a draw and wave: 41888 ops x 32768 shots (d=17 memory, p =
+// 0.003) 0.88 ms where a wave that drew one op's 64 shots took 1.27 ms; 5904
+// ops x 16384 shots (d=9, p = 0.001) 95 -> 62 us.  (Collecting only which draws
+// fire, by add with carry, and drawing those again: 0.84 ms and 65 us.)
+__device__ __forceinline__ uint32_t mix64_hi(uint64_t z) {
+  // the upper half of mix64(z), but for bit 0, which its bit 31 inverts
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z ^= z >> 27;
+  const uint32_t lo = (uint32_t)z, hi = (uint32_t)(z >> 32);
+  return __umulhi(lo, 0x133111EBu) + lo * 0x94D049BBu + hi * 0x133111EBu;
 }
-#pragma clang diagnostic pop
 
-// Group-major noise planes [W][nk][2] (the frame form).  One wave task
-// covers word group w and noise ops [k0, k0 + 32): lanes 2i and 2i+1 end up
-// holding op k0 + i's X and Z mask words, so a task writes one contiguous run
-// of up to 512 bytes.  Op k's draws use stream 2 (nseq0 + k) + 1, as by plane.
-__device__ __forceinline__ void frame_noise_task(uint64_t *__restrict__ planes,
-                                                 const NoiseDesc *__restrict__ desc,
-                                                 uint32_t nk, uint64_t w, uint32_t k0,
-                                                 uint64_t seed, uint64_t nseq0,
-                                                 uint32_t kend) {
-  const uint32_t lane = lane_id();
-  const uint64_t lane_g = lane_golden();
-  const uint32_t cnt = min(32u, kend - k0);  // ops k0 .. min(k0 + 32, kend) - 1
-  // lane i < cnt derives op k0 + i's stream key
-  const uint64_t key_l = stream_key(seed, 2 * (nseq0 + k0 + min(lane, cnt - 1)) + 1);
-  uint32_t out_lo = 0, out_hi = 0;
-  for (uint32_t i = 0; i < cnt; ++i) {
-    const NoiseDesc d = desc[k0 + i];
-    const uint32_t klo = __builtin_amdgcn_readlane((uint32_t)key_l, i);
-    const uint32_t khi = __builtin_amdgcn_readlane((uint32_t)(key_l >> 32), i);
-    const uint64_t key = ((uint64_t)khi << 32) | klo;
-    bool bx, bz;
-    noise_bits(d, draw_word_lane(key, w, lane_g), bx, bz);
-    const uint64_t mx = __ballot(bx);
-    const uint64_t mz = __ballot(bz);
-    out_lo = write_lane(out_lo, (uint32_t)mx, 2 * i);
-    out_hi = write_lane(out_hi, (uint32_t)(mx >> 32), 2 * i);
-    out_lo = write_lane(out_lo, (uint32_t)mz, 2 * i + 1);
-    out_hi = write_lane(out_hi, (uint32_t)(mz >> 32), 2 * i + 1);
+// Mask bits of N shots from state x on (that of the first shot's draw).
+// `low`: no threshold of the wave's ops is above 2^31, so a draw whose bit 31
+// is set does not fire, and the others' upper halves are mix64_hi's.
+template <uint32_t N>
+__device__ __forceinline__ void noise_shots(const NoiseDesc &d, bool low, uint64_t x, uint32_t &mx,
+                                            uint32_t &mz) {
+  mx = mz = 0;
+  if (low) {
+    const bool flag = d.kind == kNoiseFlag;
+    const uint32_t tx = flag ? d.t1 << 8 : d.t1;
+    const uint32_t z0 = flag ? 0u : d.t0, zn = flag ? 0u : d.t2 - d.t0;
+    const uint32_t tm = flag ? tx : d.t2;
+#pragma unroll
+    for (uint32_t i = 0; i < N; i += 2) {
+      const uint32_t a = mix64_hi(x + i * kGolden), b = mix64_hi(x + (i + 1) * kGolden);
+      if (__ballot(min(a, b) < tm)) {
+        mx |= (a < tx ? 1u << i : 0u) | (b < tx ? 2u << i : 0u);
+        mz |= (a - z0 < zn ? 1u << i : 0u) | (b - z0 < zn ? 2u << i : 0u);
+      }
+    }
+  } else {
+    for (uint32_t i = 0; i < N; ++i) {
+      bool bx, bz;
+      noise_bits(d, mix64(x), bx, bz);
+      mx |= bx ? 1u << i : 0u;
+      mz |= bz ? 1u << i : 0u;
+      x += kGolden;
+    }
   }
-  if (lane < 2 * cnt)
-    planes[(w * nk + k0) * 2 + lane] = ((uint64_t)out_hi << 32) | out_lo;
 }
 
-// Wave task t: word group t / nkb, ops from 32 (t % nkb), nkb = ceil(nk / 32).
-// Word groups [w0, w0 + wn) and noise ops [ka, kb) of the planes.
+// Wave task t: the 64 entries from 64 t on of the numbering (word group, noise
+// op, part) over word groups [w0, w0 + wn) and ops [ka, ka + nr); a part is
+// 64 / kParts shots.
+template <uint32_t kParts>
+__device__ __forceinline__ void frame_noise_task(uint64_t *__restrict__ planes,
+                                                 const NoiseDesc *__restrict__ desc, uint32_t nk,
+                                                 uint64_t w0, uint64_t wn, uint32_t ka,
+                                                 uint32_t nr, uint64_t t, uint64_t seed,
+                                                 uint64_t nseq0) {
+  constexpr uint32_t kEnt = 64 / kParts;  // (word group, op) pairs of a task
+  const uint32_t lane = lane_id(), part = lane % kParts;
+  uint64_t w = t * kEnt / nr;
+  uint32_t k = (uint32_t)(t * kEnt - w * nr) + lane / kParts;
+  if (k >= nr) {
+    const uint32_t over = k / nr;
+    w += over;
+    k -= over * nr;
+  }
+  const bool on = w < wn;
+  w = w0 + (on ? w : wn - 1);
+  k += ka;
+  const NoiseDesc d = desc[k];
+  const bool low = !__ballot(d.kind == kNoiseFlag ? d.t1 > 1u << 23 : d.t2 > 1u << 31);
+  const uint64_t key = stream_key(seed, 2 * (nseq0 + k) + 1);
+  uint64_t x = key + (64 * w + part * kEnt + 1) * kGolden;
+  uint64_t *out = planes + (w * nk + k) * 2;
+  if (kParts == 1) {
+    uint32_t mx[2], mz[2];
+#pragma unroll 1
+    for (uint32_t h = 0; h < 2; ++h) {
+      uint32_t ax, az;
+      noise_shots<32>(d, low, x, ax, az);
+      mx[0] = h ? mx[0] : ax;
+      mz[0] = h ? mz[0] : az;
+      mx[1] = ax;
+      mz[1] = az;
+      x += 32 * kGolden;
+    }
+    if (on) {
+      out[0] = ((uint64_t)mx[1] << 32) | mx[0];
+      out[1] = ((uint64_t)mz[1] << 32) | mz[0];
+    }
+  } else if (kParts == 2) {
+    uint32_t mx, mz;
+    noise_shots<32>(d, low, x, mx, mz);
+    if (on) {
+      reinterpret_cast<uint32_t *>(out)[part] = mx;
+      reinterpret_cast<uint32_t *>(out + 1)[part] = mz;
+    }
+  } else {
+    uint32_t mx, mz;
+    noise_shots<16>(d, low, x, mx, mz);
+    if (on) {
+      reinterpret_cast<uint16_t *>(out)[part] = (uint16_t)mx;
+      reinterpret_cast<uint16_t *>(out + 1)[part] = (uint16_t)mz;
+    }
+  }
+}
+
+template <uint32_t kParts>
 __global__ __launch_bounds__(256) void k_frame_noise(uint64_t *__restrict__ planes,
                                                      const NoiseDesc *__restrict__ desc,
                                                      uint32_t nk, uint64_t w0, uint64_t wn,
-                                                     uint32_t ka, uint32_t kb,
+                                                     uint32_t ka, uint32_t kb, uint64_t tasks,
                                                      const ProgParams *__restrict__ pp) {
   const uint64_t nwv = (uint64_t)gridDim.x * (blockDim.x / 64);
   const uint64_t wave =
       blockIdx.x * (uint64_t)(blockDim.x / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const uint64_t nkb = (kb - ka + 31) / 32;
-  for (uint64_t t = wave; t < wn * nkb; t += nwv)
-    frame_noise_task(planes, desc, nk, w0 + t / nkb, ka + (uint32_t)(t % nkb) * 32, pp->seed,
-                     pp->nseq0, kb);
+  for (uint64_t t = wave; t < tasks; t += nwv)
+    frame_noise_task<kParts>(planes, desc, nk, w0, wn, ka, kb - ka, t, pp->seed, pp->nseq0);
 }
 
-// Frame batch: every circuit's tasks in one numbering (circuit c's from
+// Batch: every circuit's tasks in one numbering (circuit c's from
 // circ[c].task0, circ[ncirc] standing for the end), each wave a contiguous
 // share; the wave finds its first circuit by binary search, then walks on.
 __global__ __launch_bounds__(256) void k_batch_frame_noise(const pq::BatchCircuit *__restrict__ circ,
@@ -1837,10 +1892,8 @@ __global__ __launch_bounds__(256) void k_batch_frame_noise(const pq::BatchCircui
   for (; t < t1; ++t) {
     while (c + 1 < ncirc && circ[c + 1].task0 <= t) ++c;
     const pq::BatchCircuit &bc = circ[c];
-    const uint64_t nkb = (bc.nnoise + 31) / 32;
-    const uint64_t lt = t - bc.task0;
-    frame_noise_task(const_cast<uint64_t *>(bc.a.planes), bc.noise, bc.nnoise, lt / nkb,
-                     (uint32_t)(lt % nkb) * 32, bc.seed, bc.nseq0, bc.nnoise);
+    frame_noise_task<1>(const_cast<uint64_t *>(bc.a.planes), bc.noise, bc.nnoise, 0, bc.a.W, 0,
+                        bc.nnoise, t - bc.task0, bc.seed, bc.nseq0);
   }
 }
 
@@ -2391,18 +2444,24 @@ hipError_t launch_frame_noise(hipStream_t s, uint64_t *planes, const NoiseDesc *
                               uint32_t ka, uint32_t kb) {
   kb = std::min(kb, nk);
   if (ka >= kb || !wn) return hipSuccess;
-  const uint64_t tasks = wn * ((kb - ka + 31) / 32);
+  // Shots per lane: 64 where that leaves every SIMD two waves (2048 in all),
+  // fewer below, where the waves' own chains of draws are the bound.
+  const uint64_t entries = wn * (kb - ka);
+  const uint32_t parts = entries > 64 * 2048 ? 1 : entries > 64 * 1024 ? 2 : 4;
+  const uint64_t tasks = (entries * parts + 63) / 64;
   const uint32_t blocks = (uint32_t)std::min<uint64_t>((tasks + 3) / 4, 1u << 16);
-  hipLaunchKernelGGL(k_frame_noise, dim3(blocks), dim3(256), 0, s, planes, desc, nk, w0, wn, ka,
-                     kb, (const ProgParams *)params);
+  hipLaunchKernelGGL(parts == 1   ? k_frame_noise<1>
+                     : parts == 2 ? k_frame_noise<2>
+                                  : k_frame_noise<4>,
+                     dim3(blocks), dim3(256), 0, s, planes, desc, nk, w0, wn, ka, kb, tasks,
+                     (const ProgParams *)params);
   return hipGetLastError();
 }
 
 hipError_t launch_batch_frame_noise(hipStream_t s, const BatchCircuit *circ, uint32_t ncirc,
                                     uint64_t tasks) {
   if (!ncirc || !tasks) return hipSuccess;
-  // about 8 tasks per wave, at most 65536 blocks
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>((tasks + 31) / 32, 65536);
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>((tasks + 3) / 4, 65536);
   hipLaunchKernelGGL(k_batch_frame_noise, dim3(blocks), dim3(256), 0, s, circ, ncirc, tasks);
   return hipGetLastError();
 }
