@@ -170,6 +170,13 @@ hipError_t prepare_shared();
 hipError_t launch_shared(hipStream_t s, const ProgramArgs &a, const void *params);
 // Whether n qubits' packed columns sit in the tableau, not in the LDS.
 bool shared_wide(uint32_t n, bool masked);
+// Per-shot form of a persistent run with each word group's whole tableau in LDS
+// (pq_local.hip); it takes ProgramArgs::fresh whatever the program opens with.
+constexpr uint32_t kLocalMaxQubits = 64;
+bool local_fits(uint32_t n);
+// Raises the kernel's dynamic-LDS limit (not in a capture).
+hipError_t prepare_local();
+hipError_t launch_local(hipStream_t s, const ProgramArgs &a, const void *params);
 // The batch members whose a.shared is set, before launch_batch (whose
 // work items, word tile and counters it shares).  lds_packed / lds_wide: most
 // LDS bytes of a member with its packed columns in LDS / in the tableau (0: no

@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t wave_sum_bit1(uint32_t v) {
 struct SharedOp {
   uint32_t cw, qq;
 };
-constexpr uint32_t kOpH = 1, kOpS = 2, kOpCX = 4, kOpCZ = 8, kOpGate = 15;
+constexpr uint32_t kOpH = 1, kOpS = 2, kOpCX = 4, kOpCZ = 8;
 constexpr uint32_t kOpMeas = 1u << 4;
 constexpr uint32_t kOpMasks = 1u << 5;    // some mask word may not be zero
 constexpr uint32_t kOpNotX = 1u << 6, kOpNotZ = 1u << 7;  // a Pauli on every shot: x, z flip
