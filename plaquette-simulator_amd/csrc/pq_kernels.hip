@@ -265,11 +265,17 @@ __device__ uint32_t block_excl_sum(uint32_t v, ScanShared &sh, uint32_t *total) 
 //  1. Pivot per shot = first stabilizer row with x_q set (:297-301): an
 //     exclusive OR-scan over the stabilizer rows turns column q into
 //     disjoint "first pivot" masks, one group (p, M) per distinct pivot.
-//  2. Random shots, per group (MeasureRandom :226-265): copy row n+p to row
-//     p, clear row n+p, set its z_q and its r to the coin, all masked by M;
-//     then every row i (not p, n+p) with x_q set in M gets rowsum(i <- p),
-//     masked per shot, with the bit-sliced mod-4 phase (only columns where
-//     the source row is non-identity can contribute).
+//  2. Random shots (MeasureRandom :226-265): per group copy row n+p to row
+//     p, clear row n+p, set its z_q and its r to the coin, all masked by M,
+//     and gather the old rows n+p, each in its shots, into one source row;
+//     then every row i with x_q set in a random shot (other than its group's
+//     p, n+p) gets rowsum(i <- source row), masked per shot, with the
+//     bit-sliced mod-4 phase (only columns where the source row is
+//     non-identity can contribute).  The groups' shots are disjoint, so one
+//     pass serves them all (70 qubits, 2000 shots, 1000 ops a tenth of them
+//     flagged, 50 measurements: 2.00 -> 1.15 ms; 128 qubits, 4096 shots, 800
+//     ops, few pivots: 0.85 -> 0.80 ms).
+//     (Workgroups that share a word group take the pivots one by one.)
 //  3. Determined shots D (MeasureDetermined :190-201): one wave clears the
 //     scratch row in D and folds in stabilizer n+i for ascending i with
 //     destabilizer x_q set, reducing each step's phase across lanes.
@@ -420,22 +426,39 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
   const uint64_t coin = rm ? sh.coin : 0;
   const uint32_t ngroups = sh.ngroups;
 
-  // ---- 2. random shots, one pivot group at a time ----
+  // ---- 2. random shots ----
   const uint32_t C = 2 * n + 1;
-  for (uint32_t g = 0; g < ngroups; ++g) {
+  const uint32_t passes = S == 1 ? min(ngroups, 1u) : ngroups;
+  for (uint32_t g = 0; g < passes; ++g) {
     const uint32_t p = sh.gp[g];
-    const uint64_t M = sh.gm[g];
+    const uint64_t M = S == 1 ? rm : sh.gm[g];
     if (S == 1) {
       for (uint32_t c = tid; c < C; c += NT) {
         uint64_t *col = T + (uint64_t)c * Ru;
-        const uint64_t a = col[n + p];
-        const uint64_t b = col[p];
-        col[p] = (b & ~M) | (a & M);
-        uint64_t na = a & ~M;
-        if (c == n + q) na |= M;
-        if (c == 2 * n) na |= coin & M;
-        col[n + p] = na;
-        s_src[c] = a;
+        const uint64_t set = c == n + q ? ~0ull : c == 2 * n ? coin : 0ull;
+        uint64_t acc = 0;
+        // four pivots at a time: all loads issued before any store (no two
+        // pivots share a row)
+        for (uint32_t h = 0; h < ngroups; h += 4) {
+          uint64_t a[4], b[4];
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            if (h + u < ngroups) {
+              const uint32_t ph = sh.gp[h + u];
+              a[u] = col[n + ph];
+              b[u] = col[ph];
+            }
+#pragma unroll
+          for (uint32_t u = 0; u < 4; ++u)
+            if (h + u < ngroups) {
+              const uint32_t ph = sh.gp[h + u];
+              const uint64_t mh = sh.gm[h + u];
+              acc |= a[u] & mh;
+              col[ph] = (b[u] & ~mh) | (a[u] & mh);
+              col[n + ph] = (a[u] & ~mh) | (set & mh);
+            }
+        }
+        s_src[c] = acc;
       }
     } else {
       // every slice takes the source row before slice 0 rewrites it
@@ -463,10 +486,18 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
     const uint64_t rsrc = s_src[2 * n];
     uint32_t my_rows = 0;
     for (uint32_t i = slice * NT + tid; i < 2 * n; i += NT * S) {
-      if (i == p || i == n + p) continue;
-      const uint64_t mi = M & (own_row ? xv : xq[i]);
+      uint64_t mi = M & (own_row ? xv : xq[i]);
+      if (S == 1) {
+        const uint32_t pi = i < n ? i : i - n;
+        for (uint32_t h = 0; h < ngroups; ++h)
+          if (sh.gp[h] == pi) mi &= ~sh.gm[h];
+        if (census)
+          for (uint32_t h = 0; h < ngroups; ++h) my_rows += (mi & sh.gm[h]) ? 1u : 0u;
+      } else if (i == p || i == n + p) {
+        mi = 0;
+      }
       if (!mi) continue;
-      ++my_rows;
+      if (S > 1) ++my_rows;
       // the phase word is read with the first source columns, not after
       // the row's stores
       const uint64_t ri = T[(uint64_t)(2 * n) * Ru + i];
