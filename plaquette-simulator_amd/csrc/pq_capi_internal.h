@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "plaquette_amd.h"
@@ -26,6 +27,10 @@ struct pq_state_s {
   uint64_t *scratch = nullptr;  // 3W words: flag/noise planes for plain ops
   bool scratch_zeroed = false;
   int32_t *stage = nullptr;     // int32[B] host-vector staging
+  // device_to_host: packed shots on the device and in pinned host memory (kept
+  // from the first call on, at most kShotBytes or one shot), one call at a time
+  uint64_t *shots_dev = nullptr, *shots_host = nullptr;
+  std::mutex shots_mu;
   void *params_dev = nullptr;   // ProgParams of the running program
   void *csum = nullptr;
   // States the server creates borrow a slot stream and allocate with the

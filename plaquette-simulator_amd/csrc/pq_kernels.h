@@ -42,9 +42,11 @@ hipError_t launch_measure(hipStream_t s, uint64_t *tab, const Geom &g,
                           const MeasParams &m);
 size_t measure_lds_bytes(uint32_t n);
 uint32_t measure_max_qubits();
-hipError_t launch_unpack(hipStream_t s, const uint64_t *tab, const Geom &g,
-                         uint64_t b0, uint64_t nb, int32_t *x, int32_t *z,
-                         int32_t *r);
+// Shots [b0, b0 + nb) as packed bits, shot_words(n) words per shot: R rows of
+// ceil(n/64) words of x bits, the same of z, ceil(R/64) words of r.
+uint64_t shot_words(uint32_t n);
+hipError_t launch_shot_bits(hipStream_t s, const uint64_t *tab, const Geom &g, uint64_t b0,
+                            uint64_t nb, uint64_t *out);
 hipError_t launch_pack(hipStream_t s, uint64_t *tab, const Geom &g, uint64_t w0,
                        uint64_t nw, const int32_t *x, const int32_t *z,
                        const int32_t *r);

@@ -608,25 +608,41 @@ __global__ __launch_bounds__(kMeasThreads) void k_measure(
 // ---------------------------------------------------------------------------
 // Host I/O: flat int32 [b][row][col] <-> bit-planes.
 // ---------------------------------------------------------------------------
-__global__ void k_unpack(const uint64_t *__restrict__ tab, uint32_t n,
-                         uint32_t R, uint32_t C, uint64_t b0, uint64_t nb,
-                         int32_t *__restrict__ x, int32_t *__restrict__ z,
-                         int32_t *__restrict__ r) {
-  const uint64_t per = (uint64_t)R * n;
-  const uint64_t total = nb * per;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < total;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t b = i / per;
-    const uint64_t rem = i - b * per;
-    const uint32_t row = (uint32_t)(rem / n);
-    const uint32_t col = (uint32_t)(rem - (uint64_t)row * n);
-    const uint64_t sb = b0 + b;
-    const uint64_t *G = tab + (sb >> 6) * (uint64_t)C * R;
-    const uint32_t bit = (uint32_t)(sb & 63);
-    x[i] = (int32_t)((G[(uint64_t)col * R + row] >> bit) & 1);
-    z[i] = (int32_t)((G[(uint64_t)(n + col) * R + row] >> bit) & 1);
-    if (col == 0)
-      r[b * R + row] = (int32_t)((G[(uint64_t)(2 * n) * R + row] >> bit) & 1);
+// Shots [b0, b0 + nb) as packed bits, a record of shot_words(n) words per shot:
+// rows of ceil(n/64) words of x bits, the same of z, then ceil(R/64) words of r.
+// A wave makes one word of the record for the 64 shots of a group: its lanes
+// read 64 columns' (r: rows') words of one row, and shot s's word is the ballot
+// of their bits s.  The records are 1/32 of the int32 entries that the host
+// makes of them, so neither the link nor the copy's staging is the bound.
+__global__ __launch_bounds__(256) void k_shot_bits(const uint64_t *__restrict__ tab, uint32_t n,
+                                                   uint32_t R, uint32_t C, uint64_t b0,
+                                                   uint64_t nb, uint64_t *__restrict__ out) {
+  const uint32_t lane = lane_id();
+  const uint32_t KC = (n + 63) / 64, half = R * KC, words = 2 * half + (R + 63) / 64;
+  const uint64_t wa = b0 >> 6, groups = ((b0 + nb + 63) >> 6) - wa;
+  const uint64_t nwv = (uint64_t)gridDim.x * (blockDim.x / 64);
+  for (uint64_t t = blockIdx.x * (uint64_t)(blockDim.x / 64) + (threadIdx.x >> 6);
+       t < groups * words; t += nwv) {
+    const uint64_t w = t / words;
+    const uint32_t k = (uint32_t)(t - w * words);
+    const uint64_t *G = tab + (wa + w) * (uint64_t)C * R;
+    uint64_t v = 0;
+    if (k < 2 * half) {
+      const uint32_t kk = k < half ? k : k - half;
+      const uint32_t row = kk / KC, col = 64 * (kk - row * KC) + lane;
+      if (col < n) v = G[(uint64_t)(k < half ? col : n + col) * R + row];
+    } else {
+      const uint32_t row = 64 * (k - 2 * half) + lane;
+      if (row < R) v = G[(uint64_t)(2 * n) * R + row];
+    }
+    uint64_t mine = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < 64; ++s) {
+      const uint64_t bits = __ballot((v >> s) & 1);
+      mine = lane == s ? bits : mine;
+    }
+    const uint64_t shot = 64 * (wa + w) + lane;
+    if (shot >= b0 && shot < b0 + nb) out[(shot - b0) * words + k] = mine;
   }
 }
 
@@ -2285,13 +2301,17 @@ hipError_t launch_measure(hipStream_t s, uint64_t *tab, const Geom &g,
   return hipGetLastError();
 }
 
-hipError_t launch_unpack(hipStream_t s, const uint64_t *tab, const Geom &g,
-                         uint64_t b0, uint64_t nb, int32_t *x, int32_t *z,
-                         int32_t *r) {
-  const uint64_t total = nb * (uint64_t)g.R * g.n;
-  if (!total) return hipSuccess;
-  hipLaunchKernelGGL(k_unpack, dim3(grid_for(total, 256, 65536)), dim3(256), 0, s,
-                     tab, g.n, g.R, g.C, b0, nb, x, z, r);
+uint64_t shot_words(uint32_t n) {
+  const uint64_t R = 2ull * n + 1;
+  return 2 * R * ((n + 63) / 64) + (R + 63) / 64;
+}
+
+hipError_t launch_shot_bits(hipStream_t s, const uint64_t *tab, const Geom &g, uint64_t b0,
+                            uint64_t nb, uint64_t *out) {
+  if (!nb || !g.n) return hipSuccess;
+  const uint64_t tasks = (((b0 + nb + 63) >> 6) - (b0 >> 6)) * shot_words(g.n);
+  hipLaunchKernelGGL(k_shot_bits, dim3(grid_for(tasks, 4, 65536)), dim3(256), 0, s, tab, g.n, g.R,
+                     g.C, b0, nb, out);
   return hipGetLastError();
 }
 
