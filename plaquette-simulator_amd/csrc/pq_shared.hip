@@ -100,7 +100,7 @@ struct SharedLds {
   uint64_t rc[kMaxRowWords];  // sign bits, laid out like a column
   uint64_t sm[kMaxRowWords];  // row mask of the current random measurement
   uint64_t c0[kMaxRowWords];  // and the low bits of its rows' phase sums
-  uint32_t list[512];         // its pivot row's columns (packed columns in LDS)
+  uint32_t list[512];         // its pivot row's columns (columns in the tableau: in dynamic LDS)
   uint32_t bad;               // a word of the state is not the |0...0> tableau's
   // determined measurements of wide states, two in turn: phase count, XOR of
   // Rv rows
@@ -114,8 +114,11 @@ constexpr uint64_t kSharedLdsBytes = 159 * 1024 - sizeof(SharedLds);  // dynamic
 // Dynamic LDS words: Rv and the frame of each of the G word groups, their op
 // masks (programs with noise or flags), and the packed columns if they fit.
 // (Programs without masks keep only the measurements' two words there.)
+__host__ __device__ inline uint64_t mask_words(bool masked, uint32_t gs) {
+  return masked ? (4ull * kChunk) << gs : 2ull * kChunk;
+}
 __host__ __device__ inline uint64_t groups_words(uint32_t n, bool masked, uint32_t gs) {
-  return ((4ull * n + 1) << gs) + (masked ? (4ull * kChunk) << gs : 2ull * kChunk);
+  return ((4ull * n + 1) << gs) + mask_words(masked, gs);
 }
 __host__ __device__ inline uint64_t packed_words(uint32_t n) {
   return 2ull * n * (2ull * ((n + 63) / 64) + 1);
@@ -188,8 +191,9 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
   // packed column c (x_c, or z_{c-n}) starts at P + c * KW: one compact block,
   // in LDS, or at the start of a group's tableau block, which the run
   // overwrites anyway
-  uint64_t *P = kLds ? msk + (masked ? 4 * kChunk * G : 2 * kChunk)
-                     : T0 + ((uint32_t)__ffs((int)live) - 1) * blk;
+  uint64_t *const past = msk + mask_words(masked, gs);
+  uint64_t *P = kLds ? past : T0 + ((uint32_t)__ffs((int)live) - 1) * blk;
+  uint32_t *const list = kLds ? sh.list : reinterpret_cast<uint32_t *>(past);
 
   // ---- |0...0>: destabilizer i = X_i, stabilizer i = Z_i ----
   for (uint32_t u = tid; u < 2 * n * KW; u += NT) {
@@ -508,26 +512,36 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
           }
           __syncthreads();
           if (tid < K2 && dr) lds_xor(rc + tid, dr);
-          if (kLds) {
-            // rows p and n+p, a lane per column; columns where row n+p is not
-            // the identity go on the list
-            for (uint32_t v = wv; v < KH; v += nw) {
-              const uint32_t j = 64 * v + lane;
+          // rows p and n+p, a lane per column; columns where row n+p is not the
+          // identity go on the list
+          constexpr uint32_t kU = kLds ? 1 : 2;
+          for (uint32_t v = wv; v < KH; v += kU * nw) {
+            uint64_t wx[kU], wz[kU], dx[kU], dz[kU];
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u) {
+              const uint64_t *X = P + __umul24(min(64 * (v + u * nw) + lane, n - 1), KW) + kp;
+              wx[u] = X[KH];
+              wz[u] = X[n * KW + KH];
+              dx[u] = X[0];
+              dz[u] = X[n * KW];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kU; ++u) {
+              const uint32_t j = 64 * (v + u * nw) + lane;
               uint32_t ent = 0;
               if (j < n) {
                 uint64_t *X = P + __umul24(j, KW) + kp, *Z = X + n * KW;
-                const uint64_t wx = X[KH], wz = Z[KH], dx = X[0], dz = Z[0];
-                ent = (uint32_t)((wx >> bp) & 1) | ((uint32_t)((wz >> bp) & 1) << 1);
-                X[0] = (dx & ~bit) | (wx & bit);
-                Z[0] = (dz & ~bit) | (wz & bit);
-                X[KH] = wx & ~bit;
-                Z[KH] = (wz & ~bit) | (j == q ? bit : 0ull);
+                ent = (uint32_t)((wx[u] >> bp) & 1) | ((uint32_t)((wz[u] >> bp) & 1) << 1);
+                X[0] = (dx[u] & ~bit) | (wx[u] & bit);
+                Z[0] = (dz[u] & ~bit) | (wz[u] & bit);
+                X[KH] = wx[u] & ~bit;
+                Z[KH] = (wz[u] & ~bit) | (j == q ? bit : 0ull);
               }
               const uint64_t bal = __ballot(ent != 0);
               uint32_t at = 0;
               if (lane == 0 && bal) at = atomicAdd(&sh.nl, (uint32_t)__popcll(bal));
               at = rfl(at) + (uint32_t)__popcll(bal & ((1ull << lane) - 1));
-              if (ent) sh.list[at] = j | (ent << 16);
+              if (ent) list[at] = j | (ent << 16);
             }
           }
           // (from the last threads down: the columns start at thread 0)
@@ -556,7 +570,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
               }
             }
           }
-          if (kLds) __syncthreads();
+          __syncthreads();
           // phases: per row, the sum mod 4 over columns of the phase exponent
           // of row * (row n+p): each thread's columns in registers, then
           // LDS atomics; the low bits' old value gives the carry, and the high
@@ -568,7 +582,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
             const uint32_t nl = sh.nl;
             if (mk)
               for (uint32_t e = my_j; e < nl; e += rpp) {
-                const uint32_t ent = sh.list[e];
+                const uint32_t ent = list[e];
                 uint64_t *X = P + (__umul24(ent & 0xFFFFu, KW) + my_i), *Z = X + n * KW;
                 const uint64_t x = *X, z = *Z;
                 const uint64_t fx = (ent >> 16) & 1 ? mk : 0ull, fz = ent >> 17 ? mk : 0ull;
@@ -577,44 +591,32 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
                 *Z = z ^ fz;
               }
           } else {
-            // K2 lanes of one wave per column (a column's words are one run).
-            // Row n+p's bits come from the lane that holds its word, before
-            // any of the column's lanes stores.
+            // K2 lanes of one wave per listed column (a column's words are one
+            // run), kWideCols columns a lane in flight.  One CU's VALU and its
+            // path to the L2 are the bound: the columns where row n+p is the
+            // identity, the row's bits by ballots, and the rows p and n+p are not
+            // in this pass (n = 1024, 1409 of these in a run: 20 -> 9 us each).
             const uint32_t cpw = 64 / K2, sub = lane / K2, i = lane - sub * K2;
-            const bool use = sub < cpw;
-            const uint64_t mi = __shfl(xqv, i, 64);
-            const uint64_t mk = use ? mi : 0ull;
-            const uint32_t src = min(sub, cpw - 1) * K2 + KH + kp;
-            const uint32_t cstep = nw * cpw;
-            for (uint32_t jw = wv * cpw; jw < n; jw += kWideCols * cstep) {
+            const uint64_t mk = sub < cpw ? sh.sm[i] : 0ull;
+            const uint32_t nl = sh.nl, cstep = nw * cpw;
+            for (uint32_t e0 = wv * cpw; e0 < nl; e0 += kWideCols * cstep) {
               uint64_t x[kWideCols], z[kWideCols];
+              uint32_t ent[kWideCols];
 #pragma unroll
               for (uint32_t u = 0; u < kWideCols; ++u) {
-                const uint32_t j = min(jw + u * cstep + sub, n - 1);
-                const uint64_t *X = P + j * KW + i;
+                const uint32_t e = e0 + u * cstep + sub;
+                ent[u] = e < nl ? list[e] : 0u;
+                const uint64_t *X = P + (__umul24(ent[u] & 0xFFFFu, KW) + i);
                 x[u] = X[0];
                 z[u] = X[n * KW];
               }
 #pragma unroll
               for (uint32_t u = 0; u < kWideCols; ++u) {
-                const uint32_t j = jw + u * cstep + sub;
-                const uint64_t xp = (__ballot((x[u] >> bp) & 1) >> src) & 1;
-                const uint64_t zp = (__ballot((z[u] >> bp) & 1) >> src) & 1;
-                if (use && j < n) {
-                  const uint64_t fx = mk & (0ull - xp), fz = mk & (0ull - zp);
-                  phase_acc(x[u], z[u], fx, fz, c0, c1);
-                  uint64_t nx = x[u] ^ fx, nzv = z[u] ^ fz;
-                  if (i == kp) {
-                    nx = (nx & ~bit) | (xp << bp);
-                    nzv = (nzv & ~bit) | (zp << bp);
-                  } else if (i == KH + kp) {
-                    nx &= ~bit;
-                    nzv = (nzv & ~bit) | (j == q ? bit : 0ull);
-                  }
-                  uint64_t *X = P + j * KW + i;
-                  if (nx != x[u]) X[0] = nx;
-                  if (nzv != z[u]) X[n * KW] = nzv;
-                }
+                const uint64_t fx = (ent[u] >> 16) & 1 ? mk : 0ull, fz = ent[u] >> 17 ? mk : 0ull;
+                phase_acc(x[u], z[u], fx, fz, c0, c1);
+                uint64_t *X = P + (__umul24(ent[u] & 0xFFFFu, KW) + i);
+                if (fx) X[0] = x[u] ^ fx;
+                if (fz) X[n * KW] = z[u] ^ fz;
               }
             }
             ci = i;
@@ -930,8 +932,9 @@ bool shared_fits(uint32_t n) { return n >= 1 && n <= kSharedMaxQubits; }
 bool shared_wide(uint32_t n, bool masked) { return !packed_in_lds(n, masked); }
 
 static size_t lds_bytes(uint32_t n, bool masked, uint32_t gshift) {
+  // the packed columns, or the list of a random measurement's columns
   return 8 * (groups_words(n, masked, gshift) +
-              (packed_in_lds(n, masked) ? packed_words(n) : 0));
+              (packed_in_lds(n, masked) ? packed_words(n) : (n + 1) / 2));
 }
 
 size_t shared_lds_bytes(uint32_t n, bool masked) { return lds_bytes(n, masked, 0); }
