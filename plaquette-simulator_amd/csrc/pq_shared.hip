@@ -26,6 +26,7 @@
 #include "pq_kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 #include "plaquette_amd.h"
 
@@ -743,9 +744,52 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
   __syncthreads();
 
   // ---- the 64-shot words ----
-  // <E, P_i> of 64 rows at a time: a column's word is the lane mask.  Row
-  // words times column shares times groups over the waves, gathered in Rv.
-  {
+  // <E, P_i> of 64 rows at a time, row words times column shares over the
+  // waves, gathered in Rv.
+  auto add_signs = [&](uint32_t g, uint32_t kk, bool share0, uint64_t acc) {
+    if (share0) acc ^= 0ull - ((rc[kk] >> lane) & 1);
+    const uint32_t ii = 64 * (kk < KH ? kk : kk - KH) + lane;
+    if (kk == K2) {
+      if (lane == 0) lds_xor(Rv + g * R + 2 * n, acc);
+    } else if (ii < n) {
+      lds_xor(Rv + g * R + (kk < KH ? 0 : n) + ii, acc);
+    }
+  };
+  if (kLds) {
+    // A lane takes its row's bit of a column as a mask, once for all groups:
+    // VALU-bound.  Column words and frames read from lanes as scalars instead
+    // stalled on every one: 449 qubits, one group 106 -> 50 us of the run's 1180;
+    // 161 qubits, four groups 56 -> 28 us of 337.
+    const uint32_t parts = max(1u, 2 * nw / KW), per = (n + parts - 1) / parts;
+    for (uint32_t task = wv; task < KW * parts; task += nw) {
+      const uint32_t kk = task / parts, pt = task - kk * parts;
+      const uint32_t ja = pt * per, jb = min(n, ja + per);
+      const int32_t *Px = reinterpret_cast<const int32_t *>(P + kk) + (lane >> 5);
+      const int32_t *Pz = Px + 2 * n * KW;
+      const uint32_t sh31 = 31 - (lane & 31);
+      auto run = [&](auto groups) {
+        constexpr uint32_t kG = decltype(groups)::value;
+        uint64_t acc[kG] = {};
+#pragma unroll 4
+        for (uint32_t j = ja; j < jb; ++j) {
+          const uint64_t mx = (uint64_t)(int64_t)((Px[2 * j * KW] << sh31) >> 31);
+          const uint64_t mz = (uint64_t)(int64_t)((Pz[2 * j * KW] << sh31) >> 31);
+#pragma unroll
+          for (uint32_t g = 0; g < kG; ++g)
+            acc[g] ^= (mx & E[g * 2 * n + n + j]) ^ (mz & E[g * 2 * n + j]);
+        }
+#pragma unroll
+        for (uint32_t g = 0; g < kG; ++g) add_signs(g, kk, pt == 0, acc[g]);
+      };
+      if (gs == 0)
+        run(std::integral_constant<uint32_t, 1>());
+      else if (gs == 1)
+        run(std::integral_constant<uint32_t, 2>());
+      else
+        run(std::integral_constant<uint32_t, 4>());
+    }
+  } else {
+    // columns in the tableau: 64 of them at a time, a column's word as lane mask
     const uint32_t parts = max(1u, 2 * nw / (KW << gs));
     const uint32_t per = (n + parts - 1) / parts;
     for (uint32_t task = wv; task < (KW * parts) << gs; task += nw) {
@@ -766,13 +810,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
           acc ^= __builtin_amdgcn_inverse_ballot_w64(sz) ? ex : 0ull;
         }
       }
-      if (pt == 0) acc ^= 0ull - ((rc[kk] >> lane) & 1);
-      const uint32_t ii = 64 * (kk < KH ? kk : kk - KH) + lane;
-      if (kk == K2) {
-        if (lane == 0) lds_xor(Rv + g * R + 2 * n, acc);
-      } else if (ii < n) {
-        lds_xor(Rv + g * R + (kk < KH ? 0 : n) + ii, acc);
-      }
+      add_signs(g, kk, pt == 0, acc);
     }
   }
   __syncthreads();
