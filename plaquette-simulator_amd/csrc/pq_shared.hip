@@ -37,7 +37,9 @@ namespace {
 #define PQ_CONST __attribute__((address_space(4)))
 
 constexpr uint32_t kChunk = 448;       // staged ops; must equal kStage in pq_kernels.hip
-constexpr uint32_t kWideCols = 5;      // columns a lane has in flight (wide states)
+// wide states: columns a lane has in flight, in determined chains and in the
+// rowsums of random measurements (more spill registers)
+constexpr uint32_t kWideCols = 5, kRandCols = 6;
 constexpr uint32_t kWindow = 64;       // measurements whose pivots are checked at once
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
@@ -593,18 +595,18 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
               }
           } else {
             // K2 lanes of one wave per listed column (a column's words are one
-            // run), kWideCols columns a lane in flight.  One CU's VALU and its
+            // run), kRandCols columns a lane in flight.  One CU's VALU and its
             // path to the L2 are the bound: the columns where row n+p is the
             // identity, the row's bits by ballots, and the rows p and n+p are not
             // in this pass (n = 1024, 1409 of these in a run: 20 -> 9 us each).
             const uint32_t cpw = 64 / K2, sub = lane / K2, i = lane - sub * K2;
             const uint64_t mk = sub < cpw ? sh.sm[i] : 0ull;
             const uint32_t nl = sh.nl, cstep = nw * cpw;
-            for (uint32_t e0 = wv * cpw; e0 < nl; e0 += kWideCols * cstep) {
-              uint64_t x[kWideCols], z[kWideCols];
-              uint32_t ent[kWideCols];
+            for (uint32_t e0 = wv * cpw; e0 < nl; e0 += kRandCols * cstep) {
+              uint64_t x[kRandCols], z[kRandCols];
+              uint32_t ent[kRandCols];
 #pragma unroll
-              for (uint32_t u = 0; u < kWideCols; ++u) {
+              for (uint32_t u = 0; u < kRandCols; ++u) {
                 const uint32_t e = e0 + u * cstep + sub;
                 ent[u] = e < nl ? list[e] : 0u;
                 const uint64_t *X = P + (__umul24(ent[u] & 0xFFFFu, KW) + i);
@@ -612,7 +614,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
                 z[u] = X[n * KW];
               }
 #pragma unroll
-              for (uint32_t u = 0; u < kWideCols; ++u) {
+              for (uint32_t u = 0; u < kRandCols; ++u) {
                 const uint64_t fx = (ent[u] >> 16) & 1 ? mk : 0ull, fz = ent[u] >> 17 ? mk : 0ull;
                 phase_acc(x[u], z[u], fx, fz, c0, c1);
                 uint64_t *X = P + (__umul24(ent[u] & 0xFFFFu, KW) + i);
@@ -755,7 +757,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
       lds_xor(Rv + g * R + (kk < KH ? 0 : n) + ii, acc);
     }
   };
-  if (kLds) {
+  {
     // A lane takes its row's bit of a column as a mask, once for all groups:
     // VALU-bound.  Column words and frames read from lanes as scalars instead
     // stalled on every one: 449 qubits, one group 106 -> 50 us of the run's 1180;
@@ -787,30 +789,6 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
         run(std::integral_constant<uint32_t, 2>());
       else
         run(std::integral_constant<uint32_t, 4>());
-    }
-  } else {
-    // columns in the tableau: 64 of them at a time, a column's word as lane mask
-    const uint32_t parts = max(1u, 2 * nw / (KW << gs));
-    const uint32_t per = (n + parts - 1) / parts;
-    for (uint32_t task = wv; task < (KW * parts) << gs; task += nw) {
-      const uint32_t g = task & g_mask, tk = task >> gs;
-      const uint32_t kk = tk / parts, pt = tk - kk * parts;
-      const uint32_t ja = pt * per, jb = min(n, ja + per);
-      const uint64_t *Eg = E + g * 2 * n;
-      uint64_t acc = 0;
-      for (uint32_t j0 = ja; j0 < jb; j0 += 64) {
-        const uint32_t jl = min(j0 + lane, n - 1);
-        const uint64_t xw = P[jl * KW + kk], zw = P[(n + jl) * KW + kk];
-        const uint64_t xe = Eg[jl], ze = Eg[n + jl];
-        const uint32_t cnt = min(64u, jb - j0);
-        for (uint32_t t = 0; t < cnt; ++t) {
-          const uint64_t sx = read_lane64(xw, t), sz = read_lane64(zw, t);
-          const uint64_t ex = read_lane64(xe, t), ez = read_lane64(ze, t);
-          acc ^= __builtin_amdgcn_inverse_ballot_w64(sx) ? ez : 0ull;
-          acc ^= __builtin_amdgcn_inverse_ballot_w64(sz) ? ex : 0ull;
-        }
-      }
-      add_signs(g, kk, pt == 0, acc);
     }
   }
   __syncthreads();
