@@ -432,10 +432,12 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     // from |0...0> the shared-X/Z kernel, as in a standalone run; a captured
     // launch holds both kernels, and the members' arguments say which
     // one runs each
-    uint32_t shared = 0;
+    uint32_t shared = 0, gshift = 0;
     if (s->tab && shared_allowed(s, p)) {
       size_t &lds = shared_lds[shared_wide((uint32_t)s->n, p->masked) ? 1 : 0];
-      lds = std::max(lds, shared_lds_bytes((uint32_t)s->n, p->masked));
+      gshift = shared_batch_gshift((uint32_t)s->n, s->W, p->masked, b->nitems,
+                                   (uint32_t)cu_count());
+      lds = std::max(lds, shared_lds_bytes((uint32_t)s->n, p->masked, gshift));
       if (s->xz_identity) shared = s->exposed ? kSharedVerify : kSharedKnown;
     }
     if ((rc = ensure_shared(s, p, shared, false))) return rc;
@@ -450,6 +452,7 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     bc.a = program_args(s, p, b->lds_budget);
     bc.a.census = nullptr;
     bc.a.shared = shared;
+    bc.a.gshift = gshift;
     bc.a.done = shared == kSharedVerify ? p->d_done : nullptr;
     bc.seed = (uint64_t)s->seed;
     bc.mseq0 = s->meas_seq;

@@ -108,7 +108,7 @@ struct ProgramArgs {
   uint32_t shared;
   uint32_t *done;
   uint32_t masked;   // the program has noise or flagged ops
-  uint32_t gshift;   // log2 of the word groups per workgroup (launch_shared sets it)
+  uint32_t gshift;   // log2 of the word groups per workgroup (launch_shared sets it, a batch's host side its members')
   uint64_t *packed;  // shared_packed_bytes(n), or null: the X/Z words are written in the kernel
 };
 // (kSharedChecked: inside launch_shared, done[] already tells which groups run)
@@ -161,8 +161,9 @@ constexpr uint32_t kSharedThreads = 768;
 constexpr uint32_t kSharedMaxQubits = 2048;
 constexpr uint32_t kSharedMaxGroups = 4;
 bool shared_fits(uint32_t n);
-// Dynamic LDS of one word group per workgroup (as batches run).
-size_t shared_lds_bytes(uint32_t n, bool masked);
+// Dynamic LDS of 1 << gshift word groups per workgroup, and a batch member's gshift.
+size_t shared_lds_bytes(uint32_t n, bool masked, uint32_t gshift);
+uint32_t shared_batch_gshift(uint32_t n, uint64_t W, bool masked, uint64_t groups, uint32_t cus);
 // Whether the run checks the tableau and writes the X/Z words in launches of
 // their own; it then needs ProgramArgs::packed.
 bool shared_split(uint32_t n, uint64_t W, bool masked);
