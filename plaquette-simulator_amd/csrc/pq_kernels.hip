@@ -2104,13 +2104,41 @@ __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w)
       } else if (kind == kFrameRandom) {
         // MeasureRandom (MeasurementFunctors.hpp:225-265) with pivot p: the
         // rowsum rows, then Rv[p], Rv[n+p] = coin ^ E.x[q] and the record.
+        if (rfl(sbuf[pos + 6]) > 64) {
+          // many rows (random circuits on many qubits): every thread takes some,
+          // the last wave draws the coin meanwhile
+          const uint32_t p = h1, ne = rfl(sbuf[pos + 6]);
+          const uint64_t Rs = Rl[n + p];
+          const uint32_t *ents = sbuf + pos + 8;
+          for (uint32_t e = tid; e < ne; e += kFrameThreads) Rl[ents[e]] ^= Rs;
+          uint64_t coin = 0;
+          if (wv == kFrameWaves - 1) {
+            const uint64_t key = stream_key(seed, 2 * (mseq0 + rfl(sbuf[pos + 3])));
+            const uint32_t u = (uint32_t)(draw_keyed(key, 64 * w + lane) >> 40);
+            coin = __ballot(u < rfl(sbuf[pos + 4]));
+          }
+          __syncthreads();  // all have read Rv[n+p]
+          if (tid == kFrameThreads - 64) {
+            const uint32_t slot = sbuf[pos + 2], ridx = sbuf[pos + 5];
+            Rl[p] = Rs;
+            Rl[n + p] = coin ^ dyn[sbuf[pos + 7]];
+            a.recs[(2ull * slot) * a.W + w] = coin;
+            a.recs[(2ull * slot + 1) * a.W + w] = 0ull;
+            if (ridx != kNone) dyn[a.lds_rec + ridx] = coin;
+          }
+          pos += 8 + ne;
+          __syncthreads();
+          continue;
+        }
         // A run of them (up to 64): the waves draw the coins in turn, then
         // wave 0 takes the measurements one after the other.  They are short
-        // (about 4 rows each) and each reads what the one before wrote: within
-        // a wave LDS order is enough, so a run costs two barriers, and its
-        // chain neither waits for a draw nor for the next header (d=9, 16384
-        // shots, with the determined ones after their run: 80 + 20 steps for
-        // 80 + 82, k_frame 148 -> 108 us; d=17, 32768 shots: 678 -> 500 us).
+        // (about 4 rows each in code circuits) and each reads what the one before
+        // wrote: within a wave LDS order is enough, so a run costs two barriers,
+        // and its chain neither waits for a draw nor for the next header (d=9,
+        // 16384 shots, with the determined ones after their run: 80 + 20 steps
+        // for 80 + 82, k_frame 148 -> 108 us; d=17, 32768 shots: 678 -> 500 us).
+        // Longer ones than a wave: as above (n=1024, 4096 shots, 100000 ops, about
+        // 400 rows each: 5.06 ms a pass, 7.09 by one wave).
         uint32_t m = 0, at = pos;
         for (;;) {
           if ((m & (kFrameWaves - 1)) == wv) {
@@ -2121,7 +2149,7 @@ __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w)
           }
           at += 8 + rfl(sbuf[at + 6]);
           ++m;
-          if (m == 64 || at >= cw || rfl(sbuf[at]) != kFrameRandom) break;
+          if (m == 64 || at >= cw || rfl(sbuf[at]) != kFrameRandom || rfl(sbuf[at + 6]) > 64) break;
         }
         __syncthreads();
         if (wv == 0) {
@@ -2133,7 +2161,7 @@ __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w)
             const uint32_t ridx = __builtin_amdgcn_readlane(hd, 5);
             const uint32_t ne = __builtin_amdgcn_readlane(hd, 6);
             const uint32_t exq = __builtin_amdgcn_readlane(hd, 7);
-            const uint32_t row = ent, here = pos;
+            const uint32_t row = ent;
             pos += 8 + ne;
             ++i;
             if (i < m) {
@@ -2142,7 +2170,6 @@ __device__ __forceinline__ void frame_word_group(const FrameArgs &a, uint64_t w)
             }
             const uint64_t Rs = Rl[n + p], ex = dyn[exq];
             if (lane < ne) Rl[row] ^= Rs;
-            for (uint32_t e = 64 + lane; e < ne; e += 64) Rl[sbuf[here + 8 + e]] ^= Rs;
             const uint64_t coin = read_lane64(coins, i - 1);
             if (lane == 0) {
               Rl[p] = Rs;
