@@ -126,6 +126,20 @@ def _gate_columns(code, a, b, n):
     return set(), set()
 
 
+def shared_minimum_bytes(ops, n, W):
+    """Least HBM bytes of a persistent run from |0...0> whose X/Z all shots share.
+
+    Nothing of the tableau has to be read; its words and each record's two are
+    written once, and a word group's noise masks (16 B per noise op) are read."""
+    R = 2 * n + 1
+    codes = ops[:, 0]
+    return 8 * W * (R * R + 2 * int((codes == 14).sum()) + 2 * int((codes == 10).sum()))
+
+
+SHARED_MODEL = ("X/Z shared by all shots, simulated as bits: the tableau's words and the records "
+                "written once, the noise masks read once")
+
+
 def fused_minimum_bytes(ops, n, W, census):
     """Least HBM bytes one run of `ops` can move in the fused persistent form.
 
@@ -263,6 +277,7 @@ def bench_mixed(args):
     # sequential baseline with census (algorithmic bytes) then without
     abytes = 0
     fbytes = 0
+    sbytes = 0
     for w, st, pr in zip(ws, states, progs):
         pr.set_census(True)
         st.reset_clifford_state()
@@ -272,6 +287,7 @@ def bench_mixed(args):
         words = (w.batch_size + 63) // 64
         abytes += algorithmic_bytes(w.ops, w.num_qubits, words, c)["total"]
         fbytes += fused_minimum_bytes(w.ops, w.num_qubits, words, c)["total"]
+        sbytes += shared_minimum_bytes(w.ops, w.num_qubits, words)
     for st in states:
         st.synchronize()
     progress("mixed: census done")
@@ -352,14 +368,12 @@ def bench_mixed(args):
                    "tableau_bytes": sum(((w.batch_size + 63) // 64) * (2 * w.num_qubits + 1) ** 2 * 8
                                         for w in ws)},
         "batch_kernel_ms": kernel_ms,
-        "roofline": {"bound": "hbm", "achieved": fbytes / (kernel_ms / 1e3) / 1e9,
+        "roofline": {"bound": "hbm", "achieved": sbytes / (kernel_ms / 1e3) / 1e9,
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": fbytes / (kernel_ms / 1e3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "k_batch", "kernel_ms": kernel_ms,
-                     "model": "fused minimum: each gate segment reads every column it "
-                              "uses and writes every column it changes once; "
-                              "measurements by census",
-                     "algorithmic_bytes": fbytes,
+                     "frac": sbytes / (kernel_ms / 1e3) / 1e9 / HBM_PEAK_GBS, "traffic": None,
+                     "kernel": "k_batch_shared", "kernel_ms": kernel_ms,
+                     "model": SHARED_MODEL, "algorithmic_bytes": sbytes,
+                     "fused_minimum_bytes": fbytes,
                      "per_op_model": {"bytes": abytes,
                                       "achieved": abytes / (kernel_ms / 1e3) / 1e9,
                                       "frac": abytes / (kernel_ms / 1e3) / 1e9 / HBM_PEAK_GBS}},
@@ -609,7 +623,8 @@ def bench_random_n1024(args):
     prog = ps.Program(st, w.ops)
     # workgroups per word group (0: chosen for the device; 64 word groups
     # cannot fill 256 compute units one workgroup each)
-    prog.set_slices(args.slices)
+    if args.slices:  # asking for a slice count keeps the per-shot kernel
+        prog.set_slices(args.slices)
     prog.set_census(True)
     st.reset_clifford_state()
     prog.run(st, "persistent")
@@ -633,7 +648,8 @@ def bench_random_n1024(args):
     kms, launches = prog.kernel_ms()
     kernel_ms = kms / max(1, launches)
     ms_step = 1e3 * wall / steps
-    achieved = fbytes["total"] / (kernel_ms / 1e3) / 1e9
+    sbytes = shared_minimum_bytes(w.ops, n, words)
+    achieved = sbytes / (kernel_ms / 1e3) / 1e9
     per_op_gbs = abytes["total"] / (kernel_ms / 1e3) / 1e9
     progress(f"n1024: persistent {ms_step:.1f} ms/step")
     # frame form (no flagged ops here, so X/Z are the same in every shot)
@@ -672,12 +688,9 @@ def bench_random_n1024(args):
                    "seed": w.seed, "word_groups": words, "slices": slices},
         "meas_shots_per_s": w.measurements * B / (ms_step / 1e3),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": None, "kernel": "k_program",
-                     "kernel_ms": kernel_ms,
-                     "model": "fused minimum: each gate segment reads every column it "
-                              "uses and writes every column it changes once; "
-                              "measurements by census",
-                     "algorithmic_bytes": fbytes["total"],
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": None,
+                     "kernel": "k_program_shared", "kernel_ms": kernel_ms,
+                     "model": SHARED_MODEL, "algorithmic_bytes": sbytes,
                      "per_op_model": {"bytes": abytes["total"], "achieved": per_op_gbs,
                                       "frac": per_op_gbs / HBM_PEAK_GBS}},
         "algorithmic_bytes": abytes,
@@ -685,19 +698,6 @@ def bench_random_n1024(args):
         "census": census,
         "frame_form": frame,
     }
-    # measured HBM bytes of one k_program launch of this workload (rocprofv3
-    # request counters by size, one workgroup per word group)
-    traffic_file = os.path.join(ROOT, "profiles", "k_program_random_n1024_traffic.json")
-    if os.path.exists(traffic_file):
-        tr = json.load(open(traffic_file))
-        rf = out["roofline"]
-        rf["traffic"] = tr.get("bytes_per_launch")
-        rf["traffic_source"] = ("profiles/k_program_random_n1024_traffic.json: " +
-                                tr.get("method", "rocprofv3 counters"))
-        if tr.get("bytes_per_launch"):
-            gbs = tr["bytes_per_launch"] / (kernel_ms / 1e3) / 1e9
-            rf["traffic_gbs"] = gbs
-            rf["traffic_frac"] = gbs / HBM_PEAK_GBS
     if not args.no_cpu:
         out["cpu_baseline"] = cpu_baseline_prefix(w, args.cpu_seconds)
     print(json.dumps(out))
@@ -873,7 +873,8 @@ def main():
     gate_shots = w.gates * B
     value = gate_shots / (ms_step / 1e3)
     fbytes = fused_minimum_bytes(w.ops, n, words, census)
-    achieved = fbytes["total"] / (kernel_ms / 1e3) / 1e9
+    sbytes = shared_minimum_bytes(w.ops, n, words)
+    achieved = sbytes / (kernel_ms / 1e3) / 1e9
     per_op_gbs = abytes["total"] / (kernel_ms / 1e3) / 1e9
     out = {
         "metric": METRIC,
@@ -894,17 +895,14 @@ def main():
                    "form": "persistent"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "k_program", "kernel_ms": kernel_ms,
-                     "model": "fused minimum: each gate segment reads every column it "
-                              "uses and writes every column it changes once; "
-                              "measurements by census",
-                     "algorithmic_bytes": fbytes["total"],
+                     "kernel": "k_program_shared", "kernel_ms": kernel_ms,
+                     "model": SHARED_MODEL, "algorithmic_bytes": sbytes,
                      # the per-op, unfused count (every op's columns from HBM),
                      # labelled apart: a fused kernel moves far less than this
                      "per_op_model": {"bytes": abytes["total"], "achieved": per_op_gbs,
                                       "frac": per_op_gbs / HBM_PEAK_GBS}},
         "meas_shots_per_s": w.measurements * B / (ms_step / 1e3),
-        "hbm_frac_step": fbytes["total"] / (ms_step / 1e3) / (HBM_PEAK_GBS * 1e9),
+        "hbm_frac_step": sbytes / (ms_step / 1e3) / (HBM_PEAK_GBS * 1e9),
         "fused_minimum_bytes": fbytes,
         "graph_ms_per_step": graph_ms,
         "graph_gate_shots_per_s": gate_shots / (graph_ms / 1e3),
