@@ -1007,8 +1007,11 @@ int build_frame_plan(pq_program_s *p, uint64_t groups) {
   // per wave.  Each group runs a chain of short dependent steps, so several
   // groups per CU hide each other's latencies: the largest staging that
   // keeps as many groups per CU as the launch has (up to kFrameGroupsPerCu)
-  // is taken; a launch of at most one group per CU gets the largest staging,
-  // double-buffered.
+  // is taken, but never one that takes a CU's LDS for a single group where two
+  // fit: another state's groups run beside this launch's (d=9, 16384 shots, one
+  // group per CU: 110 -> 80 us a pass with several states in flight and 176 ->
+  // 177 us alone, against 107 KB of double buffers; room for three instead: 78
+  // and 183 us, and d=17, 32768 shots 851 -> 868 us).
   const uint64_t nb_cap = (2 * p->nnoise + 63) / 64 * 64;
   auto lds_of = [&](const Staging &o) {
     const uint64_t nb = std::min<uint64_t>(o.nb, nb_cap), sb = std::max(o.sb, need);
@@ -1018,7 +1021,7 @@ int build_frame_plan(pq_program_s *p, uint64_t groups) {
     const uint64_t l = lds_of(o);
     return l <= kFrameLdsMax ? kFrameLdsMax / l : 0;
   };
-  const uint64_t want = std::max<uint64_t>(1, groups / kCus + (groups % kCus != 0));
+  const uint64_t want = std::max<uint64_t>(2, groups / kCus + (groups % kCus != 0));
   const uint64_t target = std::min<uint64_t>(std::min<uint64_t>(kFrameGroupsPerCu, want),
                                              per_cu(kStaging[0]));
   if (!target)
