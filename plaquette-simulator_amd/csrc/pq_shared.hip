@@ -761,7 +761,10 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
     // A lane takes its row's bit of a column as a mask, once for all groups:
     // VALU-bound.  Column words and frames read from lanes as scalars instead
     // stalled on every one: 449 qubits, one group 106 -> 50 us of the run's 1180;
-    // 161 qubits, four groups 56 -> 28 us of 337.
+    // 161 qubits, four groups 56 -> 28 us of 337.  Two columns at a time: four
+    // took the kernel from 128 to 159 VGPRs, at which no other kernel's wave fits
+    // beside it on a CU (d=9, 16384 shots, several states in flight: 266 us a
+    // pass with four, 210 with two, 255 with one).
     const uint32_t parts = max(1u, 2 * nw / KW), per = (n + parts - 1) / parts;
     for (uint32_t task = wv; task < KW * parts; task += nw) {
       const uint32_t kk = task / parts, pt = task - kk * parts;
@@ -772,7 +775,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
       auto run = [&](auto groups) {
         constexpr uint32_t kG = decltype(groups)::value;
         uint64_t acc[kG] = {};
-#pragma unroll 4
+#pragma unroll 2
         for (uint32_t j = ja; j < jb; ++j) {
           const uint64_t mx = (uint64_t)(int64_t)((Px[2 * j * KW] << sh31) >> 31);
           const uint64_t mz = (uint64_t)(int64_t)((Pz[2 * j * KW] << sh31) >> 31);
