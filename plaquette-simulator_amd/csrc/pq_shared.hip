@@ -764,7 +764,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
     // 161 qubits, four groups 56 -> 28 us of 337.  Two columns at a time: four
     // took the kernel from 128 to 159 VGPRs, at which no other kernel's wave fits
     // beside it on a CU (d=9, 16384 shots, several states in flight: 266 us a
-    // pass with four, 210 with two, 255 with one).
+    // pass with four, 200-240 with two, 255 with one).
     const uint32_t parts = max(1u, 2 * nw / KW), per = (n + parts - 1) / parts;
     for (uint32_t task = wv; task < KW * parts; task += nw) {
       const uint32_t kk = task / parts, pt = task - kk * parts;
