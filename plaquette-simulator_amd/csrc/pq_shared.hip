@@ -740,6 +740,9 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
       b = mend;
       if (b < wn) cw = rfl(sh.ops[b].cw);
     }
+    // every wave has read op b (which the window may end at, behind a
+    // measurement): the next window's ops and masks take their place
+    __syncthreads();
     base += b;
   }
   if (on && rp) lds_xor(rc + my_k, rp);

@@ -244,3 +244,36 @@ def test_batch_members_in_both_kernels(ps, form):
         for (st, _), (rs, rp) in zip(got, ref):
             rp.run(rs, "persistent")
             assert st.compare(rs) == (0, 0)
+
+
+@pytest.mark.parametrize("n,B,width,runs", [
+    (100, 130, 100, 30),   # 130 ops a round: a layer behind measurements spans ops 390..490
+    (161, 64, 161, 17), (33, 70, 33, 31), (64, 16385, 64, 20),
+    # columns in the tableau
+    (500, 70, 300, 13), (520, 323, 200, 9)])
+def test_windows_that_end_between_measurements_and_a_layer(ps, n, B, width, runs):
+    """Ops are staged 448 at a time, and a layer that does not fit opens the next
+    window.  Rounds of one layer and one run of measurements, so that windows end
+    right behind measurements, with the next layer's first op read already."""
+    from plaquette_simulator import workloads as W
+    rng = np.random.default_rng(n)
+    b = W.OpList()
+    for r in range(9):
+        for q in range(width):
+            code = int(rng.choice([W.OP_H, W.OP_S, W.OP_X, W.OP_H]))
+            b.gate(code, q)
+            if rng.random() < 0.05:
+                b.noise(q, 0.1, 0.1, 0.1)
+        for _ in range(runs):
+            b.measure(int(rng.integers(0, n)))
+        for q in range(r % 2, n - 1, 2):
+            b.cx(q, q + 1)
+        for _ in range(runs):
+            b.measure(int(rng.integers(0, n)))
+    ops = b.array()
+    say(f"[case] windows n={n} B={B} ops={len(ops)}")
+    orc = O.OracleState(n, B, 23)
+    orc.run_program(ops.astype(np.int32))
+    st = ps.CliffordState(n, B, 23, True)
+    ps.Program(st, ops).run(st, "persistent")
+    check(st, orc)
