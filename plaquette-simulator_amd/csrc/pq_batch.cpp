@@ -387,6 +387,7 @@ static int run_frame_batch(pq_batch b) {
       // or now if the raw tableau pointer was handed out
       s->xz_pending = false;
       s->xz_plan = b->members[c].second->frame;
+      s->xz_unchecked = false;
       if (s->exposed) {
         int rc = materialize_tableau(s);
         if (rc) return rc;
@@ -438,7 +439,7 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
       gshift = shared_batch_gshift((uint32_t)s->n, s->W, p->masked, b->nitems,
                                    (uint32_t)cu_count());
       lds = std::max(lds, shared_lds_bytes((uint32_t)s->n, p->masked, gshift));
-      if (s->xz_identity) shared = s->exposed ? kSharedVerify : kSharedKnown;
+      if (s->xz_identity) shared = xz_certain(s) ? kSharedKnown : kSharedVerify;
     }
     if ((rc = ensure_shared(s, p, shared, false))) return rc;
     if (shared == kSharedKnown) {

@@ -277,6 +277,7 @@ extern "C" int pq_reset(pq_state s) {
   }
   s->xz_plan.reset();
   s->xz_identity = true;
+  s->xz_unchecked = false;
   return PQ_OK;
 }
 
@@ -300,6 +301,7 @@ extern "C" int pq_copy_from(pq_state dst, pq_state src) {
   ARGCHK(dst->n == src->n && dst->B == src->B, "DeviceToDevice needs equal n and B");
   if (!dst->tab || dst == src) return PQ_OK;
   dst->xz_identity = src->xz_identity;
+  dst->xz_unchecked = src->exposed || src->xz_unchecked;
   // Kokkos::deep_copy has finished before either state changes again
   // (CliffordState.hpp:268-274).  Here the copy runs on the source's stream
   // after the destination's queued work, and the destination's stream waits

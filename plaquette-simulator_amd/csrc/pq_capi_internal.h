@@ -48,6 +48,10 @@ struct pq_state_s {
   bool xz_pending = false;
   // the raw tableau pointer was handed out: resets write X/Z at once
   bool exposed = false;
+  // X/Z were copied from a state whose holder of the raw pointer may have
+  // changed them: xz_identity is what the calls say, not what the words are,
+  // until a reset or a frame run determines them
+  bool xz_unchecked = false;
   // a frame run left X/Z unwritten: every group's X/Z is this plan's shared
   // X/Z, written by materialize_tableau (never set with xz_pending)
   std::shared_ptr<FramePlan> xz_plan;
@@ -62,6 +66,11 @@ struct pq_state_s {
   std::vector<char> rec_valid;
   ~pq_state_s();
 };
+
+// Whether X/Z are known to be |0...0> without a look at the words.
+inline bool xz_certain(const pq_state_s *s) {
+  return s->xz_identity && !s->exposed && !s->xz_unchecked;
+}
 
 int pq_set_error(int code, const char *msg);
 

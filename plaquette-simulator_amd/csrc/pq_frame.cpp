@@ -1249,6 +1249,7 @@ int run_frame(pq_state s, pq_program_s *p) {
     // tableau pointer was handed out
     s->xz_pending = false;
     s->xz_plan = p->frame;
+    s->xz_unchecked = false;
     if (s->exposed) {
       int rc2 = materialize_tableau(s);
       if (rc2) return rc2;

@@ -822,12 +822,12 @@ static int program_run(pq_state s, pq_program p, int form) {
   if (form == PQ_RUN_FRAME) return run_frame(s, p);
   // X/Z are the |0...0> tableau: the shared-X/Z kernel, which reads no X/Z
   // (they may be pending) and writes them all.  The holder of a raw pointer
-  // may have changed them, so an exposed state's word groups are checked, and
-  // so are a captured run's at every replay.
+  // may have changed them, so the word groups of an exposed state, or of a copy
+  // of one, are checked, and so are a captured run's at every replay.
   uint32_t shared = 0;
   if ((form == PQ_RUN_PERSISTENT && s->xz_identity) || form == PQ_RUN_GRAPH)
     if (shared_allowed(s, p))
-      shared = form == PQ_RUN_GRAPH || s->exposed ? kSharedVerify : kSharedKnown;
+      shared = form == PQ_RUN_GRAPH || !xz_certain(s) ? kSharedVerify : kSharedKnown;
   if ((rc = ensure_shared(s, p, shared, shared_split((uint32_t)s->n, s->W, p->masked)))) return rc;
   if (shared == kSharedKnown) {
     s->xz_pending = false;

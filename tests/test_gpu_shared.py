@@ -277,3 +277,86 @@ def test_windows_that_end_between_measurements_and_a_layer(ps, n, B, width, runs
     st = ps.CliffordState(n, B, 23, True)
     ps.Program(st, ops).run(st, "persistent")
     check(st, orc)
+
+
+_COPIES = """
+import sys
+import torch  # first: its HIP runtime must be the one the process loads
+assert torch.cuda.is_available()
+sys.path[:0] = sys.argv[1:]
+import plaquette_simulator as ps
+from test_gpu_shared import mixed_ops
+
+def edited(n, B):
+    st = ps.CliffordState(n, B, 21, True)
+    planes = torch.from_dlpack(st.planes_dlpack()).view(torch.int64)
+    st.reset_clifford_state()
+    st.synchronize()
+    planes[0, [0, n]] = planes[0, [n, 0]]  # H on qubit 0 of the first 64 shots
+    torch.cuda.synchronize()
+    return st, planes
+
+def copy_of(st, how, n, B):
+    if how == "copy":
+        return st.copy()
+    if how == "copy of a copy":
+        return st.copy().copy()
+    dst = ps.CliffordState(n, B, 21, True)
+    if how == "into a reset state":
+        dst.reset_clifford_state()
+    dst.device_to_device(st)
+    return dst
+
+for n, B in ((70, 200), (70, 14000), (500, 300)):
+    ops = mixed_ops(n, 600, 4, 0.1)
+    for how in ("copy", "copy of a copy", "into a state", "into a reset state"):
+        for form in ("persistent", "graph", "batch"):
+            st, planes = edited(n, B)
+            got, ref = copy_of(st, how, n, B), copy_of(st, how, n, B)
+            assert got.compare(st) == (0, 0)
+            pg, pr = ps.Program(got, ops), ps.Program(ref, ops)
+            pr.set_slices(1)  # keeps the per-shot kernel, which reads the words
+            if form == "batch":
+                batch = ps.Batch()
+                batch.add(got, pg)
+                batch.run("persistent")
+                batch.wait()
+            else:
+                pg.run(got, form)
+            pr.run(ref, "persistent")
+            got.synchronize()
+            ref.synchronize()
+            assert got.compare(ref) == (0, 0), (n, B, how, form)
+            # a reset determines the words again
+            got.reset_clifford_state()
+            ref.reset_clifford_state()
+            pg.run(got, "persistent")
+            pr.run(ref, "persistent")
+            assert got.compare(ref) == (0, 0), (n, B, how, form, "reset")
+            del got, ref, pg, pr, planes, st
+    # a copy of an exposed |0...0> state still takes the frame form
+    st = ps.CliffordState(n, B, 21, True)
+    planes = torch.from_dlpack(st.planes_dlpack())
+    a, b = st.copy(), st.copy()
+    pa, pb = ps.Program(a, ops), ps.Program(b, ops)
+    pa.run(a, "frame")
+    pb.run(b, "persistent")
+    assert a.compare(b) == (0, 0), (n, B, "frame")
+print("copies ok")
+"""
+
+
+def test_copies_of_a_state_changed_through_the_raw_pointer(ps):
+    """A copy holds the words that the raw pointer's holder wrote, whatever the
+    calls on its source say: it runs from those words.  (In a child process that
+    imports torch before the engine.)"""
+    pytest.importorskip("torch")
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    say("[case] copies of a state changed through the raw pointer (child process)")
+    r = subprocess.run([sys.executable, "-c", _COPIES,
+                        os.path.join(root, "plaquette-simulator_amd"),
+                        os.path.join(root, "tests"), os.path.join(root, "oracle")],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "copies ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
