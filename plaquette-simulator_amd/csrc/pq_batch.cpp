@@ -420,6 +420,13 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     int rc = build(b);
     if (rc) return rc;
   }
+  // What can refuse the run comes first, and a member's state changes only once
+  // the launch is enqueued: a member whose X/Z wait to be written (a reset, a
+  // frame run) keeps them waiting if a later one is refused.
+  for (auto &m : b->members) {
+    int rc = check_records(m.first, m.second);
+    if (rc) return rc;
+  }
   // the pinned descriptor buffer is reused: the previous upload must be done
   HIPCHK(hipEventSynchronize(b->ev_upload));
   const uint32_t nc = (uint32_t)b->members.size();
@@ -442,11 +449,8 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
       if (s->xz_identity) shared = xz_certain(s) ? kSharedKnown : kSharedVerify;
     }
     if ((rc = ensure_shared(s, p, shared, false))) return rc;
-    if (shared == kSharedKnown) {
-      s->xz_pending = false;
-      s->xz_plan.reset();
-    }
-    if ((rc = materialize_tableau(s))) return rc;
+    // (the shared-X/Z kernel reads no X/Z of a known |0...0> and writes them all)
+    if (shared != kSharedKnown && (rc = materialize_tableau(s))) return rc;
     HIPCHK(hipStreamSynchronize(s->stream));  // the member's own queued work first
     if (p->done_ev) HIPCHK(hipEventSynchronize(p->done_ev));  // the program's last run
     BatchCircuit &bc = b->h_circ[c];
@@ -460,10 +464,6 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
     bc.nseq0 = s->noise_seq;
     bc.noise = p->d_noise;
     bc.nnoise = (uint32_t)p->nnoise;
-
-    s->meas_seq += p->nmeas;
-    s->xz_identity = false;
-    s->noise_seq += p->nnoise;
     gens[c] = s->arena_gen;
   }
   if (shared_lds != b->shared_lds) b->drop_graph();
@@ -505,6 +505,15 @@ extern "C" int pq_batch_run(pq_batch b, int form) {
       b->graph_gens = gens;
     }
     HIPCHK(hipGraphLaunch(b->gexec, b->stream));
+  }
+  for (uint32_t c = 0; c < nc; ++c) {
+    pq_state s = b->members[c].first;
+    pq_program p = b->members[c].second;
+    s->meas_seq += p->nmeas;
+    s->noise_seq += p->nnoise;
+    s->xz_identity = false;
+    s->xz_pending = false;
+    s->xz_plan.reset();
   }
   if (b->timed) HIPCHK(hipEventRecord(b->ev_b, b->stream));
   return PQ_OK;

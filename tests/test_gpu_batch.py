@@ -209,3 +209,51 @@ def test_batch_frame_refusals(ps):
     with pytest.raises(RuntimeError, match="reset"):
         batch2.run("frame")
     assert all(st.num_records == 0 for st in st2)
+
+
+@pytest.mark.parametrize("form", ["persistent", "graph"])
+@pytest.mark.parametrize("before", ["reset", "frame"])
+def test_batch_refused_run_leaves_members_unchanged(ps, form, before):
+    """A member whose program names a record that its state does not have refuses
+    the run; members before it, whose X/Z a reset or a frame run left to be
+    written, still hold |0...0>, with their sequence numbers and records."""
+    from plaquette_simulator import workloads as W
+    n, B, seed, ops = members()[1]
+    say(f"[case] refused batch form={form} after {before}")
+    flips = W.OpList()  # leaves X/Z as they are
+    for q in range(n):
+        flips.gate(W.OP_X, q)
+        flips.measure(q)
+    bad = W.OpList()
+    for q in range(4):
+        bad.gate(W.OP_H, q)
+        bad.measure(q, 0.5, 3)  # the state has no record 3
+    got, ref = (ps.CliffordState(n, B, seed, True) for _ in range(2))
+    other = ps.CliffordState(4, 64, 1, True)
+    progs = []
+    for st in (got, ref):
+        prog = ps.Program(st, ops)
+        prog.run(st, "persistent")  # X/Z of a circuit
+        st.reset_clifford_state()
+        if before == "frame":
+            ps.Program(st, flips.array()).run(st, "frame")
+        progs.append(prog)
+    batch = ps.Batch()
+    batch.add(got, progs[0])
+    batch.add(other, ps.Program(other, bad.array()))
+    nrec = got.num_records
+    with pytest.raises(RuntimeError, match="record"):
+        batch.run(form)
+    assert got.num_records == nrec and other.num_records == 0
+    assert np.array_equal(got.read_planes(), ref.read_planes())
+    # and again with X/Z still waiting, then a run of the member by itself
+    for st in (got, ref):
+        st.reset_clifford_state()
+    with pytest.raises(RuntimeError, match="record"):
+        batch.run(form)
+    progs[0].run(got, "frame")
+    progs[1].run(ref, "frame")
+    got.sync_records()
+    ref.sync_records()
+    assert got.compare(ref) == (0, 0)
+    same(snapshot(ref), snapshot(got))
