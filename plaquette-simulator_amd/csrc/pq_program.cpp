@@ -829,10 +829,6 @@ static int program_run(pq_state s, pq_program p, int form) {
     if (shared_allowed(s, p))
       shared = form == PQ_RUN_GRAPH || !xz_certain(s) ? kSharedVerify : kSharedKnown;
   if ((rc = ensure_shared(s, p, shared, shared_split((uint32_t)s->n, s->W, p->masked)))) return rc;
-  if (shared == kSharedKnown) {
-    s->xz_pending = false;
-    s->xz_plan.reset();
-  }
   // X/Z still the identity after a reset, and the whole tableau is held in LDS
   // or the program opens with a row-tiled gate segment over every qubit: the
   // persistent kernel writes the words itself, so the identity fill is not needed
@@ -841,10 +837,9 @@ static int program_run(pq_state s, pq_program p, int form) {
                       (!p->segs.empty() && p->segs[0].kind == 0 && p->segs[0].nq == s->n &&
                        program_tile_rows(program_args(s, p, kProgramLdsBytes).lds_words,
                                          (uint32_t)s->n) > 0));
-  if (fresh)
-    s->xz_pending = false;  // written by the run
-  else if ((rc = materialize_tableau(s)))
-    return rc;
+  // X/Z that the run writes wait until it is enqueued: it may still be refused
+  const bool writes_xz = fresh || shared == kSharedKnown;
+  if (!writes_xz && (rc = materialize_tableau(s))) return rc;
   s->xz_identity = false;
   if (form == PQ_RUN_PLAIN) return run_plain(s, p);
   if (s->n > measure_max_qubits())
@@ -853,7 +848,14 @@ static int program_run(pq_state s, pq_program p, int form) {
                            s->noise_seq));
   s->meas_seq += p->nmeas;
   s->noise_seq += p->nnoise;
-  if (form == PQ_RUN_PERSISTENT) return enqueue_persistent(s, p, p->timing_on, true, fresh, shared);
+  if (form == PQ_RUN_PERSISTENT) {
+    rc = enqueue_persistent(s, p, p->timing_on, true, fresh, shared);
+    if (rc == PQ_OK && writes_xz) {
+      s->xz_pending = false;
+      s->xz_plan.reset();
+    }
+    return rc;
+  }
   if (form != PQ_RUN_GRAPH) return pq_set_error(PQ_ERR_ARG, "unknown run form");
   if (p->gexec && (p->graph_state != s || p->graph_arena_gen != s->arena_gen)) {
     (void)hipGraphExecDestroy(p->gexec);

@@ -179,3 +179,27 @@ def test_barrier_give_up_is_reported_and_the_run_ends(ps):
     a, used, failed = run_sliced(ps, n, B, seed, ops, 2)
     assert (used, failed) == (2, 0)
     check_against_oracle(a, n, B, seed, ops)
+
+
+def test_refused_run_leaves_a_reset_state_at_zero(ps):
+    # a reset leaves X/Z to be written by the run, here by its first gate
+    # segment; a run refused for its slice count writes nothing
+    from plaquette_simulator import workloads as W
+    n, B = 64, 64 * 64
+    b = W.OpList()
+    for q in range(n):
+        for _ in range(3):
+            b.h(q)
+            b.s(q)
+    b.measure(0)
+    ops = b.array()
+    say(f"[case] refused slices on a reset state n{n} B{B}")
+    st = ps.CliffordState(n, B, 1, True)
+    zero = st.read_planes()
+    ps.Program(st, ops).run(st, "persistent")
+    st.reset_clifford_state()
+    prog = ps.Program(st, ops)
+    prog.set_slices(1000)
+    with pytest.raises(RuntimeError, match="slices"):
+        prog.run(st, "persistent")
+    assert np.array_equal(st.read_planes(), zero)
