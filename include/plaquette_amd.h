@@ -348,8 +348,11 @@ int pq_batch_wait(pq_batch b);
 int pq_batch_set_launch(pq_batch b, uint32_t threads, uint32_t blocks,
                         uint64_t lds_budget);
 /* Times candidate launch shapes on the batch and keeps the fastest, then the
- * word tile at that shape (cached per batch shape).  Members are reset to |0...0> afterwards with their
- * sequence numbers restored. */
+ * word tile at that shape (cached per batch shape).  The shapes are timed on
+ * runs of the per-shot kernel, the only one that they are for, the word tiles
+ * on runs from |0...0>; best_ms is the time of such a run (-1: from the
+ * cache).  Members are reset to |0...0> afterwards with their sequence numbers
+ * restored. */
 int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads, uint64_t *lds_budget,
                       float *best_ms);
 int pq_batch_info(pq_batch b, uint64_t *members, uint64_t *items, uint32_t *threads,

@@ -571,10 +571,13 @@ extern "C" int pq_batch_info(pq_batch b, uint64_t *members, uint64_t *items,
 // setting how many workgroups share a CU and how many waves run fully
 // determined measurements in parallel) on the batch itself and keeps the
 // fastest, then the word tile (1, 2 or 4 word groups per work item) at that
-// shape.  Trial runs are real runs: afterwards every member is reset to
-// |0...0> and its coin/noise sequence numbers are restored.  Choices are
-// cached per batch shape (member qubit counts, word-group counts and program
-// sizes) for the life of the process.
+// shape.  The launch shape is k_batch_t's alone, so its trials run from the
+// states that the trial before left, which no member runs packed; the word
+// tile is every kernel's, so its trials run from |0...0>, where the tuner
+// leaves the members.  Trial runs are real runs: afterwards every member is
+// reset and its coin/noise sequence numbers are restored.  Choices are
+// cached per batch shape (member qubit counts, word-group counts, program
+// sizes and which members may run packed) for the life of the process.
 extern "C" int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads_out,
                                  uint64_t *lds_out, float *ms_out) {
   if (!b) return pq_set_error(PQ_ERR_ARG, "null batch");
@@ -591,6 +594,7 @@ extern "C" int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads_out,
     key.push_back(m.first->n);
     key.push_back(m.first->W);
     key.push_back(m.second->instrs.size());
+    key.push_back(shared_allowed(m.first, m.second) ? 1 : 0);
   }
   {
     std::lock_guard<std::mutex> g(mu);
@@ -613,10 +617,16 @@ extern "C" int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads_out,
   uint64_t bl = b->lds_budget;
   const bool was_timed = b->timed;
   b->timed = true;
-  // average HIP-event time of `reps` runs after one warm-up run
-  auto time_runs = [&](float *avg) -> int {
+  // average HIP-event time of `reps` runs after one warm-up run, each from
+  // |0...0> or from what the last one left
+  auto time_runs = [&](bool from_zero, float *avg) -> int {
     float tot = 0;
     for (int r = 0; r < std::max(1, reps) + 1; ++r) {
+      if (from_zero)
+        for (auto &m : b->members) {
+          int rc = pq_reset(m.first);
+          if (rc) return rc;
+        }
       int rc = pq_batch_run(b, PQ_RUN_PERSISTENT);
       if (rc) return rc;
       float ms = 0;
@@ -639,7 +649,7 @@ extern "C" int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads_out,
       rc = pq_batch_set_launch(b, t, 0, l);
       if (rc) return rc;
       float avg = 0;
-      if ((rc = time_runs(&avg))) return rc;
+      if ((rc = time_runs(false, &avg))) return rc;
       if (avg < best) {
         best = avg;
         bt = t;
@@ -649,10 +659,11 @@ extern "C" int pq_batch_autotune(pq_batch b, int reps, uint32_t *threads_out,
   }
   // then the word tile (word groups per work item) at the best shape
   if ((rc = pq_batch_set_launch(b, bt, 0, bl))) return rc;
-  for (uint32_t wt : {2u, 4u}) {
+  best = 1e30f;
+  for (uint32_t wt : {1u, 2u, 4u}) {
     if ((rc = pq_batch_set_word_tile(b, wt))) return rc;
     float avg = 0;
-    if ((rc = time_runs(&avg))) return rc;
+    if ((rc = time_runs(true, &avg))) return rc;
     if (avg < best) {
       best = avg;
       bw = wt;
