@@ -91,6 +91,17 @@ constexpr uint32_t kLayerLenMask = 0x7FFu;
 // once in a batch of fully determined measurements.
 constexpr uint32_t kMeasSuperseded = 1u;
 constexpr uint32_t kMeasLeftShift = 8;
+// Most ops of a batch, and instructions that a kernel stages at a time.  The
+// compiler cuts batches, runs and layer parts at every kStage instructions of
+// a segment; the kernels rely on it (a layer part runs whole).
+constexpr uint32_t kBatch = 8;
+constexpr uint32_t kStage = 448;
+// Run parameters, written on the device before each run (launch_set_params).
+struct ProgParams {
+  uint64_t seed;
+  uint64_t mseq0;  // measurement sequence number of the program's first M
+  uint64_t nseq0;  // noise sequence number of the program's first NOISE
+};
 
 // Segment of a compiled program: a run of gate batches or a run of
 // measurements.  Gate segments hold `count` instructions in batches.  A gate

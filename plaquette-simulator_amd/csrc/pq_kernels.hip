@@ -749,14 +749,6 @@ __global__ void k_set_params(uint64_t *p, uint64_t seed, uint64_t mseq0,
   }
 }
 
-struct ProgParams {
-  uint64_t seed;
-  uint64_t mseq0;  // measurement sequence number of the program's first M
-  uint64_t nseq0;  // noise sequence number of the program's first NOISE
-};
-
-constexpr int kBatch = 8;
-
 // The compiled program and the noise planes are read-only while k_program
 // runs; reading them through the constant address space lets uniform loads
 // become scalar (SMEM) loads, so a batch's column loads are not serialised
@@ -800,7 +792,6 @@ constexpr uint32_t kMeasWindow0 = 8;  // first window of a run
 // planes, flags) are staged in LDS by the whole workgroup in one round trip;
 // after that every batch costs exactly one global round trip (its column
 // loads), and the stores are fire-and-forget.
-constexpr uint32_t kStage = 448;
 constexpr uint32_t kStageWords = kStage * (sizeof(DInstr) / 8 + 4);
 // Row-tiled segments stage each op in one word (TileOp) beside its masks.
 constexpr uint32_t kTileStageWords = kStage * 5;

@@ -34,7 +34,6 @@ namespace {
 
 constexpr uint32_t kLocalThreads = 768;
 constexpr uint32_t kLocalWaves = kLocalThreads / 64;
-constexpr uint32_t kLocalStage = 448;  // staged ops at most
 constexpr uint32_t kLocalSteps = (kLocalMaxQubits + kLocalWaves - 1) / kLocalWaves;
 static_assert(kLocalSteps % 2 == 0, "steps run in pairs");
 
@@ -95,25 +94,27 @@ constexpr uint32_t kOpLenShift = 12, kOpLenMask = 0xFFFu;
 // Dynamic LDS words besides the staged ops (5 words each): the tableau, a row of
 // source words, the rows' masks and the low bits of their phase sums, and the
 // waves' pieces of the determined chain.
-__host__ __device__ inline uint32_t local_words(uint32_t n) {
+__host__ __device__ constexpr uint32_t local_words(uint32_t n) {
   const uint32_t R = 2 * n + 1;
   return R * R + R + 4 * n + kLocalWaves * 128;
 }
 constexpr uint32_t kLocalLdsBytes = 159 * 1024;
-__host__ __device__ inline uint32_t local_stage(uint32_t n) {
+__host__ __device__ constexpr uint32_t local_stage(uint32_t n) {
   const uint32_t room = (kLocalLdsBytes / 8 - local_words(n)) / 5;
-  return room < kLocalStage ? room : kLocalStage;
+  return room < kStage ? room : kStage;
 }
+// a layer, of at most a qubit's op each, runs whole
+static_assert(local_stage(kLocalMaxQubits) >= kLocalMaxQubits, "a layer fits the window");
 
 __global__ __launch_bounds__(kLocalThreads) void k_program_local(ProgramArgs a,
-                                                                 const uint64_t *__restrict__ pp) {
+                                                                 const ProgParams *__restrict__ pp) {
   extern __shared__ uint64_t dyn[];
   __shared__ uint64_t s_racc;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = rfl(tid >> 6);
   constexpr uint32_t NT = kLocalThreads, NW = kLocalWaves;
   const uint32_t n = a.n, R = a.R, stage = local_stage(n);
   const uint64_t W = a.W;
-  const uint64_t seed = pp[0], mseq0 = pp[1];
+  const uint64_t seed = pp->seed, mseq0 = pp->mseq0;
   uint64_t *const T = dyn;              // word (column c, row i) at c * R + i
   uint64_t *const rcol = T + 2 * n * R;
   uint64_t *const s_src = T + R * R;
@@ -464,7 +465,7 @@ hipError_t prepare_local() {
 hipError_t launch_local(hipStream_t s, const ProgramArgs &a, const void *params) {
   if (!a.nwords) return hipSuccess;
   hipLaunchKernelGGL(k_program_local, dim3((uint32_t)std::min<uint64_t>(a.nwords, 1u << 20)),
-                     dim3(kLocalThreads), local_lds_bytes(a.n), s, a, (const uint64_t *)params);
+                     dim3(kLocalThreads), local_lds_bytes(a.n), s, a, (const ProgParams *)params);
   return hipGetLastError();
 }
 

@@ -85,7 +85,7 @@ static void mark_runs(pq_program_s *p, const DSegment &sg) {
   uint32_t start = sg.begin;
   for (uint32_t k = sg.begin + 1; k <= end; ++k) {
     const bool brk = k == end || (p->instrs[k].pad & kLayerStart) ||
-                     (k - sg.begin) % kProgramStage == 0 ||
+                     (k - sg.begin) % kStage == 0 ||
                      p->instrs[k].code != p->instrs[k - 1].code;
     if (brk) {
       p->instrs[start].pad |= (k - start) << kRunShift;
@@ -94,7 +94,7 @@ static void mark_runs(pq_program_s *p, const DSegment &sg) {
   }
   start = sg.begin;
   for (uint32_t k = sg.begin + 1; k <= end; ++k)
-    if (k == end || (p->instrs[k].pad & kLayerStart) || (k - sg.begin) % kProgramStage == 0) {
+    if (k == end || (p->instrs[k].pad & kLayerStart) || (k - sg.begin) % kStage == 0) {
       p->instrs[start].pad |= (k - start) << kLayerLenShift;
       start = k;
     }
@@ -173,8 +173,8 @@ static void emit_gate_segment(pq_program_s *p, const std::vector<DInstr> &seg) {
     while (e < order.size() && layer[order[e]] == layer[order[k]]) ++e;
     for (uint32_t b = k; b < e;) {
       // batches never straddle a staging chunk of the kernel
-      const uint32_t pos = (uint32_t)(p->instrs.size() - sg.begin) % kProgramStage;
-      const uint32_t len = std::min<uint32_t>({kProgramBatch, e - b, kProgramStage - pos});
+      const uint32_t pos = (uint32_t)(p->instrs.size() - sg.begin) % kStage;
+      const uint32_t len = std::min<uint32_t>({kBatch, e - b, kStage - pos});
       for (uint32_t u = 0; u < len; ++u) {
         DInstr I = seg[order[b + u]];
         I.pad = (u == 0) ? (len | (b == k ? kLayerStart : 0u)) : 0u;

@@ -11,9 +11,7 @@
 #include "pq_common.h"
 #include "pq_frame.h"
 
-constexpr uint32_t kProgramBatch = 8;  // must equal kBatch in pq_kernels.hip
 constexpr uint32_t kProgramThreadsMax = 768;  // largest block of the persistent kernel builds
-constexpr uint32_t kProgramStage = 448;       // must equal kStage there
 // Gate segments with more qubits than a row tile of kWindowCutRows rows can
 // hold (in the default LDS budget) are cut into qubit windows, each small
 // enough for a tile of kWindowRows rows.

@@ -36,7 +36,6 @@ namespace {
 
 #define PQ_CONST __attribute__((address_space(4)))
 
-constexpr uint32_t kChunk = 448;       // staged ops; must equal kStage in pq_kernels.hip
 // wide states: columns a lane has in flight, in determined chains and in the
 // rowsums of random measurements (more spill registers)
 constexpr uint32_t kWideCols = 5, kRandCols = 6;
@@ -99,7 +98,7 @@ constexpr uint32_t kOpLenShift = 12, kOpLenMask = 0xFFFu;
 
 constexpr uint32_t kMaxRowWords = 2 * (kSharedMaxQubits / 64) + 2;
 struct SharedLds {
-  SharedOp ops[kChunk + 1];
+  SharedOp ops[kStage + 1];
   uint64_t rc[kMaxRowWords];  // sign bits, laid out like a column
   uint64_t sm[kMaxRowWords];  // row mask of the current random measurement
   uint64_t c0[kMaxRowWords];  // and the low bits of its rows' phase sums
@@ -118,7 +117,7 @@ constexpr uint64_t kSharedLdsBytes = 159 * 1024 - sizeof(SharedLds);  // dynamic
 // masks (programs with noise or flags), and the packed columns if they fit.
 // (Programs without masks keep only the measurements' two words there.)
 __host__ __device__ inline uint64_t mask_words(bool masked, uint32_t gs) {
-  return masked ? (4ull * kChunk) << gs : 2ull * kChunk;
+  return masked ? (4ull * kStage) << gs : 2ull * kStage;
 }
 __host__ __device__ inline uint64_t groups_words(uint32_t n, bool masked, uint32_t gs) {
   return ((4ull * n + 1) << gs) + mask_words(masked, gs);
@@ -227,7 +226,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
   uint64_t rp = 0;    // sign flips of row word my_k, not yet in rc
   uint32_t slot2 = 0; // which of sh.tot / sh.rx is in use (wide states)
   for (uint32_t base = 0; base < a.ninstr;) {
-    const uint32_t wn = min(kChunk, a.ninstr - base);
+    const uint32_t wn = min(kStage, a.ninstr - base);
     // instructions [base, base + wn) and their masks, whatever segments they
     // belong to: two dependent loads per window, not per segment
     bool flags = false;
@@ -240,7 +239,7 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
       SharedOp J;
       if (code == PQ_OP_M) {
         J.cw = kOpMeas | (pad & kMeasSuperseded ? kOpDropped : 0u) |
-               (min(pad >> kMeasLeftShift, kChunk) << kOpLenShift);
+               (min(pad >> kMeasLeftShift, kStage) << kOpLenShift);
         J.qq = qa;
         if (g == 0) {
           msk[t * mstep] = (uint64_t)slot | ((uint64_t)t0 << 32);
@@ -847,10 +846,6 @@ __device__ uint32_t shared_words(const ProgramArgs &a, uint64_t seed, uint64_t m
   __syncthreads();
   return live;
 }
-
-struct ProgParams {
-  uint64_t seed, mseq0, nseq0;
-};
 
 // One workgroup per G = 1 << a.gshift word groups.  With a.done, groups that
 // ran are marked there and the per-shot kernel launched behind this one passes
