@@ -270,12 +270,17 @@ int pq_set_window_qubits(uint32_t qubits);
 int pq_frame_plan(uint64_t n, const pq_op *ops, uint64_t nops, uint64_t info[16],
                   uint32_t *stream, uint32_t *chunks, uint32_t *preload, uint64_t *x,
                   uint64_t *z);
-/* Launch shape of the persistent kernel (0 keeps the current value; threads
- * a multiple of 64, at most 768, or 512 for states of 193..512 qubits and for
- * states above 512 qubits whose program has no row-tiled gate segment). */
+/* Launch shape of the per-shot persistent kernel (0 keeps the current value;
+ * threads a multiple of 64, at most 768, or 512 for states of 193..512 qubits
+ * and for states above 512 qubits whose program has no row-tiled gate segment).
+ * The kernels that keep a whole tableau packed (programs without flagged
+ * H/S/CX/CZ from |0...0>, up to 2048 qubits) or in LDS (up to 64 qubits) choose
+ * their own; asking for fewer than 256 threads keeps a program from both. */
 int pq_program_set_launch(pq_program p, uint32_t threads, uint32_t blocks);
-/* Workgroups per 64-shot word group in persistent runs: 0 chooses (states of
- * 512+ qubits with at most half as many word groups as the device has
+/* Workgroups per 64-shot word group in persistent runs of the per-shot kernel.
+ * Any call, with 0 too, keeps the program on that kernel from then on (the
+ * packed and the LDS-resident one, which it runs in otherwise where they take
+ * it, have no slices): 0 chooses (states of 512+ qubits with at most half as many word groups as the device has
  * compute units split each group's rows between two workgroups of one
  * cooperative launch),
  * 1 keeps one workgroup per group, k > 1 asks for k (PQ_ERR_ARG at the run
@@ -340,7 +345,8 @@ int pq_batch_destroy(pq_batch b);
 int pq_batch_add(pq_batch b, pq_state s, pq_program p);
 int pq_batch_run(pq_batch b, int form);
 int pq_batch_wait(pq_batch b);
-/* Launch shape: threads per workgroup (multiple of 64, <= 768; above 512 the
+/* Launch shape of the per-shot kernel (members that run packed choose their
+ * own, see pq_program_set_launch): threads per workgroup (multiple of 64, <= 768; above 512 the
  * determined chains of members of 193..512 qubits keep their scratch row in
  * LDS instead of registers), workgroups (0 = CUs x workgroups per CU) and the
  * dynamic-LDS budget per workgroup (40 KB..158 KB; it sets workgroups per CU

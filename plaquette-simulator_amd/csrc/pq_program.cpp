@@ -699,8 +699,9 @@ static int choose_slices(pq_state s, pq_program p, const ProgramArgs &a, bool al
 // Whether a persistent run may take the shared-X/Z kernel when X/Z are the
 // |0...0> tableau: no flagged H/S/CX/CZ, at least as many ops as qubits (it
 // writes the whole tableau, where a shorter program touches a few columns),
-// no census (which counts the per-shot kernel's work) and no launch shape or
-// slice count asked for.
+// no census (which counts the per-shot kernel's work), no slice count and no
+// block of fewer than 256 threads asked for (what is asked for beyond that
+// shapes the per-shot kernel alone).
 bool shared_allowed(const pq_state_s *s, const pq_program_s *p) {
   return p->uniform && shared_fits((uint32_t)s->n) && p->instrs.size() >= s->n &&
          !p->census_on && !p->slices_set && p->threads >= 256;
