@@ -331,6 +331,7 @@ struct MeasShared {
   uint64_t coin;  // coin word
 };
 
+template <bool kSliced>
 __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
                              uint32_t R, uint32_t q, uint32_t coin_T,
                              uint64_t coin_key, const uint64_t *coin_plane,
@@ -343,7 +344,9 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
   // with slices, every slice finds the same pivots and coins; slice 0 alone
   // rewrites the pivot rows and runs the determined shots, and the rowsum
   // rows are split between the slices
-  const uint32_t slice = ss ? ss->slice : 0, S = ss ? ss->slices : 1;
+  // (a build of its own each: the slices' loops in the other's registers cost
+  // the sliced runs 7 to 11% at 520 and 1024 qubits)
+  const uint32_t slice = kSliced ? ss->slice : 0, S = kSliced ? ss->slices : 1;
   const uint64_t Ru = R;
   const uint64_t *xq = T + (uint64_t)q * Ru;
 
@@ -353,7 +356,7 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
   // rows from it and the rowsums their masks.  The random shots' rewrites
   // change x_q only in the shots of their own group, and every later use
   // masks it by another group's shots (or by D), so the value stays valid.
-  const bool own_row = S == 1 && 2 * n <= NT;
+  const bool own_row = !kSliced && 2 * n <= NT;
   const uint64_t xv = (own_row && tid < 2 * n) ? xq[tid] : 0ull;
   const uint32_t cp = (n + NT - 1) / NT;
   const uint32_t p0 = min(n, tid * cp), p1 = min(n, p0 + cp);
@@ -377,7 +380,7 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
       sh.gp[g] = tid - n;
       sh.gm[g] = first;
     }
-  } else if (S == 1) {
+  } else if (!kSliced) {
     for (uint32_t p = p0; p < p1 && !force_determined; ++p) {
       const uint64_t v = xq[n + p];
       const uint64_t first = v & ~before;
@@ -428,11 +431,11 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
 
   // ---- 2. random shots ----
   const uint32_t C = 2 * n + 1;
-  const uint32_t passes = S == 1 ? min(ngroups, 1u) : ngroups;
+  const uint32_t passes = kSliced ? ngroups : min(ngroups, 1u);
   for (uint32_t g = 0; g < passes; ++g) {
     const uint32_t p = sh.gp[g];
-    const uint64_t M = S == 1 ? rm : sh.gm[g];
-    if (S == 1) {
+    const uint64_t M = kSliced ? sh.gm[g] : rm;
+    if (!kSliced) {
       for (uint32_t c = tid; c < C; c += NT) {
         uint64_t *col = T + (uint64_t)c * Ru;
         const uint64_t set = c == n + q ? ~0ull : c == 2 * n ? coin : 0ull;
@@ -486,18 +489,17 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
     const uint64_t rsrc = s_src[2 * n];
     uint32_t my_rows = 0;
     for (uint32_t i = slice * NT + tid; i < 2 * n; i += NT * S) {
+      if (kSliced && (i == p || i == n + p)) continue;
       uint64_t mi = M & (own_row ? xv : xq[i]);
-      if (S == 1) {
+      if (!kSliced) {
         const uint32_t pi = i < n ? i : i - n;
         for (uint32_t h = 0; h < ngroups; ++h)
           if (sh.gp[h] == pi) mi &= ~sh.gm[h];
         if (census)
           for (uint32_t h = 0; h < ngroups; ++h) my_rows += (mi & sh.gm[h]) ? 1u : 0u;
-      } else if (i == p || i == n + p) {
-        mi = 0;
       }
       if (!mi) continue;
-      if (S > 1) ++my_rows;
+      if (kSliced) ++my_rows;
       // the phase word is read with the first source columns, not after
       // the row's stores
       const uint64_t ri = T[(uint64_t)(2 * n) * Ru + i];
@@ -529,7 +531,7 @@ __device__ void measure_word(uint64_t *__restrict__ T, uint64_t w, uint32_t n,
     if (census && my_rows) atomicAdd(&sh.krows, my_rows);
     __syncthreads();
     // all slices' rowsums are in before the next pivot group or phase
-    if (S > 1) slice_barrier(*ss);
+    if (kSliced) slice_barrier(*ss);
   }
 
   // ---- 3. determined shots ----
@@ -601,7 +603,7 @@ __global__ __launch_bounds__(kMeasThreads) void k_measure(
   uint32_t *s_list = reinterpret_cast<uint32_t *>(dyn + (2 * n + 1));
   const uint64_t C = 2ull * n + 1;
   for (uint64_t w = blockIdx.x; w < W; w += gridDim.x)
-    measure_word(tab + w * C * R, w, n, R, q, coin_T, coin_key, coin_plane,
+    measure_word<false>(tab + w * C * R, w, n, R, q, coin_T, coin_key, coin_plane,
                  rec, rec + W, s_src, s_list, sh, force_determined != 0);
 }
 
@@ -1578,11 +1580,11 @@ struct PhaseTimes {
 };
 
 // The whole compiled program on 64-shot word group w of one state.
-template <int NREG>
+template <int NREG, bool SLICED>
 __device__ void program_word(const pq::ProgramArgs &a, uint64_t seed, uint64_t mseq0,
                              uint64_t w, uint64_t *dyn, MeasShared &sh,
                              PhaseTimes *tm, SliceSync *ss = nullptr) {
-  const uint32_t slice = ss ? ss->slice : 0, S = ss ? ss->slices : 1;
+  const uint32_t slice = SLICED ? ss->slice : 0, S = SLICED ? ss->slices : 1;
   const uint32_t n = a.n;
   uint64_t *s_src = dyn;
   uint32_t *s_list = reinterpret_cast<uint32_t *>(dyn + (2 * n + 1));
@@ -1684,7 +1686,7 @@ __device__ void program_word(const pq::ProgramArgs &a, uint64_t seed, uint64_t m
         const uint64_t key = stream_key(seed, 2 * (mseq0 + m));
         const uint64_t *cp = a.coin_planes ? a.coin_planes + m * a.W : nullptr;
         uint64_t *rec = a.recs + (2ull * I.slot) * a.W;
-        measure_word(T, w, n, a.R, I.qa, I.t0, key, cp, rec, rec + a.W, s_src,
+        measure_word<SLICED>(T, w, n, a.R, I.qa, I.t0, key, cp, rec, rec + a.W, s_src,
                      s_list, sh, false, a.census, ss);
         // slice 0's pivot rows, record and scratch row are in for every slice
         if (S > 1) slice_barrier(*ss);
@@ -1731,12 +1733,12 @@ __global__ __launch_bounds__(MAXT) void k_program_t(pq::ProgramArgs a,
       ss.ctr = a.sync + wi;
       ss.err = a.sync_err;
       if (a.sync_spin) ss.spin_limit = a.sync_spin;
-      program_word<NREG>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm, &ss);
+      program_word<NREG, true>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm, &ss);
     }
   } else {
     for (uint64_t wi = blockIdx.x; wi < a.nwords; wi += gridDim.x) {
       if (a.done && a.done[a.word0 + wi]) continue;  // k_program_shared ran it
-      program_word<NREG>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm);
+      program_word<NREG, false>(la, seed, mseq0, a.word0 + wi, dyn, sh, tm);
     }
   }
   if (census) {
@@ -1779,7 +1781,7 @@ __global__ __launch_bounds__(MAXT) void k_batch_t(
     if (bc.a.shared == kSharedKnown) continue;  // k_batch_shared ran them
     for (uint64_t wi = w; wi < wend; ++wi) {
       if (bc.a.done && bc.a.done[wi]) continue;
-      program_word<NREG>(bc.a, bc.seed, bc.mseq0, wi, dyn, sh, nullptr);
+      program_word<NREG, false>(bc.a, bc.seed, bc.mseq0, wi, dyn, sh, nullptr);
     }
   }
 }
