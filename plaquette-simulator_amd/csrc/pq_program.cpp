@@ -431,10 +431,7 @@ int compile_frame_only(pq_program_s *p) {
 }
 
 void pq_program_s::drop_graph() {
-  if (gexec) (void)hipGraphExecDestroy(gexec);
-  if (graph) (void)hipGraphDestroy(graph);
-  gexec = nullptr;
-  graph = nullptr;
+  for (Graph &g : graphs) g.drop();
 }
 
 pq_program_s::~pq_program_s() {
@@ -824,11 +821,11 @@ static int program_run(pq_state s, pq_program p, int form) {
   // X/Z are the |0...0> tableau: the shared-X/Z kernel, which reads no X/Z
   // (they may be pending) and writes them all.  The holder of a raw pointer
   // may have changed them, so the word groups of an exposed state, or of a copy
-  // of one, are checked, and so are a captured run's at every replay.
+  // of one, are checked.
   uint32_t shared = 0;
-  if ((form == PQ_RUN_PERSISTENT && s->xz_identity) || form == PQ_RUN_GRAPH)
-    if (shared_allowed(s, p))
-      shared = form == PQ_RUN_GRAPH || !xz_certain(s) ? kSharedVerify : kSharedKnown;
+  if ((form == PQ_RUN_PERSISTENT || form == PQ_RUN_GRAPH) && s->xz_identity &&
+      shared_allowed(s, p))
+    shared = xz_certain(s) ? kSharedKnown : kSharedVerify;
   if ((rc = ensure_shared(s, p, shared, shared_split((uint32_t)s->n, s->W, p->masked)))) return rc;
   // X/Z still the identity after a reset, and the whole tableau is held in LDS
   // or the program opens with a row-tiled gate segment over every qubit: the
@@ -858,13 +855,13 @@ static int program_run(pq_state s, pq_program p, int form) {
     return rc;
   }
   if (form != PQ_RUN_GRAPH) return pq_set_error(PQ_ERR_ARG, "unknown run form");
-  if (p->gexec && (p->graph_state != s || p->graph_arena_gen != s->arena_gen)) {
-    (void)hipGraphExecDestroy(p->gexec);
-    (void)hipGraphDestroy(p->graph);
-    p->gexec = nullptr;
-    p->graph = nullptr;
-  }
-  if (!p->gexec) {
+  // One captured launch per choice of kernels: what a replay runs is decided by
+  // its state here, as a persistent run's is (a launch that checked the state
+  // at every replay and kept both kernels made replays that do not start from
+  // |0...0> up to 1.5 times longer: n=161, 16384 shots, 161 ops 133 -> 195 us).
+  pq_program_s::Graph &G = p->graphs[shared];
+  if (G.exec && (G.state != s || G.arena_gen != s->arena_gen)) G.drop();
+  if (!G.exec) {
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     rc = enqueue_persistent(s, p, false, false, false, shared);
     hipGraph_t g = nullptr;
@@ -874,12 +871,16 @@ static int program_run(pq_state s, pq_program p, int form) {
       return rc;
     }
     HIPCHK(e);
-    p->graph = g;
-    HIPCHK(hipGraphInstantiate(&p->gexec, p->graph, nullptr, nullptr, 0));
-    p->graph_state = s;
-    p->graph_arena_gen = s->arena_gen;
+    G.graph = g;
+    HIPCHK(hipGraphInstantiate(&G.exec, G.graph, nullptr, nullptr, 0));
+    G.state = s;
+    G.arena_gen = s->arena_gen;
   }
-  HIPCHK(hipGraphLaunch(p->gexec, s->stream));
+  HIPCHK(hipGraphLaunch(G.exec, s->stream));
+  if (writes_xz) {
+    s->xz_pending = false;
+    s->xz_plan.reset();
+  }
   return PQ_OK;
 }
 

@@ -36,10 +36,20 @@ struct pq_program_s {
   uint64_t *d_planes = nullptr;  // noise planes [nnoise][2][W]
   uint64_t *d_side = nullptr;    // frame form, two-part runs: [W][2n + nref] words
   uint32_t threads = 0, blocks = 0;
-  hipGraph_t graph = nullptr;
-  hipGraphExec_t gexec = nullptr;
-  pq_state graph_state = nullptr;
-  uint64_t graph_arena_gen = 0;
+  // the graph form's captured launches, by which kernels they hold (0,
+  // kSharedKnown, kSharedVerify); each replay takes the one of its state
+  struct Graph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    pq_state state = nullptr;
+    uint64_t arena_gen = 0;
+    void drop() {
+      if (exec) (void)hipGraphExecDestroy(exec);
+      if (graph) (void)hipGraphDestroy(graph);
+      exec = nullptr;
+      graph = nullptr;
+    }
+  } graphs[3];
   hipStream_t alloc_stream = nullptr;  // stream-ordered allocation (server use)
   unsigned long long *d_census = nullptr;  // 8 counters when census is on
   bool census_on = false;

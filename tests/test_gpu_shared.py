@@ -360,3 +360,47 @@ def test_copies_of_a_state_changed_through_the_raw_pointer(ps):
                         os.path.join(root, "tests"), os.path.join(root, "oracle")],
                        capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and "copies ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("n,B", [(2, 64), (40, 150), (70, 200), (161, 2700), (500, 70)])
+def test_graph_replays_follow_their_state(ps, n, B):
+    """One program replayed from states that take different kernels: |0...0> after
+    a reset or behind a frame run that ends there, what the last replay left, one
+    from the host, one whose planes were handed out; then another state."""
+    from plaquette_simulator import workloads as W
+    ops = mixed_ops(n, 3 * n + 60, n, 0.1)
+    flips = W.OpList()  # X/Z end as they start
+    for q in range(n):
+        flips.gate(W.OP_X, q)
+        flips.noise(q, 0.2, 0.1, 0.1)
+    st, ref = (ps.CliffordState(n, B, 9, True) for _ in range(2))
+    prog, pref = ps.Program(st, ops), ps.Program(ref, ops)
+    fst, fref = ps.Program(st, flips.array()), ps.Program(ref, flips.array())
+    pref.set_slices(1)  # the per-shot kernel
+    held = []
+    for i, step in enumerate(["", "", "reset", "", "reset", "frame", "host", "reset", "", "expose",
+                              "reset", "", "frame", ""]):
+        say(f"[case] n={n} B={B} graph replay {i} {step}")
+        for s, f in ((st, fst), (ref, fref)):
+            if step in ("reset", "frame"):
+                s.reset_clifford_state()
+            if step == "frame":
+                f.run(s, "frame")
+            if step == "host" and n <= 70:  # (int lists: small states only)
+                x, z, r = s.device_to_host_numpy()
+                s.host_to_device(x.ravel(), z.ravel(), r.ravel())
+        if step == "expose":
+            held.append(st.planes_dlpack())
+        prog.run(st, "graph")
+        pref.run(ref, "persistent")
+        assert st.compare(ref) == (0, 0)
+    other, oref = (ps.CliffordState(n, B, 10, True) for _ in range(2))
+    for _ in range(2):
+        prog.run(other, "graph")
+        pref.run(oref, "persistent")
+        assert other.compare(oref) == (0, 0)
+    st.reset_clifford_state()
+    ref.reset_clifford_state()
+    prog.run(st, "graph")
+    pref.run(ref, "persistent")
+    assert st.compare(ref) == (0, 0)
