@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -13,7 +14,15 @@
 
 struct FramePlan;
 
+// Names a state for as long as the process lives (its address may be another's
+// later).
+inline uint64_t next_state_id() {
+  static std::atomic<uint64_t> next{1};
+  return next.fetch_add(1, std::memory_order_relaxed);
+}
+
 struct pq_state_s {
+  const uint64_t id = next_state_id();
   uint64_t n = 0, B = 0, R = 0, C = 0, W = 0;
   int64_t seed = 0;
   int device = 0;

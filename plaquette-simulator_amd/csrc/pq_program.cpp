@@ -860,7 +860,7 @@ static int program_run(pq_state s, pq_program p, int form) {
   // at every replay and kept both kernels made replays that do not start from
   // |0...0> up to 1.5 times longer: n=161, 16384 shots, 161 ops 133 -> 195 us).
   pq_program_s::Graph &G = p->graphs[shared];
-  if (G.exec && (G.state != s || G.arena_gen != s->arena_gen)) G.drop();
+  if (G.exec && (G.state_id != s->id || G.arena_gen != s->arena_gen)) G.drop();
   if (!G.exec) {
     HIPCHK(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     rc = enqueue_persistent(s, p, false, false, false, shared);
@@ -873,7 +873,7 @@ static int program_run(pq_state s, pq_program p, int form) {
     HIPCHK(e);
     G.graph = g;
     HIPCHK(hipGraphInstantiate(&G.exec, G.graph, nullptr, nullptr, 0));
-    G.state = s;
+    G.state_id = s->id;
     G.arena_gen = s->arena_gen;
   }
   HIPCHK(hipGraphLaunch(G.exec, s->stream));

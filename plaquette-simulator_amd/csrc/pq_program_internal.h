@@ -41,8 +41,7 @@ struct pq_program_s {
   struct Graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    pq_state state = nullptr;
-    uint64_t arena_gen = 0;
+    uint64_t state_id = 0, arena_gen = 0;  // the state whose buffers it holds
     void drop() {
       if (exec) (void)hipGraphExecDestroy(exec);
       if (graph) (void)hipGraphDestroy(graph);

@@ -404,3 +404,22 @@ def test_graph_replays_follow_their_state(ps, n, B):
     prog.run(st, "graph")
     pref.run(ref, "persistent")
     assert st.compare(ref) == (0, 0)
+
+
+def test_graph_of_a_state_that_is_gone(ps):
+    """A program outlives the states that it ran on: a later state may have the
+    address of one that is gone, and does not replay its captured launch."""
+    n, B = 60, 200
+    ops = mixed_ops(n, 300, 3, 0.1)
+    home = ps.CliffordState(n, B, 1, True)
+    prog = ps.Program(home, ops)
+    kept = []
+    for i in range(6):
+        say(f"[case] graph on state {i}")
+        st, ref = (ps.CliffordState(n, B, 30 + i, True) for _ in range(2))
+        prog.run(st, "graph")
+        ps.Program(ref, ops).run(ref, "persistent")
+        assert st.compare(ref) == (0, 0)
+        if i % 2:
+            kept.append(ref)  # takes the memory of the one before
+        del st, ref
