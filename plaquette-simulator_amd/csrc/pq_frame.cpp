@@ -984,7 +984,6 @@ struct Staging {
 constexpr Staging kStaging[] = {{512, 2048, 1}, {1024, 4096, 1}, {2048, 4096, 1},
                                 {2048, 8192, 1}, {2048, 8192, 2}};
 constexpr uint32_t kFrameGroupsPerCu = 4;  // resident groups that hide a group's latencies
-constexpr uint64_t kCus = 256;             // compute units of an MI355X
 
 int build_frame_plan(pq_program_s *p, uint64_t groups) {
   auto F = std::make_shared<FramePlan>();

@@ -714,6 +714,27 @@ static bool local_allowed(const pq_state_s *s, const pq_program_s *p) {
          !p->slices_set && p->threads >= 256;
 }
 
+// Whether the shared-X/Z kernel pays on |0...0> words that have to be looked at
+// first: the per-shot kernel is then launched behind it for the groups that turn
+// out different, 5 us, and the check reads the tableau.  The LDS-resident kernel
+// runs such a state by itself in as long a chain of steps, so what is left to
+// gain is per op: nothing up to 32 qubits while each group has a compute unit
+// (20 qubits, 1024 shots: 80 ops 51 -> 43 us by the LDS-resident kernel alone, 4000
+// ops 667 -> 623), more with every qubit above (1024 shots; 41 qubits: 328 ops 125
+// -> 115 us, 820 ops 118 -> 123; 50 qubits: 200 ops 90 -> 84, 1000 ops 134 -> 158; 64
+// qubits: 64 ops 36 -> 29, 128 ops 71 -> 76, 1280 ops 151 -> 221; 16384 shots, whose
+// check takes longer, 64 qubits: 256 ops 119 -> 111, 512 ops 192 -> 217), and as
+// much as the groups that share a workgroup once groups wait for compute units
+// (40000 shots; 32 qubits: 32 ops 50 -> 38 us, 64 ops 69 -> 96; 5 qubits: 5 ops 36 ->
+// 30, 20 ops 44 -> 52).  States that are too large for the LDS-resident kernel gain
+// from n ops on (65 qubits, 1024 shots, 65 ops: 53 us by k_program_t, 40).
+static bool check_pays(const pq_state_s *s, const pq_program_s *p) {
+  const uint64_t ops = p->instrs.size();
+  if (!local_fits((uint32_t)s->n)) return true;
+  if (s->W > kCus) return ops >= 2 * s->n && ops >= 48;
+  return s->n > 32 && ops * (s->n - 32) >= 4500 + 33 * s->W;
+}
+
 int ensure_shared(pq_state s, pq_program p, uint32_t shared, bool split) {
   if (shared == kSharedVerify && !p->d_done)
     HIPCHK(dev_alloc((void **)&p->d_done, s->W * sizeof(uint32_t), p->alloc_stream));
@@ -824,8 +845,12 @@ static int program_run(pq_state s, pq_program p, int form) {
   // of one, are checked.
   uint32_t shared = 0;
   if ((form == PQ_RUN_PERSISTENT || form == PQ_RUN_GRAPH) && s->xz_identity &&
-      shared_allowed(s, p))
-    shared = xz_certain(s) ? kSharedKnown : kSharedVerify;
+      shared_allowed(s, p)) {
+    if (xz_certain(s))
+      shared = kSharedKnown;
+    else if (check_pays(s, p))
+      shared = kSharedVerify;
+  }
   if ((rc = ensure_shared(s, p, shared, shared_split((uint32_t)s->n, s->W, p->masked)))) return rc;
   // X/Z still the identity after a reset, and the whole tableau is held in LDS
   // or the program opens with a row-tiled gate segment over every qubit: the

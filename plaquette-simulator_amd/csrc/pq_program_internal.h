@@ -11,6 +11,7 @@
 #include "pq_common.h"
 #include "pq_frame.h"
 
+constexpr uint64_t kCus = 256;               // compute units of an MI355X
 constexpr uint32_t kProgramThreadsMax = 768;  // largest block of the persistent kernel builds
 // Gate segments with more qubits than a row tile of kWindowCutRows rows can
 // hold (in the default LDS budget) are cut into qubit windows, each small

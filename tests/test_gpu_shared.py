@@ -423,3 +423,53 @@ def test_graph_of_a_state_that_is_gone(ps):
         if i % 2:
             kept.append(ref)  # takes the memory of the one before
         del st, ref
+
+
+_SMALL = """
+import sys
+import torch  # first: its HIP runtime must be the one the process loads
+assert torch.cuda.is_available()
+sys.path[:0] = sys.argv[1:]
+import plaquette_simulator as ps
+from test_gpu_shared import mixed_ops
+# both sides of the line between the packed and the LDS-resident kernel: 33 and
+# 64 qubits with few ops and many, groups that wait for compute units
+for n, B, nops in ((2, 64, 30), (2, 17000, 40), (2, 17000, 70), (32, 130, 900), (33, 60, 5200),
+                   (64, 64, 100), (64, 64, 260), (64, 16385, 110), (64, 16385, 200)):
+    ops = mixed_ops(n, nops, 4, 0.1)
+    for edit in (False, True):
+        for form in ("persistent", "graph"):
+            got = []
+            for per_shot in (False, True):
+                st = ps.CliffordState(n, B, 21, True)
+                planes = torch.from_dlpack(st.planes_dlpack()).view(torch.int64)
+                st.reset_clifford_state()
+                st.synchronize()
+                if edit:  # z of the last row, in two shots of the last group
+                    planes[-1, 2 * n - 1, 2 * n - 1] = 5
+                torch.cuda.synchronize()
+                prog = ps.Program(st, ops)
+                if per_shot:
+                    prog.set_slices(1)
+                prog.run(st, "persistent" if per_shot else form)
+                st.synchronize()
+                got.append((st, planes))
+            assert got[0][0].compare(got[1][0]) == (0, 0), (n, B, nops, edit, form)
+            del got, planes, st
+print("small ok")
+"""
+
+
+def test_small_states_with_the_raw_pointer_out(ps):
+    """Small states whose words have to be looked at take the packed kernel, with
+    the check and the LDS-resident one behind it, or the latter alone."""
+    pytest.importorskip("torch")
+    import os
+    import subprocess
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    say("[case] small states with the raw pointer out (child process)")
+    r = subprocess.run([sys.executable, "-c", _SMALL,
+                        os.path.join(root, "plaquette-simulator_amd"),
+                        os.path.join(root, "tests"), os.path.join(root, "oracle")],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "small ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
