@@ -98,3 +98,30 @@ def test_d9_figures_for_the_documented_census():
     f = bench.fused_minimum_bytes(w.ops, w.num_qubits, words, census)
     assert a["total"] == 36631785472
     assert f["total"] == 6192017408
+
+
+def test_traffic_counts_every_kernel_of_the_run(tmp_path):
+    """The run's kernels are all that its events span: the packed kernel and the one
+    that writes the 64-shot words, behind the calibration copy; not the warm-up
+    run before it, nor the noise."""
+    from plaquette_simulator import profiling as P
+    kernels = ["k_program_noise(x)", "void pq::(anonymous namespace)::k_program_shared<true>(a, b)",
+               "pq::(anonymous namespace)::k_shared_expand(a)", "__amd_rocclr_copyBuffer",
+               "void pq::(anonymous namespace)::k_frame_noise<1u>(a)",
+               "void pq::(anonymous namespace)::k_program_shared<true>(a, b)",
+               "pq::(anonymous namespace)::k_shared_expand(a)", "k_checksum(x)"]
+    dirs = []
+    for name, kib in (("FETCH_SIZE", [9, 900, 90, 50, 7, 300, 20, 8]),
+                      ("WRITE_SIZE", [9, 900, 90, 100, 7, 30, 200, 8])):
+        d = tmp_path / name
+        d.mkdir()
+        rows = ["Dispatch_Id,Kernel_Name,Counter_Name,Counter_Value"]
+        rows += [f'{i},"{k}",{name},{v}' for i, (k, v) in enumerate(zip(kernels, kib))]
+        (d / "run_counter_collection.csv").write_text("\n".join(rows) + "\n")
+        dirs.append(str(d))
+    res = P.traffic(*dirs, str(tmp_path / "t.json"), str(tmp_path / "t.md"), copy_bytes=100 * 1024)
+    assert res["fetch"]["bytes"] == 320 * 1024 * 2  # the counter reads half of the copy's bytes
+    assert res["write"]["bytes"] == 230 * 1024
+    assert res["bytes_per_launch"] == (640 + 230) * 1024
+    P.pmc(str(tmp_path / "p.md"), *dirs)
+    assert "k_program_shared<true> | k_shared_expand | calibration copy" in (tmp_path / "p.md").read_text()
