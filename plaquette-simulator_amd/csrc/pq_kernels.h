@@ -156,7 +156,10 @@ hipError_t launch_program(hipStream_t s, const ProgramArgs &a, uint32_t threads,
                           uint32_t blocks, const void *params);
 // Shared-X/Z form of a persistent run (pq_shared.hip): programs without
 // flagged H/S/CX/CZ on the |0...0> tableau, one workgroup per 1, 2 or 4 word
-// groups.
+// groups.  768 threads: the wide columns need the waves (4096 shots, us with 256,
+// 512 and 768 threads: d=9 423, 330, 307; d=13 1321, 930, 841; 1024 random qubits
+// 7050, 4706, 3772); few qubits would lose less at their barriers with fewer
+// (64: 348, 354, 367; 20: 106, 107, 112; d=3: 59.8, 57.5, 59.2).
 constexpr uint32_t kSharedThreads = 768;
 constexpr uint32_t kSharedMaxQubits = 2048;
 constexpr uint32_t kSharedMaxGroups = 4;

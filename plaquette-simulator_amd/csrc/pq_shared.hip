@@ -4,12 +4,13 @@
 // program without flagged H/S/CX/CZ that starts from |0...0> keeps the X/Z
 // words of a 64-shot group all zeros or all ones throughout: one bit instead
 // of 64 per entry.  The kernels here run a whole compiled program on that
-// packed tableau, in one workgroup per word group, and write the group's 64-shot
-// words once at the end.  Per word group they keep
+// packed tableau, in one workgroup per 1, 2 or 4 word groups, and write the
+// groups' 64-shot words once at the end.  Per workgroup they keep
 //  * X and Z as bits, one column of KW = 2 KH + 1 words per x_q and z_q
 //    (KH = ceil(n/64)): KH words of destabilizer rows, KH words of stabilizer
 //    rows, so rows i and n+i share a bit position, and one word whose bit 0
 //    is the scratch row;
+// and per word group
 //  * the signs as R[i] = Rv[i] ^ rc[i] ^ <E, P_i>: a 64-shot word per row
 //    that only measurements change, a bit per row for what all shots share
 //    (gate phases, rowsum phases), and a Pauli frame E (an x and a z word of
@@ -20,9 +21,9 @@
 //
 // What this saves: the per-shot kernel (k_program_t) moves and computes
 // R = 2n+1 words of 64 shots per column and gate; here a column is 2 n/64 words
-// of rows.  n <= about 460: the packed columns (2n (2 n/64 + 1) words) sit in
-// LDS; up to 2048 qubits they sit at the start of the group's tableau block,
-// which the run overwrites anyway.
+// of rows.  Up to 464 qubits (487 in programs without noise and flags) the packed
+// columns (2n (2 n/64 + 1) words) sit in LDS; up to 2048 they sit at the start
+// of a group's tableau block, which the run overwrites anyway.
 #include "pq_kernels.h"
 
 #include <algorithm>
@@ -972,7 +973,16 @@ uint32_t shared_batch_gshift(uint32_t n, uint64_t W, bool masked, uint64_t group
 }
 
 // Word groups per workgroup.  Groups that share a workgroup share the packed
-// X/Z work; more workgroups finish sooner on an empty GPU.
+// X/Z work; more workgroups finish sooner on an empty GPU.  Columns in LDS: at
+// least 64 workgroups, so that four states' run side by side on 256 compute units
+// (d=9, 16384 shots, us for 1, 2, 3, 6 and 12 states in flight: 421, 542, 648, 1285,
+// 2552 with 64 workgroups of four groups; 377, 500, 797, 1465, 2643 with 128 of
+// two; 64 random qubits, 8192 shots: 375, 384, 391, 756, 1493; 367, 376, 717, 1078,
+// 2135; with 32 workgroups one state of 8192 shots takes 383 instead of 337).
+// Columns in the tableau, whose work is the L2's: as many groups as fit (n=1024,
+// 4096 shots, 1 and 2 states: 3766, 4415 us; one group per workgroup 4120, 6160).
+// Up to 16 groups in all one per workgroup would be the faster (n=1024, 1024 shots:
+// 3267 against 2892 us).
 uint32_t shared_gshift(uint32_t n, uint64_t W, bool masked) {
   uint32_t gs = 0;
   const uint64_t least = packed_in_lds(n, masked) ? 64 : 1;
@@ -984,7 +994,10 @@ uint32_t shared_gshift(uint32_t n, uint64_t W, bool masked) {
 
 // Whether the tableau check and the 64-shot words are launches of their own,
 // over the whole GPU: for a small state the two launches cost more than they
-// save.
+// save.  What they save grows with the tableau words a workgroup would write:
+// at 33 MB, alone, checked: 64 qubits 236 us with, 249 without; 161 qubits 377,
+// 393; 300 qubits 378, 475; below, at 8 MB: 64 qubits 217, 205 (four states in
+// flight 488, 405), 161 qubits 362, 384 (780, 768), 300 qubits 362, 462.
 bool shared_split(uint32_t n, uint64_t W, bool masked) {
   return !packed_in_lds(n, masked) || W * (2ull * n + 1) * (2ull * n + 1) * 8 >= (32ull << 20);
 }
