@@ -645,6 +645,9 @@ def bench_random_n1024(args):
         prog.run(st, "persistent")
     st.synchronize()
     wall = time.perf_counter() - t0
+    slices, failed = prog.slice_status(st)  # of the timed runs (1: packed)
+    if failed:
+        raise RuntimeError("a barrier between the slices of a word group gave up")
     kms, launches = prog.kernel_ms()
     kernel_ms = kms / max(1, launches)
     ms_step = 1e3 * wall / steps
@@ -797,6 +800,7 @@ def main():
     kernel_ms = kms / max(1, launches)
 
     # graph form (same kernels, captured once, replayed)
+    st.reset_clifford_state()
     prog.run(st, "graph")
     st.synchronize()
     t0 = time.perf_counter()
